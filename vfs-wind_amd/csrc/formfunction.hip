@@ -50,7 +50,7 @@ struct FaceArgs {
 // reads outside the tile go to HBM.  The tile holds exactly the values the
 // DMDA index with periodic wrap would return.  nvert (blanking codes, small
 // integers) is kept as float in LDS, which represents them exactly.
-constexpr int FT_I = 32, FT_J = 16, FT_K = 16;
+constexpr int FT_I = 32, FT_J = 16;
 
 template <bool SO>
 struct TileDims {
@@ -341,10 +341,10 @@ __device__ inline void face_point(const FaceArgs &a, const TileAcc<SO> &T, int i
     for (int c = 0; c < 3; c++) { a.out[(6 + c) * n + q] = dv[c]; a.out[(15 + c) * n + q] = vs[c]; }
 }
 
-// One block owns an FT_I x FT_J column of points and marches FT_K planes in
+// One block owns an FT_I x FT_J column of points and marches kc planes in
 // k, keeping a rolling 3-plane LDS tile of ucat / nvert / nu_t.
 template <bool SO, bool DER>
-__global__ void __launch_bounds__(FT_I * FT_J) k_face_fluxes(FaceArgs a)
+__global__ void __launch_bounds__(FT_I * FT_J) k_face_fluxes(FaceArgs a, int kc)
 {
     using D = TileDims<SO>;
     __shared__ double sx[3 * D::HP], sy[3 * D::HP], sz[3 * D::HP], st[3 * D::HP];
@@ -355,8 +355,8 @@ __global__ void __launch_bounds__(FT_I * FT_J) k_face_fluxes(FaceArgs a)
     const int bi = b % nbi;
     b /= nbi;
     const int bj = b % nbj, bk = b / nbj;
-    const int i0 = bi * FT_I, j0 = bj * FT_J, k0 = bk * FT_K;
-    const int k1 = k0 + FT_K < g.mz ? k0 + FT_K : g.mz;
+    const int i0 = bi * FT_I, j0 = bj * FT_J, k0 = bk * kc;
+    const int k1 = k0 + kc < g.mz ? k0 + kc : g.mz;
     const int tx = threadIdx.x % FT_I, ty = threadIdx.x / FT_I;
     const bool les = a.les != 0;
     auto load_plane = [&](int kk, int slot) {
@@ -434,12 +434,12 @@ constexpr int FX_J = FT_J + 1;
 static_assert(FT_I == 32, "a row of the tile is half a wavefront (the i-face exchange shuffles within it)");
 constexpr int HX_T0 = 64;  // first thread of the second wavefront
 static_assert(FT_I * FT_J >= HX_T0 + FT_J && FT_J * 2 <= 64, "halo lanes of the i faces");
-inline unsigned face_fp_blocks(const Grid &g)
+inline long long face_fp_tiles(const Grid &g)
 {
-    return (unsigned)(((g.mx - 2 + FT_I - 1) / FT_I) * ((g.my - 2 + FT_J - 1) / FT_J) * ((g.mz - 2 + FT_K - 1) / FT_K));
+    return (long long)((g.mx - 2 + FT_I - 1) / FT_I) * ((g.my - 2 + FT_J - 1) / FT_J);
 }
 template <bool NB>
-__global__ void __launch_bounds__(FT_I * FT_J) __attribute__((amdgpu_waves_per_eu(2))) k_face_fp(FaceArgs a, double *__restrict__ fp)
+__global__ void __launch_bounds__(FT_I * FT_J) __attribute__((amdgpu_waves_per_eu(2))) k_face_fp(FaceArgs a, int kc, double *__restrict__ fp)
 {
     using D = TileDims<true>;
     __shared__ double sx[3 * D::HP], sy[3 * D::HP], sz[3 * D::HP], st[3 * D::HP];
@@ -447,8 +447,8 @@ __global__ void __launch_bounds__(FT_I * FT_J) __attribute__((amdgpu_waves_per_e
     __shared__ double fxj[6][FX_J][FT_I];  // j-face div xyz, visc xyz; row 0 = face j0-1
     __shared__ double hx[6][FT_J];         // i-face div xyz, visc xyz at i0-1 of each row
     const Grid &g = a.g;
-    // The tiles cover the interior points (1 .. m-2 on each axis; face_fp_blocks
-    // blocks): the faces at index 0 are the halo faces of the first tiles, and
+    // The tiles cover the interior points (1 .. m-2 on each axis; kc planes a
+    // block): the faces at index 0 are the halo faces of the first tiles, and
     // the ghost points' projections are not written (zero at the non-periodic
     // ghosts since allocation, copies at the periodic ones by the periodic fix
     // that follows).  Tiles are taken in XCD order, so the tiles that share a
@@ -458,8 +458,8 @@ __global__ void __launch_bounds__(FT_I * FT_J) __attribute__((amdgpu_waves_per_e
     const int bi = b % nbi;
     b /= nbi;
     const int bj = b % nbj, bk = b / nbj;
-    const int i0 = 1 + bi * FT_I, j0 = 1 + bj * FT_J, k0 = 1 + bk * FT_K;
-    const int k1 = k0 + FT_K < g.mz - 1 ? k0 + FT_K : g.mz - 1;
+    const int i0 = 1 + bi * FT_I, j0 = 1 + bj * FT_J, k0 = 1 + bk * kc;
+    const int k1 = k0 + kc < g.mz - 1 ? k0 + kc : g.mz - 1;
     const int tx = threadIdx.x % FT_I, ty = threadIdx.x / FT_I;
     const int i = i0 + tx, j = j0 + ty;
     const bool inb = i < g.mx && j < g.my;
@@ -718,11 +718,11 @@ __device__ inline void fp_at(const CellArgs &a, int k, int j, int i, double f[3]
 }
 
 // Fp of every point as the projection reads it (fp_at), written once to a
-// 3-plane scratch.  A block owns an FT_I x FT_J column and marches FT_K planes
+// 3-plane scratch.  A block owns an FT_I x FT_J column and marches kc planes
 // in k; on the second-order path a thread keeps its k-face fluxes in
 // registers, where they become the k-1 face of the next plane.
 template <bool SO>
-__global__ void __launch_bounds__(FT_I * FT_J) k_cell_fp(CellArgs a, double *__restrict__ fp)
+__global__ void __launch_bounds__(FT_I * FT_J) k_cell_fp(CellArgs a, int kc, double *__restrict__ fp)
 {
     const Grid &g = a.g;
     const int nbi = (g.mx + FT_I - 1) / FT_I, nbj = (g.my + FT_J - 1) / FT_J;
@@ -730,9 +730,9 @@ __global__ void __launch_bounds__(FT_I * FT_J) k_cell_fp(CellArgs a, double *__r
     const int bi = b % nbi;
     b /= nbi;
     const int bj = b % nbj, bk = b / nbj;
-    const int i = bi * FT_I + threadIdx.x % FT_I, j = bj * FT_J + threadIdx.x / FT_I, k0 = bk * FT_K;
+    const int i = bi * FT_I + threadIdx.x % FT_I, j = bj * FT_J + threadIdx.x / FT_I, k0 = bk * kc;
     if (i >= g.mx || j >= g.my) return;
-    const int k1 = k0 + FT_K < g.mz ? k0 + FT_K : g.mz;
+    const int k1 = k0 + kc < g.mz ? k0 + kc : g.mz;
     const long long n = g.n;
     double km1[6];
     bool have = false;
@@ -779,7 +779,7 @@ __global__ void __launch_bounds__(FT_I * FT_J) k_cell_fp(CellArgs a, double *__r
 
 // Contravariant projection of Fp and boundary zeroing (momentum.c:1715-1938),
 // marching in k with the k+1 neighbour carried in registers.
-__global__ void __launch_bounds__(FT_I * FT_J) k_cell_rhs(CellArgs a, const double *__restrict__ fp)
+__global__ void __launch_bounds__(FT_I * FT_J) k_cell_rhs(CellArgs a, int kc, const double *__restrict__ fp)
 {
     const Grid &g = a.g;
     const int nbi = (g.mx + FT_I - 1) / FT_I, nbj = (g.my + FT_J - 1) / FT_J;
@@ -787,9 +787,9 @@ __global__ void __launch_bounds__(FT_I * FT_J) k_cell_rhs(CellArgs a, const doub
     const int bi = b % nbi;
     b /= nbi;
     const int bj = b % nbj, bk = b / nbj;
-    const int i = bi * FT_I + threadIdx.x % FT_I, j = bj * FT_J + threadIdx.x / FT_I, k0 = bk * FT_K;
+    const int i = bi * FT_I + threadIdx.x % FT_I, j = bj * FT_J + threadIdx.x / FT_I, k0 = bk * kc;
     if (i >= g.mx || j >= g.my) return;
-    const int k1 = k0 + FT_K < g.mz ? k0 + FT_K : g.mz;
+    const int k1 = k0 + kc < g.mz ? k0 + kc : g.mz;
     const long long n = g.n;
     const int mx = g.mx, my = g.my, mz = g.mz;
     double fk_[3], z1[3], nvk = 0;
@@ -893,21 +893,18 @@ __global__ void __launch_bounds__(FT_I * FT_J) k_cell_rhs(CellArgs a, const doub
 // reads no cell metrics (the same products, hence the same bits).
 // The cell pass needs no LDS tile: a block takes CR_T consecutive points of
 // a k plane (the plane flattened, so 6 KB of each AoS array per block and no
-// block covers only the last few points of a row) and marches FT_K planes.
+// block covers only the last few points of a row) and marches kc planes.
 constexpr int CR_T = 256;
-inline unsigned cell_rhs_blocks(const Grid &g)
-{
-    return (unsigned)(((g.plane + CR_T - 1) / CR_T) * ((g.mz + FT_K - 1) / FT_K));
-}
-__global__ void __launch_bounds__(CR_T) k_cell_rhs_pr(CellArgs a, const double *__restrict__ pr)
+inline long long cell_rhs_tiles(const Grid &g) { return (g.plane + CR_T - 1) / CR_T; }
+__global__ void __launch_bounds__(CR_T) k_cell_rhs_pr(CellArgs a, int kc, const double *__restrict__ pr)
 {
     const Grid &g = a.g;
     const long long nbp = (g.plane + CR_T - 1) / CR_T;
     const long long bp = blockIdx.x % nbp, bk = blockIdx.x / nbp;
     const long long pp = bp * CR_T + threadIdx.x;
     if (pp >= g.plane) return;
-    const int i = (int)(pp % g.mx), j = (int)(pp / g.mx), k0 = (int)bk * FT_K;
-    const int k1 = k0 + FT_K < g.mz ? k0 + FT_K : g.mz;
+    const int i = (int)(pp % g.mx), j = (int)(pp / g.mx), k0 = (int)bk * kc;
+    const int k1 = k0 + kc < g.mz ? k0 + kc : g.mz;
     const long long n = g.n;
     const int mx = g.mx, my = g.my, mz = g.mz;
     double pk_next = 0, nvk = 0;
@@ -1022,6 +1019,32 @@ int nvert_all_zero(vfs_ctx *c, bool *zero)
     return VFS_OK;
 }
 
+// Longest run of planes of the cell passes (what a run keeps in registers is
+// one of their streams only: nothing is gained beyond this).
+constexpr int CELL_K = 16;
+
+// Planes a block of a face pass marches.  Its registers and LDS leave one
+// block per CU, so a pass takes ceil(blocks / CUs) turns of kc planes, the
+// `extra` planes it computes a second time and the three plane loads before
+// the first one: the run that makes this shortest is taken.  Against runs of
+// 16 planes everywhere: k_face_fp 100 -> 14 us on 16x12x16 cells, 105 -> 24 us
+// on 64x48x64, 107 -> 39 us on 96x64x80, 797 -> 777 us on 256x192x256 (runs of
+// 32); fourth-order k_face_fluxes 372 -> 316 us on 136x104x88.
+static int face_planes(long long tiles, int nk, int extra)
+{
+    constexpr int CUS = 256, FILL = 3, LONGEST = 64;
+    int best = 1;
+    long long cost = -1;
+    for (int kc = 1; kc <= LONGEST && kc <= nk; kc++) {
+        const long long turns = (tiles * ((nk + kc - 1) / kc) + CUS - 1) / CUS, t = turns * (kc + extra + FILL);
+        if (cost < 0 || t < cost) {
+            cost = t;
+            best = kc;
+        }
+    }
+    return best;
+}
+
 bool formfunction2_fused(const vfs_ctx *c)
 {
     // VFS_FUSED_FP=0 keeps the flux planes (the face pass, then k_cell_fp)
@@ -1051,7 +1074,8 @@ int formfunction2(vfs_ctx *c, double scale, const double *pucont, double rk_alph
     fa.second_order = c->p.second_order;
     fa.laplacian = c->p.laplacian;
     fa.out = c->face;
-    const unsigned nbt = (unsigned)(((g.mx + FT_I - 1) / FT_I) * ((g.my + FT_J - 1) / FT_J) * ((g.mz + FT_K - 1) / FT_K));
+    const long long tiles = (long long)((g.mx + FT_I - 1) / FT_I) * ((g.my + FT_J - 1) / FT_J);
+    auto blocks = [](long long t, int nk, int kc) { return dim3((unsigned)(t * ((nk + kc - 1) / kc))); };
     const long long np[3] = {2LL * g.my * g.mz, 2LL * g.mx * g.mz, 2LL * g.mx * g.my};
     const int per[3] = {g.pi, g.pj, g.pk};
     const bool fused = formfunction2_fused(c);
@@ -1063,16 +1087,17 @@ int formfunction2(vfs_ctx *c, double scale, const double *pucont, double rk_alph
         if (rc) return rc;
     }
     prof_begin(c, K_FACE);
-    if (fused && nb)
-        hipLaunchKernelGGL(k_face_fp<true>, dim3(face_fp_blocks(g)), dim3(FT_I * FT_J), 0, st, fa, c->fpc);
-    else if (fused)
-        hipLaunchKernelGGL(k_face_fp<false>, dim3(face_fp_blocks(g)), dim3(FT_I * FT_J), 0, st, fa, c->fpc);
-    else if (fa.second_order && c->face_derived)
-        hipLaunchKernelGGL((k_face_fluxes<true, true>), dim3(nbt), dim3(FT_I * FT_J), 0, st, fa);
-    else if (fa.second_order)
-        hipLaunchKernelGGL((k_face_fluxes<true, false>), dim3(nbt), dim3(FT_I * FT_J), 0, st, fa);
-    else
-        hipLaunchKernelGGL((k_face_fluxes<false, false>), dim3(nbt), dim3(FT_I * FT_J), 0, st, fa);
+    if (fused) {
+        // a block also computes the k faces below its first plane
+        const int kc = face_planes(face_fp_tiles(g), g.mz - 2, 1);
+        hipLaunchKernelGGL(nb ? k_face_fp<true> : k_face_fp<false>, blocks(face_fp_tiles(g), g.mz - 2, kc), dim3(FT_I * FT_J), 0,
+                           st, fa, kc, c->fpc);
+    } else {
+        const int kc = face_planes(tiles, g.mz, 0);
+        auto kern = !fa.second_order ? k_face_fluxes<false, false>
+                                     : (c->face_derived ? k_face_fluxes<true, true> : k_face_fluxes<true, false>);
+        hipLaunchKernelGGL(kern, blocks(tiles, g.mz, kc), dim3(FT_I * FT_J), 0, st, fa, kc);
+    }
     prof_end(c);
     VFS_LAUNCH_CHECK("face fluxes");
     if (fused) {
@@ -1111,19 +1136,21 @@ int formfunction2(vfs_ctx *c, double scale, const double *pucont, double rk_alph
     ca.cn_da = cn ? cn->da : 0.0;
     ca.cn_db = cn ? cn->db : 0.0;
     if (!fused) {
+        const int kc = march_planes(tiles, g.mz, CELL_K, 1024);
         prof_begin(c, K_CELLFP);
-        if (ca.second_order)
-            hipLaunchKernelGGL(k_cell_fp<true>, dim3(nbt), dim3(FT_I * FT_J), 0, st, ca, c->fpc);
-        else
-            hipLaunchKernelGGL(k_cell_fp<false>, dim3(nbt), dim3(FT_I * FT_J), 0, st, ca, c->fpc);
+        hipLaunchKernelGGL(ca.second_order ? k_cell_fp<true> : k_cell_fp<false>, blocks(tiles, g.mz, kc), dim3(FT_I * FT_J), 0, st,
+                           ca, kc, c->fpc);
         prof_end(c);
     }
     prof_begin(c, K_CELL);
     if (fused && nb) ca.nvert = nullptr;  // the cell pass then skips its blanking tests
-    if (fused)
-        hipLaunchKernelGGL(k_cell_rhs_pr, dim3(cell_rhs_blocks(g)), dim3(CR_T), 0, st, ca, (const double *)c->fpc);
-    else
-        hipLaunchKernelGGL(k_cell_rhs, dim3(nbt), dim3(FT_I * FT_J), 0, st, ca, (const double *)c->fpc);
+    if (fused) {
+        const int kc = march_planes(cell_rhs_tiles(g), g.mz, CELL_K, 2048);
+        hipLaunchKernelGGL(k_cell_rhs_pr, blocks(cell_rhs_tiles(g), g.mz, kc), dim3(CR_T), 0, st, ca, kc, (const double *)c->fpc);
+    } else {
+        const int kc = march_planes(tiles, g.mz, CELL_K, 1024);
+        hipLaunchKernelGGL(k_cell_rhs, blocks(tiles, g.mz, kc), dim3(FT_I * FT_J), 0, st, ca, kc, (const double *)c->fpc);
+    }
     prof_end(c);
     prof_end(c, whole);
     if (pucont) ucat_stale(c);  // the RK stage wrote Ucont

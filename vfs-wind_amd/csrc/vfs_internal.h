@@ -145,6 +145,17 @@ __device__ inline void xcd_block3(unsigned &bx, unsigned &by, unsigned &bz)
 // tile, marching kc planes; blocks are numbered i-tile fastest, then j-tile,
 // then k-chunk
 constexpr int KM_I = 64, KM_J = 4, KM_K = 16;
+// Planes a block of a k-marching kernel takes: the longest run up to kmax
+// that still leaves `want` blocks (several per CU).  A run is a serial chain
+// of one global load latency per plane, so where a grid has few tiles the
+// planes are spread over blocks instead (runs of 16 planes before: the eddy
+// viscosity of 16x12x16 cells 39 -> 6 us, k_cell_rhs_pr 14 -> 4 us; of
+// 64x48x64 cells 42 -> 10 us and 19 -> 7 us; 256x192x256 keeps its runs).
+inline int march_planes(long long tiles, int nk, int kmax, long long want)
+{
+    const long long kc = tiles * nk / want;
+    return (int)(kc < 1 ? 1 : kc > kmax ? kmax : kc);
+}
 __host__ __device__ inline unsigned km_blocks(const Grid &g, int kc)
 {
     return (unsigned)(((g.mx - 2 + KM_I - 1) / KM_I) * ((g.my - 2 + KM_J - 1) / KM_J) * ((g.mz - 2 + kc - 1) / kc));

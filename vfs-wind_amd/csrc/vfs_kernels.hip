@@ -1056,21 +1056,21 @@ __global__ void k_eddy(Grid g, double cs2, const double *__restrict__ csf, const
 }
 
 // The same per interior point, with one thread per (i, j) of a 64 x 4 tile
-// marching KM_K planes: the thread's own ucat and nvert of the planes k-1,
+// marching kc planes: the thread's own ucat and nvert of the planes k-1,
 // k, k+1 stay in registers, so every value of those arrays leaves HBM once
 // (the thread-per-point form re-read the k +- 1 planes).  The ghost cells
 // get nu_t = 0 from k_zero_ghosts.
 // NB: no point is blanked (every nvert 0): the blanking tests fold away;
 // CSF: lCs is the per-point array csf (dynamic model), else the scalar cs2
 template <bool NB, bool CSF>
-__global__ void __launch_bounds__(KM_I * KM_J) k_eddy_km(Grid g, double cs2, const double *__restrict__ csf,
+__global__ void __launch_bounds__(KM_I * KM_J) k_eddy_km(Grid g, int kc, double cs2, const double *__restrict__ csf,
                                                         const double *__restrict__ ucat,
                                                         const double *__restrict__ csi, const double *__restrict__ eta,
                                                         const double *__restrict__ zet, const double *__restrict__ aj,
                                                         const double *__restrict__ nvert, double *__restrict__ nut)
 {
     int i, j, k0, k1;
-    if (!km_tile(g, KM_K, i, j, k0, k1)) return;
+    if (!km_tile(g, kc, i, j, k0, k1)) return;
     const double SOL = 0.1;
     const long long P = g.plane;
     long long q = gidx(g, k0, j, i);
@@ -1160,7 +1160,8 @@ int eddy_viscosity(vfs_ctx *c)
         if (rc) return rc;
         auto kern = nb ? (csf ? k_eddy_km<true, true> : k_eddy_km<true, false>)
                        : (csf ? k_eddy_km<false, true> : k_eddy_km<false, false>);
-        hipLaunchKernelGGL(kern, dim3(km_blocks(g, KM_K)), dim3(KM_I * KM_J), 0, c->stream, g, cs2, csp,
+        const int kc = march_planes(km_blocks(g, g.mz), g.mz - 2, KM_K, 2048);
+        hipLaunchKernelGGL(kern, dim3(km_blocks(g, kc)), dim3(KM_I * KM_J), 0, c->stream, g, kc, cs2, csp,
                            c->f[VFS_UCAT], c->f[VFS_CSI], c->f[VFS_ETA], c->f[VFS_ZET], c->f[VFS_AJ], c->f[VFS_NVERT],
                            c->f[VFS_NU_T]);
     }
