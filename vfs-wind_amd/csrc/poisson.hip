@@ -975,46 +975,68 @@ __global__ void k_restrict(Grid gc, Grid gf, const unsigned char *__restrict__ r
 // x values of the 4x4x4 fine block around the children come through the
 // per-axis canonical positions nbr_idx uses.
 // SPL: the fine x and b in the S layout (zf), a ghost x reading as zero.
+// A block takes 64 coarse points; each of its four wavefronts forms the
+// residuals of one (dk, dj) row of two children and the first adds the eight
+// from LDS.  With one thread per coarse point the coarse levels had too few
+// loads in flight: 15.3 -> 10.3 us per launch over levels 1-4 at 256x192x256
+// (FP32, seven coefficients; the finest level stays at 153 us), 61 -> 38 us
+// over all levels at 128x96x128 (FP64, nineteen).
+constexpr int RR_PTS = 64;
 template <typename T, int NQ, bool SPL = false>
-__global__ void __launch_bounds__(PTPB) k_residual_restrict(Grid gc, Grid gf, const T *__restrict__ coef,
-                                                            const unsigned char *__restrict__ rowc,
-                                                            const unsigned char *__restrict__ rowf, const T *__restrict__ x,
-                                                            const T *__restrict__ b, T *__restrict__ bc, ZGrid zf = {})
+__global__ void __launch_bounds__(4 * RR_PTS) k_residual_restrict(Grid gc, Grid gf, const T *__restrict__ coef,
+                                                                  const unsigned char *__restrict__ rowc,
+                                                                  const unsigned char *__restrict__ rowf,
+                                                                  const T *__restrict__ x, const T *__restrict__ b,
+                                                                  T *__restrict__ bc, ZGrid zf = {})
 {
-    long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-    if (t >= gc.n) return;
-    if (!rowc[t]) { bc[t] = 0; return; }
-    const int t32 = (int)t; int i = t32 % gc.mx; int r = t32 / gc.mx; int j = r % gc.my, k = r / gc.my;
-    // fine positions 2c-2 .. 2c+1 per axis (children at 2c-1 and 2c)
-    int I[4], J[4], K[4];
+    __shared__ T res[4][2][RR_PTS];
+    const int lane = threadIdx.x % RR_PTS, grp = threadIdx.x / RR_PTS;
+    const int dk = grp >> 1, dj = grp & 1;
+    const long long t = blockIdx.x * (long long)RR_PTS + lane;
+    const bool rows = t < gc.n && rowc[t];
+    T rs[2] = {0, 0};
+    if (rows) {
+        int i, j, k;
+        nat_decode(gc, (unsigned)t, k, j, i);
+        // fine positions 2c-2 .. 2c+1 along i (children at 2c-1 and 2c), and
+        // the child row's own position with its two neighbours along j and k
+        int I[4], J[3], K[3];
 #pragma unroll
-    for (int d = 0; d < 4; d++) {
-        I[d] = canon(2 * i - 2 + d, gf.mx, gf.pi);
-        J[d] = canon(2 * j - 2 + d, gf.my, gf.pj);
-        K[d] = canon(2 * k - 2 + d, gf.mz, gf.pk);
-    }
-    T s = 0;
+        for (int d = 0; d < 4; d++) I[d] = canon(2 * i - 2 + d, gf.mx, gf.pi);
 #pragma unroll
-    for (int dk = 0; dk < 2; dk++)
+        for (int d = 0; d < 3; d++) {
+            J[d] = canon(2 * j - 2 + dj + d, gf.my, gf.pj);
+            K[d] = canon(2 * k - 2 + dk + d, gf.mz, gf.pk);
+        }
 #pragma unroll
-        for (int dj = 0; dj < 2; dj++)
+        for (int di = 0; di < 2; di++) {
+            const long long qf = gidx(gf, 2 * k - 1 + dk, 2 * j - 1 + dj, 2 * i - 1 + di);
+            if (!rowf[qf]) continue;
+            T a = 0;
 #pragma unroll
-            for (int di = 0; di < 2; di++) {
-                const long long qf = gidx(gf, 2 * k - 1 + dk, 2 * j - 1 + dj, 2 * i - 1 + di);
-                if (!rowf[qf]) continue;
-                T a = 0;
-#pragma unroll
-                for (int q = 0; q < NQ; q++) {
-                    const int kq = K[dk + 1 + soff(q, 2)], jq = J[dj + 1 + soff(q, 1)], iq = I[di + 1 + soff(q, 0)];
-                    T xv;
-                    if constexpr (SPL) xv = zs_interior(gf, kq, jq, iq) ? x[zs_index32(zf, kq, jq, iq)] : T(0);
-                    else xv = x[((long long)kq * gf.my + jq) * gf.mx + iq];
-                    a += coef[q * gf.n + qf] * xv;
-                }
-                const T bq = SPL ? b[zs_index32(zf, 2 * k - 1 + dk, 2 * j - 1 + dj, 2 * i - 1 + di)] : b[qf];
-                s += bq - a;
+            for (int q = 0; q < NQ; q++) {
+                const int kq = K[1 + soff(q, 2)], jq = J[1 + soff(q, 1)], iq = I[di + 1 + soff(q, 0)];
+                T xv;
+                if constexpr (SPL) xv = zs_interior(gf, kq, jq, iq) ? x[zs_index32(zf, kq, jq, iq)] : T(0);
+                else xv = x[((long long)kq * gf.my + jq) * gf.mx + iq];
+                a += coef[q * gf.n + qf] * xv;
             }
-    bc[t] = s;
+            const T bq = SPL ? b[zs_index32(zf, 2 * k - 1 + dk, 2 * j - 1 + dj, 2 * i - 1 + di)] : b[qf];
+            rs[di] = bq - a;
+        }
+    }
+    res[grp][0][lane] = rs[0];
+    res[grp][1][lane] = rs[1];
+    __syncthreads();
+    if (grp == 0 && t < gc.n) {
+        T s = 0;  // (a child that is no row adds the zero it stored)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            s += res[r][0][lane];
+            s += res[r][1][lane];
+        }
+        bc[t] = rows ? s : T(0);
+    }
 }
 
 __device__ inline int parent_nb(int I, int d, int mc, int per)
@@ -1025,34 +1047,17 @@ __device__ inline int parent_nb(int I, int d, int mc, int per)
     return J;
 }
 
-// fine x += trilinear(coarse x)
-template <typename T>
-__global__ void k_prolong(Grid gc, Grid gf, const unsigned char *__restrict__ rowf, const T *__restrict__ xc,
-                          T *__restrict__ xf)
+// fine x += trilinear(coarse x) at the points of the colours from `first` on,
+// one thread per S position; the iterate in the S layout (SPL) or the natural
+// one.  Where the next half-sweep (colour 0) reads only colour 1 and rewrites
+// its own points whatever they hold, the caller starts at colour 1 (finest
+// level at 256x192x256: 59 -> 31 us).
+template <typename T, bool SPL>
+__global__ void __launch_bounds__(PTPB) k_prolong(Grid gc, Grid gf, ZGrid zf, int first, const unsigned char *__restrict__ rowf,
+                                                  const T *__restrict__ xc, T *__restrict__ x)
 {
-    long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-    if (t >= gf.n) return;
-    if (!rowf[t]) return;
-    const int t32 = (int)t; int i = t32 % gf.mx; int r = t32 / gf.mx; int j = r % gf.my, k = r / gf.my;
-    int I = (i + 1) / 2, J = (j + 1) / 2, K = (k + 1) / 2;
-    int I2 = parent_nb(I, (i & 1) ? -1 : 1, gc.mx, gc.pi);
-    int J2 = parent_nb(J, (j & 1) ? -1 : 1, gc.my, gc.pj);
-    int K2 = parent_nb(K, (k & 1) ? -1 : 1, gc.mz, gc.pk);
-#define XC(kk, jj, ii) xc[((long long)(kk) * gc.my + (jj)) * gc.mx + (ii)]
-    T v = T(27) * XC(K, J, I) + T(9) * (XC(K, J, I2) + XC(K, J2, I) + XC(K2, J, I)) +
-          T(3) * (XC(K, J2, I2) + XC(K2, J, I2) + XC(K2, J2, I)) + XC(K2, J2, I2);
-#undef XC
-    xf[t] += v / T(64);
-}
-
-// k_prolong on a fine iterate in the S layout: one thread per S position,
-// the same interpolation expression
-template <typename T>
-__global__ void k_prolong_split(Grid gc, Grid gf, ZGrid zf, const unsigned char *__restrict__ rowf, const T *__restrict__ xc,
-                                T *__restrict__ xs)
-{
-    const unsigned t = blockIdx.x * blockDim.x + threadIdx.x;
     const unsigned cp = (unsigned)zf.cplane, nh = (unsigned)zf.nh, nj = (unsigned)zf.njI;
+    const unsigned t = blockIdx.x * blockDim.x + threadIdx.x + first * cp;
     if (t >= 2 * cp) return;
     const unsigned col = t >= cp ? 1u : 0u;
     const unsigned rem = t - col * cp;
@@ -1061,7 +1066,8 @@ __global__ void k_prolong_split(Grid gc, Grid gf, ZGrid zf, const unsigned char 
     const int j = (int)jj + 1, k = (int)kk + 1;
     const int i = zebra_i0(k, (int)col) + 2 * (int)h;
     if (i > gf.mx - 2) return;
-    if (!rowf[((long long)k * gf.my + j) * gf.mx + i]) return;
+    const long long q = ((long long)k * gf.my + j) * gf.mx + i;
+    if (!rowf[q]) return;
     int I = (i + 1) / 2, J = (j + 1) / 2, K = (k + 1) / 2;
     int I2 = parent_nb(I, (i & 1) ? -1 : 1, gc.mx, gc.pi);
     int J2 = parent_nb(J, (j & 1) ? -1 : 1, gc.my, gc.pj);
@@ -1070,7 +1076,7 @@ __global__ void k_prolong_split(Grid gc, Grid gf, ZGrid zf, const unsigned char 
     T v = T(27) * XC(K, J, I) + T(9) * (XC(K, J, I2) + XC(K, J2, I) + XC(K2, J, I)) +
           T(3) * (XC(K, J2, I2) + XC(K2, J, I2) + XC(K2, J2, I)) + XC(K2, J2, I2);
 #undef XC
-    xs[t] += v / T(64);
+    x[SPL ? (long long)t : q] += v / T(64);
 }
 
 // natural FP64 v -> S-layout FP32 (the finest right-hand side)
@@ -1811,19 +1817,19 @@ static void vcycle(vfs_ctx *c, vfs_poisson *ps, int l, const Sweeps &S)
     // The residual is formed inside the restriction (k_residual_restrict)
     // unless VFS_MG_FUSED_RESTRICT=0 asks for the stored-residual form.
     PLevel &C = ps->L[l + 1];
-    const unsigned nbc = blocks_for(C.g.n, PTPB);
+    const unsigned nbc = blocks_for(C.g.n, PTPB), nbr = blocks_for(C.g.n, RR_PTS);
     const char *fr = std::getenv("VFS_MG_FUSED_RESTRICT");
     const bool axis = sizeof(T) == 4 && L.compact;
     if (spl) {
         if constexpr (sizeof(T) == 4)
-            hipLaunchKernelGGL((k_residual_restrict<float, 7, true>), dim3(nbc), dim3(PTPB), 0, st, C.g, L.g, L.c32, C.row, L.row,
+            hipLaunchKernelGGL((k_residual_restrict<float, 7, true>), dim3(nbr), dim3(4 * RR_PTS), 0, st, C.g, L.g, L.c32, C.row, L.row,
                                (const float *)L.xs32, (const float *)L.bs32, C.b32, L.z);
     } else if (!(fr && fr[0] == '0')) {
         if (axis)
-            hipLaunchKernelGGL((k_residual_restrict<T, 7>), dim3(nbc), dim3(PTPB), 0, st, C.g, L.g, LV<T>::coef(L), C.row, L.row,
+            hipLaunchKernelGGL((k_residual_restrict<T, 7>), dim3(nbr), dim3(4 * RR_PTS), 0, st, C.g, L.g, LV<T>::coef(L), C.row, L.row,
                                (const T *)LV<T>::x(L), (const T *)LV<T>::b(L), LV<T>::b(C), L.z);
         else
-            hipLaunchKernelGGL((k_residual_restrict<T, NST>), dim3(nbc), dim3(PTPB), 0, st, C.g, L.g, LV<T>::coef(L), C.row,
+            hipLaunchKernelGGL((k_residual_restrict<T, NST>), dim3(nbr), dim3(4 * RR_PTS), 0, st, C.g, L.g, LV<T>::coef(L), C.row,
                                L.row, (const T *)LV<T>::x(L), (const T *)LV<T>::b(L), LV<T>::b(C), L.z);
     } else {
         if (axis)
@@ -1841,12 +1847,16 @@ static void vcycle(vfs_ctx *c, vfs_poisson *ps, int l, const Sweeps &S)
             hipLaunchKernelGGL(k_zero<T>, dim3(blocks_for(C.g.n, PTPB)), dim3(PTPB), 0, st, C.g.n, LV<T>::x(C));
         vcycle<T>(c, ps, l + 1, S);
     }
+    // colour 0 needs no correction where the half-sweep that follows does not read it
+    const int first = post > 0 && line_plan<T>(L).fused ? 1 : 0;
+    const dim3 np(blocks_for((2 - first) * L.z.cplane, PTPB));
     if (spl) {
         if constexpr (sizeof(T) == 4)
-            hipLaunchKernelGGL(k_prolong_split<float>, dim3(blocks_for(2 * L.z.cplane, PTPB)), dim3(PTPB), 0, st, C.g, L.g, L.z,
-                               L.row, (const float *)C.x32, L.xs32);
+            hipLaunchKernelGGL((k_prolong<float, true>), np, dim3(PTPB), 0, st, C.g, L.g, L.z, first, L.row, (const float *)C.x32,
+                               L.xs32);
     } else {
-        hipLaunchKernelGGL(k_prolong<T>, dim3(nb), dim3(PTPB), 0, st, C.g, L.g, L.row, LV<T>::x(C), LV<T>::x(L));
+        hipLaunchKernelGGL((k_prolong<T, false>), np, dim3(PTPB), 0, st, C.g, L.g, L.z, first, L.row, (const T *)LV<T>::x(C),
+                           LV<T>::x(L));
     }
     smooth<T>(c, L, post);
 }
