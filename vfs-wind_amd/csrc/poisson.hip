@@ -1651,7 +1651,11 @@ static LinePlan line_plan(const PLevel &L)
     // on the finest level the one-pass kernel takes 16-point segments and 64
     // lines per block up to 256-point lines (a segment row is a whole
     // wavefront; the coarse levels, which fill fewer blocks, keep 8 and 32)
-    if (fusable && L.finest && L.z.njI <= line_slm<float>() * 16) p.short_seg = false;
+    // where that leaves two blocks per CU: 52 against 54 us per half-sweep at
+    // 256x192x256, but with fewer lines the shorter, more numerous blocks of
+    // the coarse levels are faster (11 against 8 us at 64x48x64; whole solves
+    // 2.73 -> 2.48 ms there, 10.2 -> 9.7 ms at 192x144x192)
+    if (fusable && L.finest && L.z.njI <= line_slm<float>() * 16 && (long long)L.z.nkI * L.z.nh >= 64 * 512) p.short_seg = false;
     if (force == 1) p.short_seg = sizeof(T) == 4;
     if (force == 2) p.short_seg = false;
     const int slm = p.short_seg ? LINE_SLM_SHORT : SLM;
