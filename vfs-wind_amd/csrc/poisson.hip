@@ -1047,6 +1047,20 @@ __device__ inline int parent_nb(int I, int d, int mc, int per)
     return J;
 }
 
+// 64 x the trilinear interpolation of the coarse xc at fine point (k, j, i)
+template <typename T>
+__device__ inline T trilinear(const Grid &gc, const T *__restrict__ xc, int k, int j, int i)
+{
+    int I = (i + 1) / 2, J = (j + 1) / 2, K = (k + 1) / 2;
+    int I2 = parent_nb(I, (i & 1) ? -1 : 1, gc.mx, gc.pi);
+    int J2 = parent_nb(J, (j & 1) ? -1 : 1, gc.my, gc.pj);
+    int K2 = parent_nb(K, (k & 1) ? -1 : 1, gc.mz, gc.pk);
+#define XC(kk, jj, ii) xc[((long long)(kk) * gc.my + (jj)) * gc.mx + (ii)]
+    return T(27) * XC(K, J, I) + T(9) * (XC(K, J, I2) + XC(K, J2, I) + XC(K2, J, I)) +
+           T(3) * (XC(K, J2, I2) + XC(K2, J, I2) + XC(K2, J2, I)) + XC(K2, J2, I2);
+#undef XC
+}
+
 // fine x += trilinear(coarse x) at the points of the colours from `first` on,
 // one thread per S position; the iterate in the S layout (SPL) or the natural
 // one.  Where the next half-sweep (colour 0) reads only colour 1 and rewrites
@@ -1068,15 +1082,522 @@ __global__ void __launch_bounds__(PTPB) k_prolong(Grid gc, Grid gf, ZGrid zf, in
     if (i > gf.mx - 2) return;
     const long long q = ((long long)k * gf.my + j) * gf.mx + i;
     if (!rowf[q]) return;
-    int I = (i + 1) / 2, J = (j + 1) / 2, K = (k + 1) / 2;
-    int I2 = parent_nb(I, (i & 1) ? -1 : 1, gc.mx, gc.pi);
-    int J2 = parent_nb(J, (j & 1) ? -1 : 1, gc.my, gc.pj);
-    int K2 = parent_nb(K, (k & 1) ? -1 : 1, gc.mz, gc.pk);
-#define XC(kk, jj, ii) xc[((long long)(kk) * gc.my + (jj)) * gc.mx + (ii)]
-    T v = T(27) * XC(K, J, I) + T(9) * (XC(K, J, I2) + XC(K, J2, I) + XC(K2, J, I)) +
-          T(3) * (XC(K, J2, I2) + XC(K2, J, I2) + XC(K2, J2, I)) + XC(K2, J2, I2);
-#undef XC
-    x[SPL ? (long long)t : q] += v / T(64);
+    x[SPL ? (long long)t : q] += trilinear(gc, xc, k, j, i) / T(64);
+}
+
+// Smoothing sweeps of a V-cycle: pre and post on the levels below
+// deep_level, deep_pre and deep_post from deep_level on (deep_level 0: every
+// level takes pre and post), coarse on a coarsest level without a dense solve.
+struct Sweeps {
+    int pre, post, coarse, deep_level, deep_pre, deep_post;
+    __host__ __device__ int pre_at(int l) const { return deep_level > 0 && l >= deep_level ? deep_pre : pre; }
+    __host__ __device__ int post_at(int l) const { return deep_level > 0 && l >= deep_level ? deep_post : post; }
+    bool operator==(const Sweeps &o) const
+    {
+        return pre == o.pre && post == o.post && coarse == o.coarse && deep_level == o.deep_level && deep_pre == o.deep_pre &&
+               deep_post == o.deep_post;
+    }
+};
+
+// ---- the small levels of a V-cycle in one block ------------------------------
+// Levels from the first one on whose vectors fit a workgroup's LDS run in one
+// launch: smoothing, residual restriction, prolongation and the coarsest solve
+// with block barriers where the separate kernels have launches.  Every value is
+// formed by the separate kernels' expressions in their order, so the cycle has
+// the same bits.  x, b, the row mask of each level and one residual live in LDS
+// (natural layout); coefficients are read from L2.  What bounds it is the chain
+// of latencies: a compact level's coefficients stay in registers over the sweeps
+// of one smoothing (both colours: 96 registers, hence at most 512 threads), and
+// the other forms compute their right-hand sides with one thread per point.
+// One V-cycle of a 16x12x16 grid: 43 us against 26 launches of 4 to 6 us; the
+// 16x12x16 and 8x6x8 levels of a 256x192x256 hierarchy, cold: 51 us against 13
+// launches of about 4 us; 16x12x16 in FP64: 102 us against 38 launches.
+constexpr int TAIL_T = 512, TAIL_DENSE = 448;  // threads; rows of the largest dense level taken
+constexpr int TAIL_LDS = 144 * 1024;           // dynamic LDS (8 KB more hold the line maps)
+template <typename T>
+struct TailLevel {
+    Grid g;
+    ZGrid z;
+    const T *coef;             // 19 planes
+    const unsigned char *row;
+    const h2_t *sh;            // FP32 smoother: ratios (compact: h4_t words) and diagonal
+    const float *sd;
+    const T *sc;               // FP64 smoother: off-line planes
+    const T *sf;               // Thomas factor planes
+    int compact, nseg, sl;
+    int xo, bo, wo;            // LDS offsets of x and b (elements) and of the row mask (bytes)
+    int nr;                    // dense rows (coarsest level)
+    const int *ridx;
+    const T *inv;
+};
+template <typename T>
+struct TailLds {
+    T *v;                      // x and b of the levels
+    T *res;                    // one residual or right-hand side
+    T *sA, *sB;                // segment maps
+    unsigned char *row;
+};
+
+// a pointer from a descriptor as one to global memory: without it the loads
+// are flat ones, which wait for LDS reads too
+template <typename P>
+__device__ __forceinline__ const __attribute__((address_space(1))) P *in_hbm(const P *p)
+{
+    return (const __attribute__((address_space(1))) P *)p;
+}
+
+// t / d for inv = 1.f / d: exact for t < 2^22 (the half keeps a multiple of d
+// above its quotient by 0.5 / d, more than the product's rounding)
+__device__ inline int tail_div(int t, float inv) { return (int)(((float)t + 0.5f) * inv); }
+// nat_decode with it
+struct TailDecode {
+    int mx, my;
+    float ix, iy;
+    __device__ TailDecode(int mx_, int my_) : mx(mx_), my(my_), ix(1.f / (float)mx_), iy(1.f / (float)my_) {}
+    __device__ void operator()(int t, int &k, int &j, int &i) const
+    {
+        const int r = tail_div(t, ix);
+        i = t - r * mx;
+        k = tail_div(r, iy);
+        j = r - k * my;
+    }
+};
+
+// this thread's segment of a level's lines
+struct TailTask {
+    int nlines, seg, line, k, h, j0, j1, base, nseg;
+    bool task;
+};
+template <typename T>
+__device__ __forceinline__ TailTask tail_task(const TailLevel<T> &L)
+{
+    TailTask t;
+    t.nlines = L.z.nkI * L.z.nh;
+    t.nseg = L.nseg;
+    t.seg = (int)threadIdx.x / t.nlines;
+    t.line = (int)threadIdx.x - t.seg * t.nlines;
+    const int kk = t.line / L.z.nh;
+    t.h = t.line - kk * L.z.nh;
+    t.k = kk + 1;
+    t.j0 = t.seg * L.sl;
+    t.j1 = t.j0 + L.sl < L.z.njI ? t.j0 + L.sl : L.z.njI;
+    t.base = (kk * L.z.njI + t.j0) * L.z.nh + t.h;  // colour-local index of the segment's first point
+    t.task = (int)threadIdx.x < t.nlines * L.nseg;
+    return t;
+}
+
+// k_zebra_scan's segmented solve: r holds the segment's right-hand sides; the
+// line's new values go to x (xp + v * stride).  A segment of fewer than eight
+// points is padded with points that hand their carry on unchanged (factors -1,
+// 1, -1 and right-hand side 0).  Wavefronts without a task only meet the
+// barriers.
+template <typename T>
+__device__ __forceinline__ void tail_solve(const TailTask &t, const TailLds<T> &M, T (&r)[8], const T (&l)[8], const T (&m)[8],
+                                           const T (&u)[8], bool act, T *__restrict__ xp, int stride)
+{
+    constexpr int SLM = 8;
+    const int tid = threadIdx.x;
+    if (t.task && t.nseg > 1) {
+        T A = 1, B = 0;
+#pragma unroll
+        for (int v = 0; v < SLM; v++) {
+            B = (r[v] - l[v] * B) * m[v];
+            A = (-l[v] * A) * m[v];
+        }
+        M.sA[tid] = A;
+        M.sB[tid] = B;
+    }
+    if (t.nseg > 1) __syncthreads();
+    if (t.task) {
+        T d = 0;
+        for (int s = 0; s < t.seg; s++) d = M.sA[s * t.nlines + t.line] * d + M.sB[s * t.nlines + t.line];
+#pragma unroll
+        for (int v = 0; v < SLM; v++) {
+            d = (r[v] - l[v] * d) * m[v];
+            r[v] = v < t.j1 - t.j0 ? d : T(0);
+        }
+    }
+    if (t.nseg > 1) {
+        __syncthreads();
+        if (t.task) {
+            T A = 1, B = 0;
+#pragma unroll
+            for (int v = SLM - 1; v >= 0; v--) {
+                B = r[v] - u[v] * B;
+                A = -u[v] * A;
+            }
+            M.sA[tid] = A;
+            M.sB[tid] = B;
+        }
+        __syncthreads();
+    }
+    if (t.task) {
+        T xl = 0;
+        for (int s = t.nseg - 1; s > t.seg; s--) xl = M.sA[s * t.nlines + t.line] * xl + M.sB[s * t.nlines + t.line];
+        const int np = act ? t.j1 - t.j0 : 0;
+#pragma unroll
+        for (int v = SLM - 1; v >= 0; v--) {
+            xl = r[v] - u[v] * xl;
+            if (v < np) xp[v * stride] = xl;
+        }
+    }
+    __syncthreads();
+}
+
+// the Thomas factors of the segment, padded
+template <typename T>
+__device__ __forceinline__ void tail_factors(const TailLevel<T> &L, const TailTask &t, int c, bool act, T (&l)[8], T (&m)[8], T (&u)[8])
+{
+    const unsigned cplane = (unsigned)L.z.cplane, ss = 2 * cplane, nh = (unsigned)L.z.nh;
+    const int np = act ? t.j1 - t.j0 : 0;
+    const unsigned q0 = c * cplane + (np > 0 ? (unsigned)t.base : 0u);
+    const auto *sf = in_hbm(L.sf);
+#pragma unroll
+    for (int v = 0; v < 8; v++) {
+        const unsigned cq = q0 + (v < np ? v * nh : 0u);
+        l[v] = sf[cq];
+        m[v] = sf[ss + cq];
+        u[v] = sf[2 * ss + cq];
+    }
+#pragma unroll
+    for (int v = 0; v < 8; v++)
+        if (v >= np) {
+            l[v] = u[v] = -1;
+            m[v] = 1;
+        }
+}
+
+// a compact segment's coefficients of one colour
+struct TailC4 {
+    h4_t w[8];
+    float d[8], l[8], m[8], u[8];
+};
+__device__ __forceinline__ void tail_c4_load(const TailLevel<float> &L, const TailTask &t, int c, TailC4 &s)
+{
+    const bool act = t.task && zebra_i0(t.k, c) + 2 * t.h <= L.g.mx - 2;
+    const int np = act ? t.j1 - t.j0 : 0;
+    const unsigned q0 = c * (unsigned)L.z.cplane + (np > 0 ? (unsigned)t.base : 0u), nh = (unsigned)L.z.nh;
+#pragma unroll
+    for (int v = 0; v < 8; v++) {
+        const unsigned cq = q0 + (v < np ? v * nh : 0u);
+        s.w[v] = in_hbm(reinterpret_cast<const h4_t *>(L.sh))[cq];
+        s.d[v] = in_hbm(L.sd)[cq];
+    }
+    tail_factors<float>(L, t, c, act, s.l, s.m, s.u);
+#pragma unroll
+    for (int v = 0; v < 8; v++)
+        if (v >= np) s.d[v] = 0;
+}
+__device__ __forceinline__ void tail_c4_half(const TailLevel<float> &L, const TailTask &t, const TailLds<float> &M, int c,
+                                             const TailC4 &s)
+{
+    const Grid &g = L.g;
+    const int plane = (int)g.plane, i = zebra_i0(t.k, c) + 2 * t.h;
+    const bool act = t.task && i <= g.mx - 2;
+    float *x = M.v + L.xo;
+    const int at = t.k * plane + (t.j0 + 1) * g.mx;
+    float r[8];
+    if (t.task) {
+        const int np = act ? t.j1 - t.j0 : 0, ic = act ? i : 1;
+        const float *x0 = x + at, *b0 = M.v + L.bo + at + ic;
+        const float *xe = x0 + canon(ic + 1, g.mx, g.pi), *xw = x0 + canon(ic - 1, g.mx, g.pi);
+        const float *xt = x0 + (canon(t.k + 1, g.mz, g.pk) - t.k) * plane + ic, *xb = x0 + (canon(t.k - 1, g.mz, g.pk) - t.k) * plane + ic;
+#pragma unroll
+        for (int v = 0; v < 8; v++) {
+            const int o = v < t.j1 - t.j0 ? v * g.mx : 0;
+            const float rv = c4_sum(s.w[v], s.d[v], xe[o], xw[o], xt[o], xb[o], b0[o]);
+            r[v] = v < np ? rv : 0.f;
+        }
+    }
+    tail_solve<float>(t, M, r, s.l, s.m, s.u, act, x + at + i, g.mx);
+}
+
+// a half-sweep of the full FP32 or the FP64 form: right-hand sides with one
+// thread per point into M.res (colour-local order), then the line solve
+template <typename T>
+__device__ __forceinline__ void tail_full_half(const TailLevel<T> &L, const TailTask &t, const TailLds<T> &M, int c)
+{
+    const Grid &g = L.g;
+    const ZGrid &z = L.z;
+    const int plane = (int)g.plane, cplane = (int)z.cplane;
+    const unsigned ss = 2 * (unsigned)cplane;
+    const int i = zebra_i0(t.k, c) + 2 * t.h;
+    const bool act = t.task && i <= g.mx - 2;
+    T *x = M.v + L.xo;
+    const T *b = M.v + L.bo;
+    T l[8], m[8], u[8], r[8];
+    if (t.task) tail_factors<T>(L, t, c, act, l, m, u);
+    const float inh = 1.f / (float)z.nh, inj = 1.f / (float)z.njI;
+    for (int q = threadIdx.x; q < cplane; q += TAIL_T) {
+        const int row = tail_div(q, inh), kk = tail_div(row, inj), j = row - kk * z.njI + 1, k = kk + 1;
+        const int iq = zebra_i0(k, c) + 2 * (q - row * z.nh);
+        const unsigned cq = (unsigned)(c * cplane + q);
+        if (iq > g.mx - 2) continue;
+        const int I[3] = {canon(iq - 1, g.mx, g.pi), iq, canon(iq + 1, g.mx, g.pi)};
+        const int J[3] = {canon(j - 1, g.my, g.pj) * g.mx, j * g.mx, canon(j + 1, g.my, g.pj) * g.mx};
+        const int K[3] = {canon(k - 1, g.mz, g.pk) * plane, k * plane, canon(k + 1, g.mz, g.pk) * plane};
+        const T bq = b[K[1] + J[1] + iq];
+        if constexpr (sizeof(T) == 4) {
+            h2_t w[NOFF / 2];
+#pragma unroll
+            for (int p = 0; p < NOFF / 2; p++) w[p] = in_hbm(L.sh)[p * ss + cq];
+            const float dq = in_hbm(L.sd)[cq];
+            float acc = 0;
+#pragma unroll
+            for (int p = 0; p < NOFF; p++) {
+                const int s = offline_slot(p);
+                acc += (float)((p & 1) ? w[p / 2].y : w[p / 2].x) * x[K[soff(s, 2) + 1] + J[soff(s, 1) + 1] + I[soff(s, 0) + 1]];
+            }
+            M.res[q] = bq - dq * acc;
+        } else {
+            T w[NOFF], acc = bq;
+#pragma unroll
+            for (int p = 0; p < NOFF; p++) w[p] = in_hbm(L.sc)[p * ss + cq];
+#pragma unroll
+            for (int p = 0; p < NOFF; p++) {
+                const int s = offline_slot(p);
+                acc -= w[p] * x[K[soff(s, 2) + 1] + J[soff(s, 1) + 1] + I[soff(s, 0) + 1]];
+            }
+            M.res[q] = acc;
+        }
+    }
+    __syncthreads();
+    if (t.task) {
+        const int np = act ? t.j1 - t.j0 : 0;
+#pragma unroll
+        for (int v = 0; v < 8; v++) {
+            const T rv = M.res[v < np ? t.base + v * z.nh : 0];
+            r[v] = v < np ? rv : T(0);
+        }
+    }
+    tail_solve<T>(t, M, r, l, m, u, act, x + t.k * plane + (t.j0 + 1) * g.mx + i, g.mx);
+}
+
+template <typename T, bool C4>
+__device__ __forceinline__ void tail_smooth(const TailLevel<T> &L, const TailLds<T> &M, int sweeps)
+{
+    if (sweeps < 1) return;
+    const TailTask t = tail_task<T>(L);
+    if constexpr (C4) {
+        TailC4 s0, s1;
+        if (t.task) {
+            tail_c4_load(L, t, 0, s0);
+            tail_c4_load(L, t, 1, s1);
+        }
+        for (int s = 0; s < sweeps; s++) {
+            tail_c4_half(L, t, M, 0, s0);
+            tail_c4_half(L, t, M, 1, s1);
+        }
+    } else {
+        for (int hs = 0; hs < 2 * sweeps; hs++) tail_full_half<T>(L, t, M, hs & 1);
+    }
+}
+
+// the residual of every row of L (its first NQ stencil slots) into M.res, the
+// coefficients of U points in flight
+template <typename T, int NQ, int U>
+__device__ __forceinline__ void tail_residual(const TailLevel<T> &L, const TailLds<T> &M)
+{
+    const Grid &g = L.g;
+    const T *x = M.v + L.xo, *b = M.v + L.bo;
+    const unsigned char *row = M.row + L.wo;
+    const unsigned n = (unsigned)g.n;
+    const int mx = g.mx, plane = (int)g.plane, ni = (mx - 2) * (g.my - 2) * (g.mz - 2);
+    const TailDecode dec(mx - 2, g.my - 2);
+    for (int t0 = threadIdx.x; t0 < ni; t0 += U * TAIL_T) {
+        T w[U][NQ];
+        int kk[U], jj[U], ii[U];
+        bool rows[U];
+#pragma unroll
+        for (int e = 0; e < U; e++) {
+            const int t = t0 + e * TAIL_T;
+            dec(t < ni ? t : 0, kk[e], jj[e], ii[e]);
+            const int q0 = ++kk[e] * plane + ++jj[e] * mx + ++ii[e];
+            rows[e] = t < ni && row[q0];
+#pragma unroll
+            for (int q = 0; q < NQ; q++) w[e][q] = in_hbm(L.coef)[q * n + (unsigned)q0];
+        }
+#pragma unroll
+        for (int e = 0; e < U; e++) {
+            if (!rows[e]) continue;
+            const int k = kk[e], j = jj[e], i = ii[e], t = k * plane + j * mx + i;
+            const int I[3] = {canon(i - 1, mx, g.pi), i, canon(i + 1, mx, g.pi)};
+            const int J[3] = {canon(j - 1, g.my, g.pj) * mx, j * mx, canon(j + 1, g.my, g.pj) * mx};
+            const int K[3] = {canon(k - 1, g.mz, g.pk) * plane, k * plane, canon(k + 1, g.mz, g.pk) * plane};
+            T a = 0;
+#pragma unroll
+            for (int q = 0; q < NQ; q++) a += w[e][q] * x[K[soff(q, 2) + 1] + J[soff(q, 1) + 1] + I[soff(q, 0) + 1]];
+            M.res[t] = b[t] - a;
+        }
+    }
+}
+
+// k_dense_solve's sums: sixteen column slices per row, added in order
+template <typename T>
+__device__ __forceinline__ void tail_dense(const TailLevel<T> &L, const TailLds<T> &M)
+{
+    constexpr int RB = TAIL_DENSE / DENSE_ROWS, SL = DENSE_ROWS * DENSE_SPLIT / TAIL_T;
+    static_assert(SL * TAIL_T == DENSE_ROWS * DENSE_SPLIT, "whole slices of 64 rows per wavefront");
+    const int tid = threadIdx.x, lr = tid % DENSE_ROWS, grp = tid / DENSE_ROWS;
+    for (int c = tid; c < L.nr; c += TAIL_T) M.res[c] = M.v[L.bo + in_hbm(L.ridx)[c]];
+    __syncthreads();
+    const int nr = L.nr, chunk = (nr + DENSE_SPLIT - 1) / DENSE_SPLIT;
+    const auto *inv = in_hbm(L.inv);
+    T acc[SL][RB];
+    unsigned at[RB];
+    int c0[SL], cn[SL];
+#pragma unroll
+    for (int q = 0; q < RB; q++) at[q] = (unsigned)(q * DENSE_ROWS + lr < nr ? q * DENSE_ROWS + lr : 0);
+#pragma unroll
+    for (int p = 0; p < SL; p++) {
+        c0[p] = (p * (TAIL_T / DENSE_ROWS) + grp) * chunk;
+        cn[p] = nr - c0[p] < chunk ? nr - c0[p] : chunk;
+#pragma unroll
+        for (int q = 0; q < RB; q++) acc[p][q] = 0;
+    }
+    // Four columns at a time, every load unconditional (rows and columns past
+    // the end read element 0): 56 loads in flight per thread.  One column at a
+    // time the 384 rows of a 256x192x256 hierarchy took 142 us, cold.
+    constexpr int CU = 4;
+    for (int c = 0; c < chunk; c += CU) {
+        T v[CU][SL][RB];
+#pragma unroll
+        for (int e = 0; e < CU; e++)
+#pragma unroll
+            for (int p = 0; p < SL; p++) {
+                const unsigned col = c + e < cn[p] ? (unsigned)(c0[p] + c + e) * (unsigned)nr : 0u;
+#pragma unroll
+                for (int q = 0; q < RB; q++) v[e][p][q] = inv[col + at[q]];
+            }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int e = 0; e < CU; e++)
+#pragma unroll
+            for (int p = 0; p < SL; p++) {
+                const bool in = c + e < cn[p];
+                const T bs = M.res[in ? c0[p] + c + e : 0];
+#pragma unroll
+                for (int q = 0; q < RB; q++) acc[p][q] = in ? acc[p][q] + v[e][p][q] * bs : acc[p][q];
+            }
+    }
+#pragma unroll
+    for (int q = 0; q < RB; q++) {
+        if (q * DENSE_ROWS < L.nr) {
+            // the slices 0 .. 7 in sA, 8 .. 15 in sB
+            M.sA[tid] = acc[0][q];
+            M.sB[tid] = acc[1][q];
+            __syncthreads();
+            const int r = q * DENSE_ROWS + lr;
+            if (grp == 0 && r < L.nr) {
+                T s = M.sA[lr];
+                for (int p = 1; p < DENSE_SPLIT; p++) s += p < 8 ? M.sA[p * DENSE_ROWS + lr] : M.sB[(p - 8) * DENSE_ROWS + lr];
+                M.v[L.xo + in_hbm(L.ridx)[r]] = s;
+            }
+            __syncthreads();
+        }
+    }
+}
+static_assert(TAIL_T == 512 && DENSE_ROWS * DENSE_SPLIT == 1024, "tail_dense keeps eight slices in each map array");
+
+// C4: every level takes the compact form.  The cycle's steps are one loop over
+// the levels down and up again, so that each part's code is there once (a cold
+// instruction cache costs more than the work on a large grid's small levels).
+template <typename T, bool C4>
+__global__ void __launch_bounds__(TAIL_T) k_mg_tail(const TailLevel<T> *__restrict__ levels, int nl, int first, Sweeps S, int ro,
+                                                    int wo, const T *__restrict__ b_in, T *__restrict__ x_out)
+{
+    extern __shared__ char smem[];
+    __shared__ T sA[TAIL_T], sB[TAIL_T];
+    const TailLds<T> M = {reinterpret_cast<T *>(smem), reinterpret_cast<T *>(smem) + ro, sA, sB,
+                          reinterpret_cast<unsigned char *>(smem) + wo};
+    const int tid = threadIdx.x;
+    // bring the dense inverse into this XCD's L2 (a line per load); the sum is
+    // only there to keep the loads
+    const unsigned ninv = (unsigned)(levels[nl - 1].nr * levels[nl - 1].nr);
+    constexpr unsigned LINE = 128 / sizeof(T);
+    T touched = 0;
+    for (unsigned q0 = tid * LINE; q0 < ninv; q0 += 8 * TAIL_T * LINE) {
+        T v[8];
+#pragma unroll
+        for (unsigned e = 0; e < 8; e++) v[e] = in_hbm(levels[nl - 1].inv)[q0 + e * TAIL_T * LINE < ninv ? q0 + e * TAIL_T * LINE : q0];
+#pragma unroll
+        for (int e = 0; e < 8; e++) touched += v[e];
+    }
+    if (touched == T(1.25e38)) x_out[0] = touched;  // (written again at the end)
+    for (int l = 0; l < nl; l++) {
+        const TailLevel<T> &L = levels[l];
+        const unsigned n = (unsigned)L.g.n;
+        for (unsigned t0 = tid; t0 < n; t0 += 4 * TAIL_T) {
+            T bv[4];
+            unsigned char rv[4];
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const unsigned t = t0 + e * TAIL_T < n ? t0 + e * TAIL_T : t0;
+                bv[e] = b_in[l == 0 ? t : 0u];
+                rv[e] = in_hbm(L.row)[t];
+            }
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const unsigned t = t0 + e * TAIL_T < n ? t0 + e * TAIL_T : t0;
+                M.v[L.xo + t] = 0;
+                M.v[L.bo + t] = bv[e];
+                M.row[L.wo + t] = rv[e];
+            }
+        }
+    }
+    __syncthreads();
+    for (int p = 0; p < 2 * nl - 1; p++) {
+        const bool down = p < nl - 1, up = p >= nl;
+        const int l = up ? 2 * nl - 2 - p : p;
+        const TailLevel<T> &L = levels[l];
+        if (up) {
+            // the interpolated correction of level l + 1
+            const TailLevel<T> &C = levels[l + 1];
+            const Grid &gc = C.g, &gf = L.g;
+            const T *xc = M.v + C.xo;
+            // (a compact level's colour 0 needs none: see k_prolong)
+            const int post = S.post_at(first + l);
+            const int c0 = C4 && post > 0 && zebra_fused_ok(gf) ? 1 : 0, np = (int)L.z.cplane;
+            const TailDecode dec(L.z.nh, L.z.njI);
+            for (int c = c0; c < 2; c++)
+                for (int q = tid; q < np; q += TAIL_T) {
+                    int kk, jj, h;
+                    dec(q, kk, jj, h);
+                    const int k = kk + 1, j = jj + 1, i = zebra_i0(k, c) + 2 * h, t = (k * gf.my + j) * gf.mx + i;
+                    if (i > gf.mx - 2 || !M.row[L.wo + t]) continue;
+                    M.v[L.xo + t] += trilinear(gc, xc, k, j, i) / T(64);
+                }
+            __syncthreads();
+        }
+        if (!down && !up && L.nr > 0) tail_dense<T>(L, M);
+        else tail_smooth<T, C4>(L, M, down ? S.pre_at(first + l) : up ? S.post_at(first + l) : S.coarse);
+        if (down) {
+            if (C4 || (sizeof(T) == 4 && L.compact)) tail_residual<T, 7, 3>(L, M);
+            else tail_residual<T, NST, sizeof(T) == 4 ? 2 : 1>(L, M);
+            __syncthreads();
+            const TailLevel<T> &C = levels[l + 1];
+            const Grid &gc = C.g, &gf = L.g;
+            const unsigned char *rowf = M.row + L.wo;
+            const TailDecode dec(gc.mx, gc.my);
+            for (int t = tid; t < (int)gc.n; t += TAIL_T) {
+                T s = 0;
+                if (M.row[C.wo + t]) {
+                    int k, j, i;
+                    dec(t, k, j, i);
+                    const int q0 = ((2 * k - 1) * gf.my + 2 * j - 1) * gf.mx + 2 * i - 1;
+#pragma unroll
+                    for (int r = 0; r < 8; r++) {
+                        const int qf = q0 + (r >> 2) * (int)gf.plane + ((r >> 1) & 1) * gf.mx + (r & 1);
+                        const T v = M.res[qf];
+                        s += rowf[qf] ? v : T(0);
+                    }
+                }
+                M.v[C.bo + t] = s;
+            }
+            __syncthreads();
+        }
+    }
+    for (int t = tid; t < (int)levels[0].g.n; t += TAIL_T) x_out[t] = M.v[levels[0].xo + t];
 }
 
 // natural FP64 v -> S-layout FP32 (the finest right-hand side)
@@ -1269,25 +1790,12 @@ struct PLevel {
     double *inv64 = nullptr;
 };
 
-// a captured coarse sub-cycle (levels 1..nl-1 of one V-cycle) and the
-// smoothing counts it was captured with
-// Smoothing sweeps of a V-cycle: pre and post on the levels below
-// deep_level, deep_pre and deep_post from deep_level on (deep_level 0: every
-// level takes pre and post), coarse on a coarsest level without a dense solve.
-struct Sweeps {
-    int pre, post, coarse, deep_level, deep_pre, deep_post;
-    int pre_at(int l) const { return deep_level > 0 && l >= deep_level ? deep_pre : pre; }
-    int post_at(int l) const { return deep_level > 0 && l >= deep_level ? deep_post : post; }
-    bool operator==(const Sweeps &o) const
-    {
-        return pre == o.pre && post == o.post && coarse == o.coarse && deep_level == o.deep_level && deep_pre == o.deep_pre &&
-               deep_post == o.deep_post;
-    }
-};
-
+// a captured coarse sub-cycle (levels 1..nl-1 of one V-cycle), the smoothing
+// counts and the first level of the one-block part it was captured with
 struct SubGraph {
     hipGraphExec_t exec = nullptr;
-    Sweeps key{-1, -1, -1, -1, -1, -1};
+    vfs::Sweeps key{-1, -1, -1, -1, -1, -1};
+    int tail = -1;
 };
 
 namespace vfs {
@@ -1299,6 +1807,12 @@ void amg_free(AmgDev *a);
 double amg_theta(const AmgDev *a);
 }  // namespace vfs
 
+// first level of the one-block part of a V-cycle (nl when there is none) and
+// its LDS: offsets of the residual (elements) and of the row masks (bytes)
+struct TailPlan {
+    int first = 8, ro = 0, wo = 0, lds = 0, compact = 0;
+};
+
 struct vfs_poisson {
     vfs::AmgDev *amg = nullptr;  // algebraic multigrid hierarchy of level 0 (when requested)
     int nl = 0;          // levels built
@@ -1308,6 +1822,9 @@ struct vfs_poisson {
     double *V = nullptr, *Z = nullptr, *w = nullptr, *dev_scalars = nullptr;
     std::vector<void *> allocs;
     SubGraph sub[2];  // [0] FP32, [1] FP64 hierarchy
+    TailPlan tail[2];  // the one-block part of a V-cycle, FP32 and FP64
+    vfs::TailLevel<float> *tl32 = nullptr;
+    vfs::TailLevel<double> *tl64 = nullptr;
 };
 
 namespace vfs {
@@ -1503,6 +2020,110 @@ static int level_dense_inverse(vfs_ctx *c, vfs_poisson *ps, PLevel &L)
     return VFS_OK;
 }
 
+// the FP32 or FP64 vectors and coefficients of a level
+template <typename T>
+struct LV;
+template <>
+struct LV<float> {
+    static float *x(PLevel &L) { return L.x32; }
+    static float *b(PLevel &L) { return L.b32; }
+    static float *r(PLevel &L) { return L.r32; }
+    static const float *coef(PLevel &L) { return L.c32; }
+    static const float *sf(PLevel &L) { return L.sc32; }
+    static float *rz(PLevel &L) { return L.rz32; }
+    static const float *inv(PLevel &L) { return L.inv32; }
+};
+template <>
+struct LV<double> {
+    static double *x(PLevel &L) { return L.x64; }
+    static double *b(PLevel &L) { return L.b64; }
+    static double *r(PLevel &L) { return L.r64; }
+    static const double *coef(PLevel &L) { return L.c64; }
+    static const double *sf(PLevel &L) { return L.sc64 + SM_LO * 2 * L.z.cplane; }
+    static double *rz(PLevel &L) { return L.rz64; }
+    static const double *inv(PLevel &L) { return L.inv64; }
+};
+
+template <typename T>
+static auto tail_kernel(const TailPlan &P)
+{
+    if constexpr (sizeof(T) == 4) return P.compact ? k_mg_tail<float, true> : k_mg_tail<float, false>;
+    else return k_mg_tail<double, false>;
+}
+
+// The first level from which the rest of the hierarchy runs in one block
+// (k_mg_tail; nl when none does): every level's lines must be solved by one
+// thread per segment of 8 points, x, b and one residual fit the LDS, and the
+// levels take one smoother form.
+template <typename T>
+static int tail_setup(vfs_ctx *c, vfs_poisson *ps, TailPlan *plan, TailLevel<T> **dev)
+{
+    const int nl = ps->nl;
+    plan->first = nl;
+    if (ps->L[nl - 1].nr > TAIL_DENSE) return VFS_OK;
+    long long sum = 0, most = 0;
+    for (int l = nl - 1; l >= 0; l--) {
+        const PLevel &L = ps->L[l];
+        const long long nseg = (L.z.njI + 7) / 8;
+        sum += L.g.n;
+        most = L.g.n > most ? L.g.n : most;
+        if (sizeof(T) == 4 && L.compact != ps->L[nl - 1].compact) break;
+        if ((long long)L.z.nkI * L.z.nh * nseg > TAIL_T || (2 * sum + most) * (long long)sizeof(T) + sum > TAIL_LDS) break;
+        plan->first = l;
+    }
+    if (plan->first == nl) return VFS_OK;
+    std::vector<TailLevel<T>> h;
+    int at = 0, res = 0, rows = 0;
+    for (int l = plan->first; l < nl; l++) {
+        PLevel &L = ps->L[l];
+        TailLevel<T> t;
+        t.g = L.g;
+        t.z = L.z;
+        t.coef = LV<T>::coef(L);
+        t.row = L.row;
+        t.sh = L.sh16;
+        t.sd = L.sd32;
+        t.sc = sizeof(T) == 8 ? reinterpret_cast<const T *>(L.sc64) : nullptr;
+        t.sf = LV<T>::sf(L);
+        t.compact = L.compact;
+        t.nseg = (L.z.njI + 7) / 8;
+        t.sl = (L.z.njI + t.nseg - 1) / t.nseg;
+        t.xo = at;
+        t.bo = at + (int)L.g.n;
+        t.wo = rows;
+        at += 2 * (int)L.g.n;
+        rows += (int)L.g.n;
+        res = res > (int)L.g.n ? res : (int)L.g.n;
+        t.nr = L.nr;
+        t.ridx = L.ridx;
+        t.inv = LV<T>::inv(L);
+        h.push_back(t);
+    }
+    plan->ro = at;
+    plan->wo = (at + res) * (int)sizeof(T);
+    plan->lds = plan->wo + rows;
+    int rc = palloc(ps, (void **)dev, h.size() * sizeof(TailLevel<T>));
+    if (rc) return rc;
+    VFS_HIP(hipMemcpyAsync(*dev, h.data(), h.size() * sizeof(TailLevel<T>), hipMemcpyHostToDevice, c->stream));
+    VFS_HIP(hipStreamSynchronize(c->stream));
+    plan->compact = sizeof(T) == 4 && ps->L[nl - 1].compact;
+    VFS_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(tail_kernel<T>(*plan)), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                TAIL_LDS));
+    return VFS_OK;
+}
+
+// The first level of the one-block part of a V-cycle now (VFS_MG_TAIL=0, or
+// any switch that asks for one form of the separate kernels, turns it off)
+template <typename T>
+static int tail_first(const vfs_poisson *ps)
+{
+    const char *e = std::getenv("VFS_MG_TAIL");
+    if (e && e[0] == '0') return ps->nl;
+    for (const char *v : {"VFS_LINE_PATH", "VFS_ZEBRA_FUSED", "VFS_MG_FUSED_RESTRICT", "VFS_MG_SPLIT", "VFS_MG_GRAPH"})
+        if (std::getenv(v)) return ps->nl;
+    return ps->tail[sizeof(T) == 4 ? 0 : 1].first;
+}
+
 static int poisson_setup(vfs_ctx *c, int levels)
 {
     // the hierarchy is kept while the requested level count is the same (the
@@ -1585,6 +2206,8 @@ static int poisson_setup(vfs_ctx *c, int levels)
         if (rc) return rc;
     }
     if (nl > 1) rc = level_dense_inverse(c, ps, ps->L[nl - 1]);
+    if (!rc) rc = tail_setup<float>(c, ps, &ps->tail[0], &ps->tl32);
+    if (!rc) rc = tail_setup<double>(c, ps, &ps->tail[1], &ps->tl64);
     if (!rc) ps->req_levels = levels;
     return rc;
 }
@@ -1603,29 +2226,6 @@ static int ensure_krylov(vfs_ctx *c, int restart)
 }
 
 // ---- V-cycle ---------------------------------------------------------------
-template <typename T>
-struct LV;
-template <>
-struct LV<float> {
-    static float *x(PLevel &L) { return L.x32; }
-    static float *b(PLevel &L) { return L.b32; }
-    static float *r(PLevel &L) { return L.r32; }
-    static const float *coef(PLevel &L) { return L.c32; }
-    static const float *sf(PLevel &L) { return L.sc32; }
-    static float *rz(PLevel &L) { return L.rz32; }
-    static const float *inv(PLevel &L) { return L.inv32; }
-};
-template <>
-struct LV<double> {
-    static double *x(PLevel &L) { return L.x64; }
-    static double *b(PLevel &L) { return L.b64; }
-    static double *r(PLevel &L) { return L.r64; }
-    static const double *coef(PLevel &L) { return L.c64; }
-    static const double *sf(PLevel &L) { return L.sc64 + SM_LO * 2 * L.z.cplane; }
-    static double *rz(PLevel &L) { return L.rz64; }
-    static const double *inv(PLevel &L) { return L.inv64; }
-};
-
 constexpr int LINE_PREFETCH = 16;
 
 // Which line-relaxation form a level takes.
@@ -1751,6 +2351,7 @@ template <typename T>
 static bool coarse_zero_free(const vfs_poisson *ps, int l, const Sweeps &S)
 {
     if (l < 1) return false;
+    if (l == tail_first<T>(ps)) return true;  // (writes every point)
     const PLevel &L = ps->L[l];
     const bool last = l == ps->nl - 1;
     if (last && L.nr > 0) return true;  // dense coarsest level
@@ -1773,9 +2374,10 @@ static void coarse_subcycle(vfs_ctx *c, vfs_poisson *ps, const Sweeps &S)
         vcycle<T>(c, ps, 1, S);
     };
     const char *env = std::getenv("VFS_MG_GRAPH");
-    if (env && env[0] == '0') { direct(); return; }
+    const int tail = tail_first<T>(ps);
+    if ((env && env[0] == '0') || tail == 1) { direct(); return; }  // (tail 1: one kernel)
     SubGraph &sg = ps->sub[sizeof(T) == 4 ? 0 : 1];
-    if (!sg.exec || !(sg.key == S)) {
+    if (!sg.exec || !(sg.key == S) || sg.tail != tail) {
         if (sg.exec) { hipGraphExecDestroy(sg.exec); sg.exec = nullptr; }
         hipGraph_t graph = nullptr;
         if (hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal) != hipSuccess) { direct(); return; }
@@ -1785,6 +2387,7 @@ static void coarse_subcycle(vfs_ctx *c, vfs_poisson *ps, const Sweeps &S)
         hipGraphDestroy(graph);
         if (e != hipSuccess) { sg.exec = nullptr; direct(); return; }
         sg.key = S;
+        sg.tail = tail;
     }
     // a replay that cannot be enqueued runs the same kernels directly
     if (hipGraphLaunch(sg.exec, st) != hipSuccess) {
@@ -1798,6 +2401,16 @@ static void vcycle(vfs_ctx *c, vfs_poisson *ps, int l, const Sweeps &S)
 {
     hipStream_t st = c->stream;
     PLevel &L = ps->L[l];
+    const int tail = tail_first<T>(ps);
+    if (l == tail) {
+        const TailPlan &P = ps->tail[sizeof(T) == 4 ? 0 : 1];
+        const TailLevel<T> *lev;
+        if constexpr (sizeof(T) == 4) lev = ps->tl32;
+        else lev = ps->tl64;
+        hipLaunchKernelGGL(tail_kernel<T>(P), dim3(1), dim3(TAIL_T), P.lds, st, lev, ps->nl - l, l, S, P.ro, P.wo,
+                           (const T *)LV<T>::b(L), LV<T>::x(L));
+        return;
+    }
     const int pre = S.pre_at(l), post = S.post_at(l);
     const unsigned nb = blocks_for(L.g.n, PTPB);
     // the finest level in the S layout (FP32 one-pass path): its iterate starts
@@ -1912,6 +2525,10 @@ static int amg_ensure(vfs_ctx *c, const vfs_solve_opts *o)
     return amg_build(c64.data(), row.data(), n, amg_nbr, &L.g, theta, &ps->amg);
 }
 
+// whether the FP32 V-cycle's finest vectors are in the S layout (a V-cycle
+// that is one block from the finest level on takes the natural one)
+static bool finest_split(const vfs_poisson *ps) { return tail_first<float>(ps) != 0 && line_plan<float>(ps->L[0]).split; }
+
 static Sweeps sweeps_of(const vfs_solve_opts *o)
 {
     return Sweeps{o->pre, o->post, o->coarse_sweeps, o->deep_level, o->deep_pre, o->deep_post};
@@ -1930,25 +2547,27 @@ static int precondition(vfs_ctx *c, const vfs_solve_opts *o, const double *v, do
         // on the one-pass path the V-cycle's finest vectors are in the S
         // layout: b converted into it, the iterate converted back into the
         // natural x (zero at the ghosts) at the end
-        const bool spl = line_plan<float>(L).split;
+        const bool spl = finest_split(ps), whole = tail_first<float>(ps) == 0;
         if (!b32_ready) {
             if (spl) hipLaunchKernelGGL(k_convert_split, dim3(nb), dim3(PTPB), 0, st, L.g, L.z, v, L.bs32);
             else hipLaunchKernelGGL((k_convert<double, float>), dim3(nb), dim3(PTPB), 0, st, n, v, L.b32);
         }
         float *x0 = L.x32;
         if (z32) L.x32 = z32;
-        if (!spl) hipLaunchKernelGGL(k_zero<float>, dim3(nb), dim3(PTPB), 0, st, n, L.x32);
+        if (!spl && !whole) hipLaunchKernelGGL(k_zero<float>, dim3(nb), dim3(PTPB), 0, st, n, L.x32);
         vcycle<float>(c, ps, 0, sweeps_of(o));
         if (spl) hipLaunchKernelGGL(k_split_to_natural, dim3(nb), dim3(PTPB), 0, st, L.g, L.z, (const float *)L.xs32, L.x32);
         if (!z32) hipLaunchKernelGGL((k_convert<float, double>), dim3(nb), dim3(PTPB), 0, st, n, L.x32, z);
         L.x32 = x0;
     } else {
-        hipMemcpyAsync(L.b64, v, n * 8, hipMemcpyDeviceToDevice, st);
-        double *x0 = L.x64;
+        // (the V-cycle does not write its right-hand side: v itself serves)
+        double *x0 = L.x64, *b0 = L.b64;
         L.x64 = z;
-        hipLaunchKernelGGL(k_zero<double>, dim3(nb), dim3(PTPB), 0, st, n, L.x64);
+        L.b64 = const_cast<double *>(v);
+        if (tail_first<double>(ps) != 0) hipLaunchKernelGGL(k_zero<double>, dim3(nb), dim3(PTPB), 0, st, n, L.x64);
         vcycle<double>(c, ps, 0, sweeps_of(o));
         L.x64 = x0;
+        L.b64 = b0;
     }
     VFS_LAUNCH_CHECK("v-cycle");
     return VFS_OK;
@@ -2145,7 +2764,7 @@ static int fgmres(vfs_ctx *c, const vfs_solve_opts *o, vfs_unet *net, vfs_solve_
             // with FP32 V-cycles the new basis vector is also written as the
             // next V-cycle's FP32 right-hand side
             // (in the S layout when the V-cycle's finest level takes it)
-            const bool spl = z32 && line_plan<float>(L).split;
+            const bool spl = z32 && finest_split(ps);
             rc = gs_step(c, jj + 1, V, w, V + (size_t)(jj + 1) * n, gs, z32 ? (spl ? L.bs32 : L.b32) : nullptr,
                          spl ? L.z : ZGrid{});
             if (rc) return rc;
