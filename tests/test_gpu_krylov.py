@@ -1,0 +1,29 @@
+"""The Gram-Schmidt sweeps with their sums finished by the last block: every
+basis-size instance (4, 8, 16, 32 vectors) on grids from a handful of blocks to
+more than the partials hold, checked with the oracle's operator."""
+import numpy as np
+import pytest
+
+from helpers import channel_pair, vfs
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("restart", [3, 7, 15, 31])
+@pytest.mark.parametrize("cells", [(4, 4, 6), (17, 11, 13), (96, 64, 80)], ids=str)
+def test_restart_lengths(cells, restart):
+    """A weak preconditioner (one level, one sweep) fills the basis; the
+    residual the solver reports is the one of its solution (the recurrences'
+    rounding is far below the tolerance)."""
+    c, o, ctx = channel_pair(*cells, les=0)
+    with ctx:
+        o.poisson_rhs()
+        ctx.poisson_rhs()
+        ctx.upload("PHI", np.zeros(o.shape))
+        opts = vfs.default_solve_opts(tol=1e-6, use_guess=0, levels=1, coarse_sweeps=1, restart=restart, maxit=40)
+        st = ctx.poisson_solve(opts, check=False)
+        r = np.linalg.norm(o["b"] - o.poisson_apply(ctx.download("PHI"))) / np.linalg.norm(o["b"])
+        assert abs(r - st.relres) <= 1e-9
+        assert r < 0.9 and (st.relres <= 1e-6 or st.iterations == 40)
+        st2 = ctx.poisson_solve(opts, check=False)  # the counters are back at zero: the same bits again
+        assert (st2.iterations, st2.relres) == (st.iterations, st.relres)

@@ -27,7 +27,7 @@
 namespace vfs {
 
 constexpr int IM_TPB = 256;
-constexpr int IM_MAXV = 33;  // GMRES basis vectors held by the dot kernel
+constexpr int IM_MAXV = KRYLOV_MAXV;  // GMRES basis vectors held by the dot kernel
 
 // wall-flux zeroing of FormFunction_SNES (momentum.c:2258-2282)
 __global__ void k_snes_bc(Grid g, double *__restrict__ ucont)
@@ -134,6 +134,13 @@ __global__ void k_im_axpby(long long n, double a, const double *__restrict__ x, 
     y[t] = a * x[t] + b * y[t];
 }
 
+// y = a x
+__global__ void k_im_scale(long long n, double a, const double *__restrict__ x, double *__restrict__ y)
+{
+    const long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x;
+    if (t < n) y[t] = a * x[t];
+}
+
 // z = x + a y
 __global__ void k_im_waxpy(long long n, const double *__restrict__ x, double a, const double *__restrict__ y,
                            double *__restrict__ z)
@@ -145,13 +152,16 @@ __global__ void k_im_waxpy(long long n, const double *__restrict__ x, double a, 
 
 // x = sum_v y[v] V_v (first) or x + sum_v y[v] V_v, the terms added in v
 // order with the fused multiply-add of a chain of k_im_axpby updates
-__global__ void k_im_update(long long n, int nv, const double *__restrict__ y, const double *__restrict__ V, long long ld,
+struct ImpY {
+    double v[IM_MAXV];
+};
+__global__ void k_im_update(long long n, int nv, ImpY y, const double *__restrict__ V, long long ld,
                             double *__restrict__ x, int first)
 {
     long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x;
     if (t >= n) return;
     double s = first ? 0.0 : x[t];
-    for (int v = 0; v < nv; v++) s = y[v] * V[v * ld + t] + s;
+    for (int v = 0; v < nv; v++) s = y.v[v] * V[v * ld + t] + s;
     x[t] = s;
 }
 
@@ -168,8 +178,9 @@ __global__ void k_im_waxpy2(long long n, const double *__restrict__ x, double a,
 
 // sum of |x| (for the differencing parameter)
 __global__ void __launch_bounds__(RED_THREADS) k_im_asum_dot(long long n, const double *__restrict__ u,
-                                                             const double *__restrict__ v, double *__restrict__ part)
+                                                             const double *__restrict__ v, double *part, double *out, RedSync rs)
 {
+    __shared__ double res[3];
     double a = 0, d = 0, vv = 0;
     for (long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x; t < n; t += (long long)gridDim.x * blockDim.x) {
         const double x = v[t];
@@ -180,7 +191,12 @@ __global__ void __launch_bounds__(RED_THREADS) k_im_asum_dot(long long n, const 
     a = block_reduce<OpSum>(a);
     d = block_reduce<OpSum>(d);
     vv = block_reduce<OpSum>(vv);
-    if (threadIdx.x == 0) { part[blockIdx.x] = a; part[RED_BLOCKS + blockIdx.x] = d; part[2 * RED_BLOCKS + blockIdx.x] = vv; }
+    if (threadIdx.x == 0) {
+        red_put(part + blockIdx.x, a);
+        red_put(part + RED_BLOCKS + blockIdx.x, d);
+        red_put(part + 2 * RED_BLOCKS + blockIdx.x, vv);
+    }
+    if (red_last(rs, gridDim.x)) red_finish_rows<OpSum>(rs, 3, gridDim.x, part, out, res);
 }
 
 }  // namespace vfs
@@ -193,16 +209,16 @@ namespace vfs {
 struct ImpState {
     long long n3 = 0;
     int m = 0;
-    double *U = nullptr, *R = nullptr, *W = nullptr, *FW = nullptr, *dx = nullptr, *V = nullptr, *h = nullptr;
+    double *U = nullptr, *R = nullptr, *W = nullptr, *FW = nullptr, *dx = nullptr, *V = nullptr;
 };
 
 // Carve the solver's vectors out of the context's persistent workspace
-// (5 + m + 1 vectors of n3 doubles and IM_MAXV scalars), allocating or
+// (5 + m + 1 vectors of n3 doubles), allocating or
 // growing it first when needed.  Every vector is written before it is read.
 static int im_workspace(vfs_ctx *c, ImpState &s)
 {
     const size_t vb = (size_t)s.n3 * sizeof(double);
-    const size_t need = (size_t)(6 + s.m) * vb + IM_MAXV * sizeof(double);
+    const size_t need = (size_t)(6 + s.m) * vb;
     if (c->imp_ws_bytes < need) {
         VFS_HIP(hipStreamSynchronize(c->stream));
         if (c->imp_ws) hipFree(c->imp_ws);
@@ -220,8 +236,7 @@ static int im_workspace(vfs_ctx *c, ImpState &s)
     s.W = p; p += s.n3;
     s.FW = p; p += s.n3;
     s.dx = p; p += s.n3;
-    s.V = p; p += (size_t)(s.m + 1) * s.n3;
-    s.h = p;
+    s.V = p;
     return VFS_OK;
 }
 
@@ -260,51 +275,12 @@ int snes_function(vfs_ctx *c, const double *u, double *r, int use_feul, const do
     return VFS_OK;
 }
 
-// the nv + 1 sums of the partials in c->red, on the host in out
-static int im_finish(vfs_ctx *c, int nv, double *out)
-{
-    hipStream_t st = c->stream;
-    hipLaunchKernelGGL(k_finish_many, dim3(nv + 1), dim3(RED_THREADS), 0, st, nv, c->red, c->red + IM_MAXV * RED_BLOCKS);
-    VFS_LAUNCH_CHECK("implicit dots");
-    VFS_HIP(hipMemcpyAsync(c->red_host, c->red + IM_MAXV * RED_BLOCKS, (nv + 1) * sizeof(double), hipMemcpyDeviceToHost, st));
-    VFS_HIP(hipStreamSynchronize(st));
-    std::memcpy(out, c->red_host, (nv + 1) * sizeof(double));
-    return VFS_OK;
-}
-
-// <w, V_v> for v < nv and <w, w> on the host
-static int im_dots(vfs_ctx *c, long long n, int nv, const double *V, const double *w, double *out)
-{
-    hipStream_t st = c->stream;
-    const dim3 gb(RED_BLOCKS), tb(RED_THREADS);
-    if (nv <= 4) hipLaunchKernelGGL((k_multidot<4, 4>), gb, tb, 0, st, n, nv, V, n, w, c->red);
-    else if (nv <= 8) hipLaunchKernelGGL((k_multidot<8, 4>), gb, tb, 0, st, n, nv, V, n, w, c->red);
-    else if (nv <= 16) hipLaunchKernelGGL((k_multidot<16, 2>), gb, tb, 0, st, n, nv, V, n, w, c->red);
-    else hipLaunchKernelGGL((k_multidot<IM_MAXV - 1, 1>), gb, tb, 0, st, n, nv, V, n, w, c->red);
-    return im_finish(c, nv, out);
-}
-
-// w -= sum_v h_v V_v (h on the device in s.h); with DOTS the partials of
-// <V_v, w_new> (v < nv) and <w_new, w_new>, else of <w_new, w_new> alone;
-// the finished sums on the host in out
-template <bool DOTS>
-static int im_multiaxpy(vfs_ctx *c, long long n, int nv, const double *h, const double *V, double *w, double *out)
-{
-    hipStream_t st = c->stream;
-    const dim3 gb(RED_BLOCKS), tb(RED_THREADS);
-    const double *g0 = nullptr;
-    if (nv <= 4) hipLaunchKernelGGL((k_multiaxpy<4, 4, DOTS>), gb, tb, 0, st, n, nv, h, V, n, w, c->red, g0, g0);
-    else if (nv <= 8) hipLaunchKernelGGL((k_multiaxpy<8, 4, DOTS>), gb, tb, 0, st, n, nv, h, V, n, w, c->red, g0, g0);
-    else if (nv <= 16) hipLaunchKernelGGL((k_multiaxpy<16, 2, DOTS>), gb, tb, 0, st, n, nv, h, V, n, w, c->red, g0, g0);
-    else hipLaunchKernelGGL((k_multiaxpy<IM_MAXV - 1, 1, DOTS>), gb, tb, 0, st, n, nv, h, V, n, w, c->red, g0, g0);
-    return im_finish(c, DOTS ? nv : 0, out);
-}
-
 static int im_norm(vfs_ctx *c, long long n, const double *w, double *out)
 {
-    double d[1];
-    int rc = im_dots(c, n, 0, nullptr, w, d);
-    *out = std::sqrt(d[0]);
+    launch_multidot(c->stream, n, 0, nullptr, w, c->red, red_sync(c));
+    VFS_LAUNCH_CHECK("implicit norm");
+    const int rc = red_wait(c);
+    if (!rc) *out = std::sqrt(c->red_host[0]);
     return rc;
 }
 
@@ -314,13 +290,11 @@ static int mffd(vfs_ctx *c, ImpState &s, const double *v, double *jv, int use_fe
 {
     hipStream_t st = c->stream;
     const long long n = s.n3;
-    hipLaunchKernelGGL(k_im_asum_dot, dim3(RED_BLOCKS), dim3(RED_THREADS), 0, st, n, s.U, v, c->red);
-    for (int q = 0; q < 3; q++)
-        hipLaunchKernelGGL(finish_reduce<OpSum>, dim3(1), dim3(RED_THREADS), 0, st, c->red + q * RED_BLOCKS, RED_BLOCKS,
-                           c->red + 3 * RED_BLOCKS + q);
+    hipLaunchKernelGGL(k_im_asum_dot, dim3(krylov_blocks(n)), dim3(RED_THREADS), 0, st, n, s.U, v, c->red, c->red + 3 * RED_BLOCKS,
+                       red_sync(c));
     VFS_LAUNCH_CHECK("mffd norms");
-    VFS_HIP(hipMemcpyAsync(c->red_host, c->red + 3 * RED_BLOCKS, 3 * sizeof(double), hipMemcpyDeviceToHost, st));
-    VFS_HIP(hipStreamSynchronize(st));
+    int rc = red_wait(c);
+    if (rc) return rc;
     const double asum = c->red_host[0], dot = c->red_host[1], vv = c->red_host[2];
     if (vv == 0) {
         VFS_HIP(hipMemsetAsync(jv, 0, n * sizeof(double), st));
@@ -333,26 +307,23 @@ static int mffd(vfs_ctx *c, ImpState &s, const double *v, double *jv, int use_fe
     // U + h v goes straight into UCONT, where the residual evaluation reads it
     hipLaunchKernelGGL(k_im_waxpy, dim3(blocks_for(n, IM_TPB)), dim3(IM_TPB), 0, st, n, s.U, hh, v, c->f[VFS_UCONT]);
     // jv = (F(U + h v) - F(U)) / h, the quotient formed with the residual
-    int rc = snes_function(c, c->f[VFS_UCONT], jv, use_feul, s.R, -1.0 / hh, 1.0 / hh);
+    rc = snes_function(c, c->f[VFS_UCONT], jv, use_feul, s.R, -1.0 / hh, 1.0 / hh);
     if (rc) return rc;
     (*nfunc)++;
     VFS_LAUNCH_CHECK("mffd");
     return VFS_OK;
 }
 
-// GMRES(m) for J dx = -R, dx from zero; returns iterations, final estimate
-static int gmres(vfs_ctx *c, ImpState &s, double rtol, int maxit, int use_feul, int *its, int *nfunc)
+// GMRES(m) for J dx = -R, dx from zero; bnorm = ||R||; returns iterations
+static int gmres(vfs_ctx *c, ImpState &s, double bnorm, double rtol, int maxit, int use_feul, int *its, int *nfunc)
 {
     hipStream_t st = c->stream;
     const long long n = s.n3;
     const int m = s.m;
     const unsigned nb = blocks_for(n, IM_TPB);
-    double d[IM_MAXV + 1];
+    int rc = VFS_OK;
     std::vector<double> H((size_t)(m + 1) * m), cs(m), sn(m), gv(m + 1), y(m);
     // r0 = -R (dx = 0); dx is first written by the first restart's update
-    int rc = im_dots(c, n, 0, nullptr, s.R, d);
-    if (rc) return rc;
-    const double bnorm = std::sqrt(d[0]);
     *its = 0;
     if (bnorm == 0) {
         VFS_HIP(hipMemsetAsync(s.dx, 0, n * sizeof(double), st));
@@ -363,17 +334,16 @@ static int gmres(vfs_ctx *c, ImpState &s, double rtol, int maxit, int use_feul, 
     while (*its < maxit) {
         double *V0 = s.V;
         if (first) {
-            hipLaunchKernelGGL(k_im_axpby, dim3(nb), dim3(IM_TPB), 0, st, n, -1.0 / beta, s.R, 0.0, V0);
+            hipLaunchKernelGGL(k_im_scale, dim3(nb), dim3(IM_TPB), 0, st, n, -1.0 / beta, (const double *)s.R, V0);
         } else {
             // r = -R - J dx
             rc = mffd(c, s, s.dx, s.FW, use_feul, nfunc);
             if (rc) return rc;
             hipLaunchKernelGGL(k_im_axpby, dim3(nb), dim3(IM_TPB), 0, st, n, -1.0, s.R, -1.0, s.FW);
-            rc = im_dots(c, n, 0, nullptr, s.FW, d);
+            rc = im_norm(c, n, s.FW, &beta);
             if (rc) return rc;
-            beta = std::sqrt(d[0]);
             if (beta <= rtol * bnorm) break;
-            hipLaunchKernelGGL(k_im_axpby, dim3(nb), dim3(IM_TPB), 0, st, n, 1.0 / beta, s.FW, 0.0, V0);
+            hipLaunchKernelGGL(k_im_scale, dim3(nb), dim3(IM_TPB), 0, st, n, 1.0 / beta, (const double *)s.FW, V0);
         }
         first = false;
         std::fill(gv.begin(), gv.end(), 0.0);
@@ -383,32 +353,16 @@ static int gmres(vfs_ctx *c, ImpState &s, double rtol, int maxit, int use_feul, 
             double *vj = s.V + (size_t)jj * n, *w = s.V + (size_t)(jj + 1) * n;
             rc = mffd(c, s, vj, w, use_feul, nfunc);
             if (rc) return rc;
-            // classical Gram-Schmidt; the first sweep w -= V h also forms the
-            // dot products a second (re-orthogonalisation) pass needs
+            // classical Gram-Schmidt with a second pass where the norm drops; w is
+            // normalised in place
             double h[IM_MAXV];
-            rc = im_dots(c, n, jj + 1, s.V, w, d);
+            launch_gram_schmidt(st, n, jj + 1, s.V, w, w, c->red, red_sync(c), NoCopy{});
+            VFS_LAUNCH_CHECK("implicit gram-schmidt");
+            rc = red_wait(c);
             if (rc) return rc;
-            for (int v = 0; v <= jj; v++) h[v] = d[v];
-            const double ww0 = d[jj + 1];
-            std::memcpy(c->red_host, h, (jj + 1) * sizeof(double));
-            VFS_HIP(hipMemcpyAsync(s.h, c->red_host, (jj + 1) * sizeof(double), hipMemcpyHostToDevice, st));
-            rc = im_multiaxpy<true>(c, n, jj + 1, s.h, s.V, w, d);
-            if (rc) return rc;
-            double ww = d[jj + 1];
-            if (ww < 0.25 * ww0) {  // second classical Gram-Schmidt pass
-                for (int v = 0; v <= jj; v++) h[v] += d[v];
-                std::memcpy(c->red_host, d, (jj + 1) * sizeof(double));
-                VFS_HIP(hipMemcpyAsync(s.h, c->red_host, (jj + 1) * sizeof(double), hipMemcpyHostToDevice, st));
-                double d2[IM_MAXV + 1];
-                rc = im_multiaxpy<false>(c, n, jj + 1, s.h, s.V, w, d2);
-                if (rc) return rc;
-                ww = d2[0];
-            }
-            const double hn = std::sqrt(ww > 0 ? ww : 0);
+            const double hn = gram_schmidt_column(c->red_host, jj + 1, h);
             for (int v = 0; v <= jj; v++) H[(size_t)v * m + jj] = h[v];
             H[(size_t)(jj + 1) * m + jj] = hn;
-            if (hn > 0)
-                hipLaunchKernelGGL(k_im_axpby, dim3(nb), dim3(IM_TPB), 0, st, n, 1.0 / hn, w, 0.0, w);
             for (int i = 0; i < jj; i++) {
                 const double tmp = cs[i] * H[(size_t)i * m + jj] + sn[i] * H[(size_t)(i + 1) * m + jj];
                 H[(size_t)(i + 1) * m + jj] = -sn[i] * H[(size_t)i * m + jj] + cs[i] * H[(size_t)(i + 1) * m + jj];
@@ -430,9 +384,9 @@ static int gmres(vfs_ctx *c, ImpState &s, double rtol, int maxit, int use_feul, 
             y[i] = H[(size_t)i * m + i] != 0 ? sacc / H[(size_t)i * m + i] : 0.0;
         }
         // dx += sum_q y_q V_q in one sweep (dx = 0 before the first restart)
-        std::memcpy(c->red_host, y.data(), jj * sizeof(double));
-        VFS_HIP(hipMemcpyAsync(s.h, c->red_host, jj * sizeof(double), hipMemcpyHostToDevice, st));
-        hipLaunchKernelGGL(k_im_update, dim3(nb), dim3(IM_TPB), 0, st, n, jj, s.h, s.V, n, s.dx, restart0 ? 1 : 0);
+        ImpY yk;
+        for (int q = 0; q < jj; q++) yk.v[q] = y[q];
+        hipLaunchKernelGGL(k_im_update, dim3(nb), dim3(IM_TPB), 0, st, n, jj, yk, s.V, n, s.dx, restart0 ? 1 : 0);
         restart0 = false;
         VFS_LAUNCH_CHECK("gmres update");
         if (std::fabs(gv[jj]) <= rtol * bnorm) break;
@@ -510,7 +464,7 @@ int vfs_implicit_matrixfree(vfs_ctx *c, const vfs_newton_opts *o, vfs_newton_sta
             eta = std::fmin(e, ew_max);
         }
         int its = 0;
-        rc = gmres(c, s, eta, maxlin, o->use_feul, &its, &nfunc);
+        rc = gmres(c, s, fnorm, eta, maxlin, o->use_feul, &its, &nfunc);
         if (rc) return fail(rc);
         lin_total += its;
         // step with halving while the residual does not decrease

@@ -1664,80 +1664,56 @@ __global__ void k_zero(long long n, T *__restrict__ x)
     if (t < n) x[t] = 0;
 }
 
-// y = a * x   (a read from device memory so no host round trip is needed)
-__global__ void k_scale_dev(long long n, const double *__restrict__ a, int inv, const double *__restrict__ x,
-                            double *__restrict__ y)
-{
-    long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-    double s = inv ? 1.0 / sqrt(a[0]) : a[0];
-    if (t < n) y[t] = s * x[t];
-}
-
-// out = <w, w> of the second Gram-Schmidt pass when it ran (gate as in
-// k_multiaxpy), else the first pass's *gww
-__global__ void __launch_bounds__(RED_THREADS) k_finish_gated(const double *__restrict__ part, int n,
-                                                              const double *__restrict__ gww, const double *__restrict__ gww0,
-                                                              double *__restrict__ out)
-{
-    if (!(gww[0] < 0.25 * gww0[0])) {
-        if (threadIdx.x == 0) out[0] = gww[0];
-        return;
-    }
-    double v = OpSum::init();
-    for (int q = threadIdx.x; q < n; q += blockDim.x) v = OpSum::op(v, part[q]);
-    v = block_reduce<OpSum>(v);
-    if (threadIdx.x == 0) out[0] = v;
-}
-
-// y = x / sqrt(ww) (0 when ww <= 0), ww read from device memory
-// y = x / sqrt(ww[0]) (0 when ww[0] <= 0); y32, when given, receives y as
-// FP32 (the next FP32 V-cycle's right-hand side)
-// (natural layout, or the S layout of zs when zs.cplane > 0: interior points only)
-__global__ void k_scale_rnorm(long long n, const double *__restrict__ ww, const double *__restrict__ x,
-                              double *__restrict__ y, float *__restrict__ y32, Grid g, ZGrid zs)
-{
-    long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-    const double hn = sqrt(ww[0] > 0 ? ww[0] : 0);
-    const double s = hn > 0 ? 1.0 / hn : 0.0;
-    if (t < n) {
-        const double v = s * x[t];
-        y[t] = v;
-        if (y32) {
-            if (zs.cplane > 0) {
-                int k, j, i;
-                nat_decode(g, (unsigned)t, k, j, i);
-                if (zs_interior(g, k, j, i)) y32[zs_index32(zs, k, j, i)] = (float)v;
-            } else {
-                y32[t] = (float)v;
-            }
+// a new basis vector also as the next V-cycle's FP32 right-hand side: natural
+// layout, or the S layout of zs when zs.cplane > 0 (interior points only)
+struct CopyRhs32 {
+    float *y32;  // null: none
+    Grid g;
+    ZGrid zs;
+    __device__ void operator()(long long t, double v) const
+    {
+        if (!y32) return;
+        if (zs.cplane > 0) {
+            int k, j, i;
+            nat_decode(g, (unsigned)t, k, j, i);
+            if (zs_interior(g, k, j, i)) y32[zs_index32(zs, k, j, i)] = (float)v;
+        } else {
+            y32[t] = (float)v;
         }
     }
-}
+};
 
-constexpr int MAXV = 33;
+constexpr int MAXV = KRYLOV_MAXV;
 
 // x = x + sum_v y[v] Z_v (Z in FP64, or FP32 from the FP32 V-cycle)
+struct KrylovY {
+    double v[MAXV];
+};
 template <typename Z_T>
-__global__ void k_multiupdate(long long n, int nv, const double *__restrict__ y, const Z_T *__restrict__ Z, long long ld,
-                              double *__restrict__ x)
+__global__ void k_multiupdate(long long n, int nv, KrylovY y, const Z_T *__restrict__ Z, long long ld, double *__restrict__ x)
 {
     long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x;
     if (t >= n) return;
     double s = x[t];
-    for (int v = 0; v < nv; v++) s += y[v] * (double)Z[v * ld + t];
+    for (int v = 0; v < nv; v++) s += y.v[v] * (double)Z[v * ld + t];
     x[t] = s;
 }
 
-// sum and count of the rows of x (plain mean, poisson_hypre.c:202-263)
-__global__ void k_row_sum(long long n, const unsigned char *__restrict__ row, const double *__restrict__ x,
-                          double *__restrict__ part)
+// sum and count of the rows of x (plain mean, poisson_hypre.c:202-263) into out
+__global__ void __launch_bounds__(RED_THREADS) k_row_sum(long long n, const unsigned char *__restrict__ row,
+                                                         const double *__restrict__ x, double *part, double *out, RedSync rs)
 {
+    __shared__ double res[2];
     double s = 0, c = 0;
     for (long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x; t < n; t += (long long)gridDim.x * blockDim.x)
         if (row[t]) { s += x[t]; c += 1; }
     s = block_reduce<OpSum>(s);
     c = block_reduce<OpSum>(c);
-    if (threadIdx.x == 0) { part[blockIdx.x] = s; part[RED_BLOCKS + blockIdx.x] = c; }
+    if (threadIdx.x == 0) {
+        red_put(part + blockIdx.x, s);
+        red_put(part + RED_BLOCKS + blockIdx.x, c);
+    }
+    if (red_last(rs, gridDim.x)) red_finish_rows<OpSum>(rs, 2, gridDim.x, part, out, res);
 }
 
 __global__ void k_sub_mean(long long n, const unsigned char *__restrict__ row, const double *__restrict__ sc,
@@ -1819,7 +1795,7 @@ struct vfs_poisson {
     int req_levels = 0;  // levels requested when it was built
     int restart = 0;
     PLevel L[8];
-    double *V = nullptr, *Z = nullptr, *w = nullptr, *dev_scalars = nullptr;
+    double *V = nullptr, *Z = nullptr, *w = nullptr;
     std::vector<void *> allocs;
     SubGraph sub[2];  // [0] FP32, [1] FP64 hierarchy
     TailPlan tail[2];  // the one-block part of a V-cycle, FP32 and FP64
@@ -2220,7 +2196,6 @@ static int ensure_krylov(vfs_ctx *c, int restart)
     int rc = palloc(ps, (void **)&ps->V, (size_t)(restart + 1) * n * 8);
     if (!rc) rc = palloc(ps, (void **)&ps->Z, (size_t)restart * n * 8);
     if (!rc) rc = palloc(ps, (void **)&ps->w, n * 8);
-    if (!rc) rc = palloc(ps, (void **)&ps->dev_scalars, 4 * MAXV * 8);
     if (!rc) ps->restart = restart;
     return rc;
 }
@@ -2576,66 +2551,11 @@ static int precondition(vfs_ctx *c, const vfs_solve_opts *o, const double *v, do
 // dots of w with V_0..V_{nv-1} plus <w,w>, returned on the host
 static int multidot(vfs_ctx *c, int nv, const double *V, const double *w, double *out)
 {
-    hipStream_t st = c->stream;
-    const long long n = c->g.n;
-    const dim3 gb(RED_BLOCKS), tb(RED_THREADS);
-    if (nv <= 4) hipLaunchKernelGGL((k_multidot<4, 4>), gb, tb, 0, st, n, nv, V, n, w, c->red);
-    else if (nv <= 8) hipLaunchKernelGGL((k_multidot<8, 4>), gb, tb, 0, st, n, nv, V, n, w, c->red);
-    else if (nv <= 16) hipLaunchKernelGGL((k_multidot<16, 2>), gb, tb, 0, st, n, nv, V, n, w, c->red);
-    else hipLaunchKernelGGL((k_multidot<MAXV - 1, 1>), gb, tb, 0, st, n, nv, V, n, w, c->red);
-    hipLaunchKernelGGL(k_finish_many, dim3(nv + 1), dim3(RED_THREADS), 0, st, nv, c->red, c->red + MAXV * RED_BLOCKS);
+    launch_multidot(c->stream, c->g.n, nv, V, w, c->red, red_sync(c));
     VFS_LAUNCH_CHECK("multidot");
-    VFS_HIP(hipMemcpyAsync(c->red_host, c->red + MAXV * RED_BLOCKS, (nv + 1) * sizeof(double), hipMemcpyDeviceToHost, st));
-    VFS_HIP(hipStreamSynchronize(st));
+    const int rc = red_wait(c);
+    if (rc) return rc;
     std::memcpy(out, c->red_host, (nv + 1) * sizeof(double));
-    return VFS_OK;
-}
-
-// w -= sum_v h_v V_v (h in dev_scalars) with the partials of k_multiaxpy
-template <bool DOTS>
-static void launch_multiaxpy(vfs_ctx *c, int nv, const double *V, double *w, const double *h = nullptr,
-                             const double *gww = nullptr, const double *gww0 = nullptr)
-{
-    hipStream_t st = c->stream;
-    const long long n = c->g.n;
-    if (!h) h = c->ps->dev_scalars;
-    const dim3 gb(RED_BLOCKS), tb(RED_THREADS);
-    if (nv <= 4) hipLaunchKernelGGL((k_multiaxpy<4, 4, DOTS>), gb, tb, 0, st, n, nv, h, V, n, w, c->red, gww, gww0);
-    else if (nv <= 8) hipLaunchKernelGGL((k_multiaxpy<8, 4, DOTS>), gb, tb, 0, st, n, nv, h, V, n, w, c->red, gww, gww0);
-    else if (nv <= 16) hipLaunchKernelGGL((k_multiaxpy<16, 2, DOTS>), gb, tb, 0, st, n, nv, h, V, n, w, c->red, gww, gww0);
-    else hipLaunchKernelGGL((k_multiaxpy<MAXV - 1, 1, DOTS>), gb, tb, 0, st, n, nv, h, V, n, w, c->red, gww, gww0);
-}
-
-// One classical Gram-Schmidt step of w against V_0..V_{nv-1} with the
-// re-orthogonalisation pass when <w, w> drops below a quarter, and
-// V_nv = w / ||w||, all on the device: the coefficients of each pass are the
-// previous pass's device results, so the host synchronises once.  out (host)
-// receives h (nv), ww0, the second-pass dots (nv), ww1 and the final <w, w>
-// at [0..nv], [40..40+nv], [80].
-constexpr int GS_D2 = 40, GS_D3 = 80;
-static_assert(GS_D2 >= MAXV && GS_D3 >= GS_D2 + MAXV, "Gram-Schmidt result slots");
-static int gs_step(vfs_ctx *c, int nv, const double *V, double *w, double *vnext, double *out, float *vnext32,
-                   ZGrid zs = {})
-{
-    hipStream_t st = c->stream;
-    const long long n = c->g.n;
-    double *R = c->red + MAXV * RED_BLOCKS;
-    const dim3 gb(RED_BLOCKS), tb(RED_THREADS);
-    if (nv <= 4) hipLaunchKernelGGL((k_multidot<4, 4>), gb, tb, 0, st, n, nv, V, n, w, c->red);
-    else if (nv <= 8) hipLaunchKernelGGL((k_multidot<8, 4>), gb, tb, 0, st, n, nv, V, n, w, c->red);
-    else if (nv <= 16) hipLaunchKernelGGL((k_multidot<16, 2>), gb, tb, 0, st, n, nv, V, n, w, c->red);
-    else hipLaunchKernelGGL((k_multidot<MAXV - 1, 1>), gb, tb, 0, st, n, nv, V, n, w, c->red);
-    hipLaunchKernelGGL(k_finish_many, dim3(nv + 1), dim3(RED_THREADS), 0, st, nv, c->red, R);
-    launch_multiaxpy<true>(c, nv, V, w, R);
-    hipLaunchKernelGGL(k_finish_many, dim3(nv + 1), dim3(RED_THREADS), 0, st, nv, c->red, R + GS_D2);
-    launch_multiaxpy<false>(c, nv, V, w, R + GS_D2, R + GS_D2 + nv, R + nv);
-    hipLaunchKernelGGL(k_finish_gated, dim3(1), dim3(RED_THREADS), 0, st, c->red, RED_BLOCKS, R + GS_D2 + nv, R + nv,
-                       R + GS_D3);
-    hipLaunchKernelGGL(k_scale_rnorm, dim3(blocks_for(n, PTPB)), dim3(PTPB), 0, st, n, R + GS_D3, w, vnext, vnext32, c->g, zs);
-    VFS_LAUNCH_CHECK("gram-schmidt");
-    VFS_HIP(hipMemcpyAsync(c->red_host, R, (GS_D3 + 1) * sizeof(double), hipMemcpyDeviceToHost, st));
-    VFS_HIP(hipStreamSynchronize(st));
-    std::memcpy(out, c->red_host, (GS_D3 + 1) * sizeof(double));
     return VFS_OK;
 }
 
@@ -2643,11 +2563,9 @@ static int remove_mean(vfs_ctx *c, const unsigned char *row, double *x)
 {
     hipStream_t st = c->stream;
     const long long n = c->g.n;
-    hipLaunchKernelGGL(k_row_sum, dim3(RED_BLOCKS), dim3(RED_THREADS), 0, st, n, row, x, c->red);
-    hipLaunchKernelGGL(finish_reduce<OpSum>, dim3(1), dim3(RED_THREADS), 0, st, c->red, RED_BLOCKS, c->red + 2 * RED_BLOCKS);
-    hipLaunchKernelGGL(finish_reduce<OpSum>, dim3(1), dim3(RED_THREADS), 0, st, c->red + RED_BLOCKS, RED_BLOCKS,
-                       c->red + 2 * RED_BLOCKS + 1);
-    hipLaunchKernelGGL(k_sub_mean, dim3(blocks_for(n, PTPB)), dim3(PTPB), 0, st, n, row, c->red + 2 * RED_BLOCKS, x);
+    double *out = c->red + 2 * RED_BLOCKS;
+    hipLaunchKernelGGL(k_row_sum, dim3(krylov_blocks(n)), dim3(RED_THREADS), 0, st, n, row, x, c->red, out, red_quiet(c));
+    hipLaunchKernelGGL(k_sub_mean, dim3(blocks_for(n, PTPB)), dim3(PTPB), 0, st, n, row, out, x);
     VFS_LAUNCH_CHECK("remove mean");
     return VFS_OK;
 }
@@ -2702,17 +2620,22 @@ static int fgmres(vfs_ctx *c, const vfs_solve_opts *o, vfs_unet *net, vfs_solve_
         const double rAy = d[0];
         rc = multidot(c, 0, V, V + n, d);
         if (rc) return rc;
-        c->red_host[0] = d[0] > 0 ? rAy / d[0] : 0.0;
-        VFS_HIP(hipMemcpyAsync(ps->dev_scalars, c->red_host, sizeof(double), hipMemcpyHostToDevice, st));
-        hipLaunchKernelGGL(k_multiupdate<double>, dim3(nb), dim3(PTPB), 0, st, n, 1, ps->dev_scalars, (const double *)Z, n, x);
+        KrylovY alpha;
+        alpha.v[0] = d[0] > 0 ? rAy / d[0] : 0.0;
+        hipLaunchKernelGGL(k_multiupdate<double>, dim3(nb), dim3(PTPB), 0, st, n, 1, alpha, (const double *)Z, n, x);
         VFS_LAUNCH_CHECK("learned warm start");
     }
     double rel_start = -1;
-    // ||b||: multidot with no basis vectors returns <b,b>
-    rc = multidot(c, 0, V, b, d);
-    if (rc) return rc;
-    double bnorm = std::sqrt(d[0]);
-    if (bnorm == 0) bnorm = 1;
+    // ||b||: multidot with no basis vectors returns <b,b>; read with the first
+    // residual's norm
+    constexpr int BB_AT = 128;  // (past every other result's place in red_host)
+    launch_multidot(st, n, 0, V, b, c->red, red_sync(c, BB_AT));
+    VFS_LAUNCH_CHECK("norm of b");
+    double bnorm = -1;
+    // with FP32 V-cycles each new basis vector is also written as the next
+    // V-cycle's FP32 right-hand side
+    const bool spl = z32 && finest_split(ps);
+    const CopyRhs32 copy{z32 ? (spl ? L.bs32 : L.b32) : nullptr, c->g, spl ? L.z : ZGrid{}};
     std::vector<double> H((size_t)(m + 1) * m), cs(m), sn(m), gv(m + 1), y(m);
     int it = 0;
     double rel = 1;
@@ -2729,16 +2652,21 @@ static int fgmres(vfs_ctx *c, const vfs_solve_opts *o, vfs_unet *net, vfs_solve_
     while (it < maxit) {
         // r = b - A x into V_0
         apply0(c, (const double *)x, b, V);
-        rc = multidot(c, 0, V, V, d);
+        launch_multidot(st, n, 0, V, V, c->red, red_sync(c));
+        hipLaunchKernelGGL(k_normalise<CopyRhs32>, dim3(nb), dim3(PTPB), 0, st, n, 1.0, (const double *)(c->red + KRYLOV_R),
+                           (const double *)V, V, copy);
+        VFS_LAUNCH_CHECK("residual");
+        rc = red_wait(c);
         if (rc) return rc;
-        double beta = std::sqrt(d[0]);
+        const double beta = std::sqrt(c->red_host[0]);
+        if (bnorm < 0) {
+            bnorm = std::sqrt(c->red_host[BB_AT]);
+            if (bnorm == 0) bnorm = 1;
+        }
         rel = beta / bnorm;
         if (rel_start < 0) rel_start = rel;
         if (trace) std::fprintf(stderr, "fgmres restart at it %d: true relres %.3e (bnorm %.3e)\n", it, rel, bnorm);
         if (rel <= tol) { converged = true; break; }
-        c->red_host[0] = 1.0 / beta;
-        VFS_HIP(hipMemcpyAsync(ps->dev_scalars, c->red_host, sizeof(double), hipMemcpyHostToDevice, st));
-        hipLaunchKernelGGL(k_scale_dev, dim3(nb), dim3(PTPB), 0, st, n, ps->dev_scalars, 0, V, V);
         std::fill(gv.begin(), gv.end(), 0.0);
         gv[0] = beta;
         int jj;
@@ -2749,7 +2677,7 @@ static int fgmres(vfs_ctx *c, const vfs_solve_opts *o, vfs_unet *net, vfs_solve_
                 rc = vfs_unet_forward(net, vj, z32 ? w : zj);
                 if (!rc && z32) hipLaunchKernelGGL((k_convert<double, float>), dim3(nb), dim3(PTPB), 0, st, n, (const double *)w, zj32);
             } else {
-                rc = precondition(c, o, vj, zj, z32 ? zj32 : nullptr, z32 && jj > 0);
+                rc = precondition(c, o, vj, zj, z32 ? zj32 : nullptr, z32);
             }
             if (rc) return rc;
             prof_begin(c, K_APPLY64);
@@ -2758,25 +2686,13 @@ static int fgmres(vfs_ctx *c, const vfs_solve_opts *o, vfs_unet *net, vfs_solve_
             else
                 apply0(c, (const double *)zj, (const double *)nullptr, w);
             prof_end(c);
-            // classical Gram-Schmidt, re-orthogonalised when the norm drops;
-            // the first pass also forms the dot products of the second
-            double gs[GS_D3 + 1];
-            // with FP32 V-cycles the new basis vector is also written as the
-            // next V-cycle's FP32 right-hand side
-            // (in the S layout when the V-cycle's finest level takes it)
-            const bool spl = z32 && finest_split(ps);
-            rc = gs_step(c, jj + 1, V, w, V + (size_t)(jj + 1) * n, gs, z32 ? (spl ? L.bs32 : L.b32) : nullptr,
-                         spl ? L.z : ZGrid{});
+            // classical Gram-Schmidt, re-orthogonalised when the norm drops
+            launch_gram_schmidt(st, n, jj + 1, V, w, V + (size_t)(jj + 1) * n, c->red, red_sync(c), copy);
+            VFS_LAUNCH_CHECK("gram-schmidt");
+            rc = red_wait(c);
             if (rc) return rc;
             double h[MAXV];
-            for (int v = 0; v <= jj; v++) h[v] = gs[v];
-            const double ww0 = gs[jj + 1], ww1 = gs[GS_D2 + jj + 1];
-            double ww = ww1;
-            if (ww1 < 0.25 * ww0) {
-                for (int v = 0; v <= jj; v++) h[v] += gs[GS_D2 + v];
-                ww = gs[GS_D3];
-            }
-            double hn = std::sqrt(ww > 0 ? ww : 0);
+            const double hn = gram_schmidt_column(c->red_host, jj + 1, h);
             for (int v = 0; v <= jj; v++) H[(size_t)v * m + jj] = h[v];
             H[(size_t)(jj + 1) * m + jj] = hn;
             for (int i = 0; i < jj; i++) {
@@ -2791,8 +2707,7 @@ static int fgmres(vfs_ctx *c, const vfs_solve_opts *o, vfs_unet *net, vfs_solve_
             H[(size_t)(jj + 1) * m + jj] = 0;
             gv[jj + 1] = -sn[jj] * gv[jj];
             gv[jj] = cs[jj] * gv[jj];
-            if (trace) std::fprintf(stderr, "  it %d: est relres %.3e  h_{j+1,j} %.3e  ww0 %.3e ww %.3e\n", it,
-                                    std::fabs(gv[jj + 1]) / bnorm, hn, ww0, ww);
+            if (trace) std::fprintf(stderr, "  it %d: est relres %.3e  h_{j+1,j} %.3e\n", it, std::fabs(gv[jj + 1]) / bnorm, hn);
             if (std::fabs(gv[jj + 1]) / bnorm <= tol) { jj++; it++; break; }
             // (written so that a NaN residual, from a network that returns non-finite values, also falls back)
             if (net && it == 2 && !(std::fabs(gv[jj + 1]) / bnorm <= 0.5 * rel_start)) {
@@ -2805,12 +2720,12 @@ static int fgmres(vfs_ctx *c, const vfs_solve_opts *o, vfs_unet *net, vfs_solve_
             for (int q = i + 1; q < jj; q++) s -= H[(size_t)i * m + q] * y[q];
             y[i] = s / H[(size_t)i * m + i];
         }
-        std::memcpy(c->red_host, y.data(), jj * sizeof(double));
-        VFS_HIP(hipMemcpyAsync(ps->dev_scalars, c->red_host, jj * sizeof(double), hipMemcpyHostToDevice, st));
+        KrylovY yk;
+        for (int q = 0; q < jj; q++) yk.v[q] = y[q];
         if (z32)
-            hipLaunchKernelGGL(k_multiupdate<float>, dim3(nb), dim3(PTPB), 0, st, n, jj, ps->dev_scalars, (const float *)Z32, n, x);
+            hipLaunchKernelGGL(k_multiupdate<float>, dim3(nb), dim3(PTPB), 0, st, n, jj, yk, (const float *)Z32, n, x);
         else
-            hipLaunchKernelGGL(k_multiupdate<double>, dim3(nb), dim3(PTPB), 0, st, n, jj, ps->dev_scalars, (const double *)Z, n, x);
+            hipLaunchKernelGGL(k_multiupdate<double>, dim3(nb), dim3(PTPB), 0, st, n, jj, yk, (const double *)Z, n, x);
         VFS_LAUNCH_CHECK("fgmres update");
     }
     if (!converged) {

@@ -11,6 +11,7 @@
 #include <string>
 
 #include "vfs_internal.h"
+#include "vfs_reduce.h"
 
 namespace {
 thread_local std::string g_err;
@@ -125,6 +126,28 @@ void prof_end(vfs_ctx *c, int idx)
     hipEventRecord((*c->ev_pool)[(*c->ev_recs)[idx].second + 1], c->stream);
 }
 
+// the flag word of red_host, on a cache line of its own at its end
+static unsigned long long *red_flag(const vfs_ctx *c) { return reinterpret_cast<unsigned long long *>(c->red_host + 4096 - 16); }
+
+RedSync red_sync(vfs_ctx *c, int at) { return {c->red_ctr, c->red_host + at, red_flag(c), ++c->red_seq}; }
+RedSync red_quiet(vfs_ctx *c) { return {c->red_ctr, nullptr, nullptr, 0}; }
+
+// Waits on the flag in pinned memory; now and then the stream is asked too, so
+// that a kernel that failed ends the wait.
+int red_wait(vfs_ctx *c)
+{
+    volatile unsigned long long *flag = red_flag(c);
+    for (unsigned spin = 1; *flag != c->red_seq; spin++) {
+        if (spin % 4096) continue;
+        const hipError_t e = hipStreamQuery(c->stream);
+        if (e == hipErrorNotReady) continue;
+        if (e != hipSuccess) return check_hip(e, "reduction");
+        if (*flag != c->red_seq) return set_error(VFS_EHIP, "reduction: the stream is idle and the result is missing");
+    }
+    __sync_synchronize();
+    return VFS_OK;
+}
+
 Grid make_grid(const vfs_params &p)
 {
     Grid g;
@@ -153,6 +176,8 @@ int vfs_ctx_create(const vfs_params *params, vfs_ctx **out)
     c->p = *params;
     c->g = vfs::make_grid(*params);
     c->face = c->pucont = c->snap = c->fpc = c->red = c->red_host = c->inflow_plane = nullptr;
+    c->red_ctr = nullptr;
+    c->red_seq = 0;
     c->ps = nullptr;
     c->cs_mode = vfs::CS_PARAM;
     c->dyn = nullptr;
@@ -191,6 +216,13 @@ int vfs_ctx_create(const vfs_params *params, vfs_ctx **out)
     if (!rc) {
         hipError_t ee = hipHostMalloc((void **)&c->red_host, 4096 * sizeof(double), hipHostMallocDefault);
         if (ee != hipSuccess) rc = vfs::check_hip(ee, "hipHostMalloc");
+        else *vfs::red_flag(c) = 0;
+    }
+    if (!rc) {
+        const size_t bytes = vfs::RED_CTRS * vfs::RED_CTR_STRIDE * sizeof(unsigned);
+        hipError_t ee = hipMalloc((void **)&c->red_ctr, bytes);
+        if (ee == hipSuccess) ee = hipMemsetAsync(c->red_ctr, 0, bytes, c->stream);
+        if (ee != hipSuccess) rc = vfs::check_hip(ee, "reduction counters");
     }
     if (!rc) {
         hipError_t ee = hipStreamSynchronize(c->stream);
@@ -214,6 +246,7 @@ int vfs_ctx_destroy(vfs_ctx *c)
     if (c->red) hipFree(c->red);
     if (c->inflow_plane) hipFree(c->inflow_plane);
     if (c->red_host) hipHostFree(c->red_host);
+    if (c->red_ctr) hipFree(c->red_ctr);
     if (c->imp_ws) hipFree(c->imp_ws);
     if (c->dyn) hipFree(c->dyn);
     if (c->ev_pool) {

@@ -203,6 +203,8 @@ struct vfs_ctx {
     double *red;      // reduction scratch (device)
     double *inflow_plane;  // my x mx Cmpnts: the inlet plane of -inlet 100 / -pseudo (user->ucont_plane)
     double *red_host; // pinned host mirror of reduction results
+    unsigned *red_ctr;              // RedSync counters (zero between kernels)
+    unsigned long long red_seq;     // the last RedSync handed to a kernel
     double mean_k_area;
     double mean_k_flux;
     // true while the face metrics are the cell-metric means vfs_form_metrics
@@ -322,6 +324,13 @@ void poisson_free(vfs_ctx *c);
 int update_pressure(vfs_ctx *c);
 int projection(vfs_ctx *c);
 int divergence(vfs_ctx *c, double *out);
+// Reductions that hand their results to the host (RedSync): red_sync numbers
+// the next one (results at red_host + at), red_wait waits for it; the stream goes
+// on meanwhile.  Only the latest one numbered may be waited for.
+struct RedSync;
+RedSync red_sync(vfs_ctx *c, int at = 0);
+RedSync red_quiet(vfs_ctx *c);  // finished on the device only
+int red_wait(vfs_ctx *c);
 // timing of individual launches (no-ops unless vfs_profile enabled it)
 // prof_begin returns the record index (-1 when profiling is off); prof_end
 // closes that record, or the most recent one when idx < 0
