@@ -427,9 +427,7 @@ __global__ void __launch_bounds__(FT_I * FT_J) k_face_fluxes(FaceArgs a, int kc)
 // nu_t, nvert, ucont and the metrics holding their periodic copies (as
 // Contra2Cart, the eddy viscosity, Formfunction_2's own Ucont fix and
 // FormMetrics leave them) the faces at index 0 computed here are bitwise
-// those copies, so that fix is not applied.  The projections are written for
-// every point of the block (zero at ghosts); the periodic ghosts are filled
-// afterwards.
+// those copies, so that fix is not applied.
 constexpr int FX_J = FT_J + 1;
 static_assert(FT_I == 32, "a row of the tile is half a wavefront (the i-face exchange shuffles within it)");
 constexpr int HX_T0 = 64;  // first thread of the second wavefront
@@ -450,8 +448,7 @@ __global__ void __launch_bounds__(FT_I * FT_J) __attribute__((amdgpu_waves_per_e
     // The tiles cover the interior points (1 .. m-2 on each axis; kc planes a
     // block): the faces at index 0 are the halo faces of the first tiles, and
     // the ghost points' projections are not written (zero at the non-periodic
-    // ghosts since allocation, copies at the periodic ones by the periodic fix
-    // that follows).  Tiles are taken in XCD order, so the tiles that share a
+    // ghosts since allocation; the cell pass does not read the periodic ones).  Tiles are taken in XCD order, so the tiles that share a
     // halo run on one XCD's L2.
     const int nbi = (g.mx - 2 + FT_I - 1) / FT_I, nbj = (g.my - 2 + FT_J - 1) / FT_J;
     int b = (int)xcd_block1();
@@ -915,10 +912,13 @@ __global__ void __launch_bounds__(CR_T) k_cell_rhs_pr(CellArgs a, int kc, const 
         const bool interior = i >= 1 && i < mx - 1 && j >= 1 && j < my - 1 && k >= 1 && k < mz - 1;
         bool zero[3] = {true, true, true};
         if (interior) {
-            const long long qi = q + 1, qj = q + mx, qk = gidx(g, k + 1, j, i);
-            const double pi0 = pr[q], pi1 = pr[qi];
-            const double pj0 = pr[n + q], pj1 = pr[n + qj];
-            const double pk0 = have ? pk_next : pr[2 * n + q], pk1 = pr[2 * n + qk];
+            const long long qi = q + 1, qj = q + mx, qk = q + g.plane;
+            // (the projections of the periodic ghosts are those of the cells they
+            // copy: read there, they need not be filled)
+            const double pi0 = pr[q], pi1 = pr[g.pi && i == mx - 2 ? q - (mx - 3) : qi];
+            const double pj0 = pr[n + q], pj1 = pr[n + (g.pj && j == my - 2 ? q - (long long)(my - 3) * mx : qj)];
+            const double pk0 = have ? pk_next : pr[2 * n + q];
+            const double pk1 = pr[2 * n + (g.pk && k == mz - 2 ? q - (long long)(mz - 3) * g.plane : qk)];
             // a.nvert == nullptr: no point is blanked (every nvert 0)
             const double *nv = a.nvert;
             const double nv0 = have ? nvk : (nv ? nv[q] : 0.0);
@@ -931,7 +931,7 @@ __global__ void __launch_bounds__(CR_T) k_cell_rhs_pr(CellArgs a, int kc, const 
             zero[2] = nv0 + nvkn > 0.1 || (!g.pk && k == mz - 2);
             nvk = nvkn;
             pk_next = pk1;
-            have = qk == q + g.plane;  // the carried values belong to the next plane
+            have = true;  // (the values carried belong to the next plane, where that is an interior one)
         } else {
             have = false;
         }
@@ -1057,7 +1057,8 @@ int formfunction2(vfs_ctx *c, double scale, const double *pucont, double rk_alph
     const Grid &g = c->g;
     hipStream_t st = c->stream;
     const int whole = prof_begin(c, K_FF);
-    int rc = periodic_fix(c, c->f[VFS_UCONT], 3, 0);  // momentum.c:638-666
+    // momentum.c:638-666 (a fresh Ucat: Contra2Cart has filled these ghosts since Ucont was last written)
+    int rc = c->ucat_fresh ? VFS_OK : periodic_fix(c, c->f[VFS_UCONT], 3, 0);
     if (rc) return rc;
     FaceArgs fa;
     fa.g = g;
@@ -1100,11 +1101,7 @@ int formfunction2(vfs_ctx *c, double scale, const double *pucont, double rk_alph
     }
     prof_end(c);
     VFS_LAUNCH_CHECK("face fluxes");
-    if (fused) {
-        // projections of the periodic ghost cells: copies of the cells they stand for
-        for (int d = 0; d < 3; d++)
-            if (per[d]) hipLaunchKernelGGL(k_periodic_soa, dim3(blocks_for(np[d], FF_TPB)), dim3(FF_TPB), 0, st, g, c->fpc, 3, d);
-    } else {
+    if (!fused) {
         for (int d = 0; d < 3; d++)
             if (per[d]) hipLaunchKernelGGL(k_periodic_soa, dim3(blocks_for(np[d], FF_TPB)), dim3(FF_TPB), 0, st, g, c->face, 18, d);
     }

@@ -29,30 +29,40 @@ namespace vfs {
 constexpr int IM_TPB = 256;
 constexpr int IM_MAXV = KRYLOV_MAXV;  // GMRES basis vectors held by the dot kernel
 
-// wall-flux zeroing of FormFunction_SNES (momentum.c:2258-2282)
+// wall-flux zeroing of FormFunction_SNES (momentum.c:2258-2282), one thread
+// per point of the six boundary planes: every rule acts on its own plane only,
+// and no two write one component of a point (a thread per grid point took
+// 65 us at 384x192x256)
+__host__ __device__ inline long long boundary_points(const Grid &g)
+{
+    return 2 * ((long long)g.my * g.mz + (long long)g.mx * g.mz + (long long)g.mx * g.my);
+}
 __global__ void k_snes_bc(Grid g, double *__restrict__ ucont)
 {
     long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-    if (t >= g.n) return;
-    const int i = t % g.mx;
-    const long long r = t / g.mx;
-    const int j = r % g.my, k = r / g.my;
+    const long long ni = 2LL * g.my * g.mz, nj = 2LL * g.mx * g.mz, nk = 2LL * g.mx * g.my;
     const int mx = g.mx, my = g.my, mz = g.mz;
+    int face, i, j, k;
+    if (t < ni) {
+        face = (int)(t & 1); j = (int)((t >> 1) % my); k = (int)((t >> 1) / my); i = face ? mx - 1 : 0;
+    } else if ((t -= ni) < nj) {
+        face = 2 + (int)(t & 1); i = (int)((t >> 1) % mx); k = (int)((t >> 1) / mx); j = face & 1 ? my - 1 : 0;
+    } else if ((t -= nj) < nk) {
+        face = 4 + (int)(t & 1); i = (int)((t >> 1) % mx); j = (int)((t >> 1) / mx); k = face & 1 ? mz - 1 : 0;
+    } else {
+        return;
+    }
     const int *b = g.bc;
 #define UC(kk, jj, ii, c) ucont[3 * (((long long)(kk) * my + (jj)) * mx + (ii)) + (c)]
-    if (i == 0 && b[0] == 1) UC(k, j, i, 0) = 0;
-    if (i == mx - 1 && b[1] == 1) UC(k, j, i - 1, 0) = 0;
-    if (j == 0 && b[2] == 1) UC(k, j, i, 1) = 0;
-    if (j == my - 1 && b[3] == 1) UC(k, j - 1, i, 1) = 0;
-    if (k == 0 && b[4] == 1) UC(k, j, i, 2) = 0;
-    if (k == mz - 1 && b[5] == 1) UC(k - 1, j, i, 2) = 0;
-    if (j == my - 1 && b[3] == 2) UC(k, j - 1, i, 1) = 0;
-    if (j == 0 && b[2] == 12) UC(k, j, i, 1) = 0;
-    if (j == my - 1 && b[3] == 12) UC(k, j - 1, i, 1) = 0;
-    if (b[0] == 10 && i == 0 && (j != 0 && j != my - 1 && k != 0 && k != mz - 1)) UC(k, j, i, 0) = 0;
-    if (b[1] == 10 && i == mx - 1 && (j != 0 && j != my - 1 && k != 0 && k != mz - 1)) UC(k, j, i - 1, 0) = 0;
-    if (b[2] == 10 && j == 0 && (i != 0 && i != mx - 1 && k != 0 && k != mz - 1)) UC(k, j, i, 1) = 0;
-    if ((b[3] == 10 || b[3] == -10) && j == my - 1 && (i != 0 && i != mx - 1 && k != 0 && k != mz - 1)) UC(k, j - 1, i, 1) = 0;
+    const bool in_jk = j != 0 && j != my - 1 && k != 0 && k != mz - 1, in_ik = i != 0 && i != mx - 1 && k != 0 && k != mz - 1;
+    switch (face) {
+    case 0: if (b[0] == 1 || (b[0] == 10 && in_jk)) UC(k, j, i, 0) = 0; break;
+    case 1: if (b[1] == 1 || (b[1] == 10 && in_jk)) UC(k, j, i - 1, 0) = 0; break;
+    case 2: if (b[2] == 1 || b[2] == 12 || (b[2] == 10 && in_ik)) UC(k, j, i, 1) = 0; break;
+    case 3: if (b[3] == 1 || b[3] == 2 || b[3] == 12 || ((b[3] == 10 || b[3] == -10) && in_ik)) UC(k, j - 1, i, 1) = 0; break;
+    case 4: if (b[4] == 1) UC(k, j, i, 2) = 0; break;
+    default: if (b[5] == 1) UC(k - 1, j, i, 2) = 0; break;
+    }
 #undef UC
 }
 
@@ -251,7 +261,7 @@ int snes_function(vfs_ctx *c, const double *u, double *r, int use_feul, const do
     const long long n3 = 3 * g.n;
     if (u != c->f[VFS_UCONT])
         VFS_HIP(hipMemcpyAsync(c->f[VFS_UCONT], u, n3 * sizeof(double), hipMemcpyDeviceToDevice, st));
-    hipLaunchKernelGGL(k_snes_bc, dim3(blocks_for(g.n, IM_TPB)), dim3(IM_TPB), 0, st, g, c->f[VFS_UCONT]);
+    hipLaunchKernelGGL(k_snes_bc, dim3(blocks_for(boundary_points(g), IM_TPB)), dim3(IM_TPB), 0, st, g, c->f[VFS_UCONT]);
     ucat_stale(c);
     VFS_LAUNCH_CHECK("snes bc");
     int rc = c2c(c);
@@ -290,7 +300,7 @@ static int mffd(vfs_ctx *c, ImpState &s, const double *v, double *jv, int use_fe
 {
     hipStream_t st = c->stream;
     const long long n = s.n3;
-    hipLaunchKernelGGL(k_im_asum_dot, dim3(krylov_blocks(n)), dim3(RED_THREADS), 0, st, n, s.U, v, c->red, c->red + 3 * RED_BLOCKS,
+    hipLaunchKernelGGL(k_im_asum_dot, dim3(reduce_blocks(n)), dim3(RED_THREADS), 0, st, n, s.U, v, c->red, c->red + 3 * RED_BLOCKS,
                        red_sync(c));
     VFS_LAUNCH_CHECK("mffd norms");
     int rc = red_wait(c);
@@ -491,7 +501,7 @@ int vfs_implicit_matrixfree(vfs_ctx *c, const vfs_newton_opts *o, vfs_newton_sta
     // U -> Ucont with Ucat as the last residual evaluation at U left it, the
     // post-solve boundary fix and FormBCS(outflow_scale = 1)
     VFS_HIP(hipMemcpyAsync(c->f[VFS_UCONT], s.U, vb, hipMemcpyDeviceToDevice, st));
-    hipLaunchKernelGGL(k_snes_bc, dim3(blocks_for(c->g.n, IM_TPB)), dim3(IM_TPB), 0, st, c->g, c->f[VFS_UCONT]);
+    hipLaunchKernelGGL(k_snes_bc, dim3(blocks_for(boundary_points(c->g), IM_TPB)), dim3(IM_TPB), 0, st, c->g, c->f[VFS_UCONT]);
     ucat_stale(c);
     rc = c2c(c);
     if (rc) return fail(rc);

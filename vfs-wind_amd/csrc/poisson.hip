@@ -2564,7 +2564,7 @@ static int remove_mean(vfs_ctx *c, const unsigned char *row, double *x)
     hipStream_t st = c->stream;
     const long long n = c->g.n;
     double *out = c->red + 2 * RED_BLOCKS;
-    hipLaunchKernelGGL(k_row_sum, dim3(krylov_blocks(n)), dim3(RED_THREADS), 0, st, n, row, x, c->red, out, red_quiet(c));
+    hipLaunchKernelGGL(k_row_sum, dim3(reduce_blocks(n)), dim3(RED_THREADS), 0, st, n, row, x, c->red, out, red_quiet(c));
     hipLaunchKernelGGL(k_sub_mean, dim3(blocks_for(n, PTPB)), dim3(PTPB), 0, st, n, row, out, x);
     VFS_LAUNCH_CHECK("remove mean");
     return VFS_OK;
@@ -2582,8 +2582,9 @@ int poisson_apply(vfs_ctx *c, const double *x, double *y)
 
 // FGMRES; with a network: warm start and first preconditioner stage from the
 // network, and *fell_back set (solve abandoned) when after three iterations
-// the residual is above half of its value after the warm start
-static int fgmres(vfs_ctx *c, const vfs_solve_opts *o, vfs_unet *net, vfs_solve_stats *stats, bool *fell_back)
+// the residual is above half of its value after the warm start; without sync
+// the last kernels may still run on return
+static int fgmres(vfs_ctx *c, const vfs_solve_opts *o, vfs_unet *net, vfs_solve_stats *stats, bool *fell_back, bool sync = true)
 {
     using clk = std::chrono::steady_clock;
     auto t0 = clk::now();
@@ -2737,7 +2738,7 @@ static int fgmres(vfs_ctx *c, const vfs_solve_opts *o, vfs_unet *net, vfs_solve_
     }
     rc = remove_mean(c, L.row, x);  // poisson_hypre.c:608
     if (rc) return rc;
-    VFS_HIP(hipStreamSynchronize(st));
+    if (sync) VFS_HIP(hipStreamSynchronize(st));
     if (stats) {
         stats->iterations = it;
         stats->relres = rel;
@@ -2748,10 +2749,10 @@ static int fgmres(vfs_ctx *c, const vfs_solve_opts *o, vfs_unet *net, vfs_solve_
     return VFS_OK;
 }
 
-int poisson_solve(vfs_ctx *c, const vfs_solve_opts *o, vfs_solve_stats *stats)
+int poisson_solve(vfs_ctx *c, const vfs_solve_opts *o, vfs_solve_stats *stats, bool sync)
 {
     bool fb = false;
-    return fgmres(c, o, nullptr, stats, &fb);
+    return fgmres(c, o, nullptr, stats, &fb, sync);
 }
 
 int poisson_solve_learned(vfs_ctx *c, vfs_unet *net, const vfs_solve_opts *o, vfs_solve_stats *stats)

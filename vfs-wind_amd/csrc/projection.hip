@@ -21,8 +21,9 @@ int periodic_fix_grid(hipStream_t st, const Grid &g, double *f, int nc, int mode
 // ---------------------------------------------------------------------------
 
 __global__ void k_poisson_rhs(Grid g, double fac, const double *__restrict__ ucont, const double *__restrict__ nvert,
-                              const double *__restrict__ aj, double *__restrict__ b, double *__restrict__ part)
+                              const double *__restrict__ aj, double *__restrict__ b, double *part, double *out, RedSync rs)
 {
+    __shared__ double res[2];
     double sb = 0, sa = 0;
     for (long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x; t < g.n; t += (long long)gridDim.x * blockDim.x) {
         const int i = t % g.mx;
@@ -47,7 +48,11 @@ __global__ void k_poisson_rhs(Grid g, double fac, const double *__restrict__ uco
     }
     sb = block_reduce<OpSum>(sb);
     sa = block_reduce<OpSum>(sa);
-    if (threadIdx.x == 0) { part[blockIdx.x] = sb; part[RED_BLOCKS + blockIdx.x] = sa; }
+    if (threadIdx.x == 0) {
+        red_put(part + blockIdx.x, sb);
+        red_put(part + RED_BLOCKS + blockIdx.x, sa);
+    }
+    if (red_last(rs, gridDim.x)) red_finish_rows<OpSum>(rs, 2, gridDim.x, part, out, res);
 }
 
 // The same over the interior with k-marching tiles (ucont.z of plane k-1
@@ -55,8 +60,9 @@ __global__ void k_poisson_rhs(Grid g, double fac, const double *__restrict__ uco
 __global__ void __launch_bounds__(KM_I * KM_J) k_poisson_rhs_km(Grid g, int kc, double fac, const double *__restrict__ ucont,
                                                                const double *__restrict__ nvert,
                                                                const double *__restrict__ aj, double *__restrict__ b,
-                                                               double *__restrict__ part)
+                                                               double *part, double *out, RedSync rs)
 {
+    __shared__ double res[2];
     double sb = 0, sa = 0;
     int i, j, k0, k1;
     if (km_tile(g, kc, i, j, k0, k1)) {
@@ -85,7 +91,11 @@ __global__ void __launch_bounds__(KM_I * KM_J) k_poisson_rhs_km(Grid g, int kc, 
     }
     sb = block_reduce<OpSum>(sb);
     sa = block_reduce<OpSum>(sa);
-    if (threadIdx.x == 0) { part[blockIdx.x] = sb; part[RED_BLOCKS + blockIdx.x] = sa; }
+    if (threadIdx.x == 0) {
+        red_put(part + blockIdx.x, sb);
+        red_put(part + RED_BLOCKS + blockIdx.x, sa);
+    }
+    if (red_last(rs, gridDim.x)) red_finish_rows<OpSum>(rs, 2, gridDim.x, part, out, res);
 }
 
 // planes per block of a k-marching reduction so that the blocks fit the
@@ -125,22 +135,18 @@ int poisson_rhs(vfs_ctx *c)
     const double coeff = 1.;  // time_coeff(), poisson.c:23-31
     const double fac = -1.0 / c->p.dt * c->p.st * coeff;
     const int kc = km_reductions() ? km_chunk(g) : 0;
-    int nparts = RED_BLOCKS;
+    double *sums = c->red + 2 * RED_BLOCKS;
     if (kc > 0) {
         int rc = zero_ghosts(c, c->f[VFS_B]);
         if (rc) return rc;
-        nparts = (int)km_blocks(g, kc);
-        hipLaunchKernelGGL(k_poisson_rhs_km, dim3(nparts), dim3(KM_I * KM_J), 0, st, g, kc, fac, c->f[VFS_UCONT],
-                           c->f[VFS_NVERT], c->f[VFS_AJ], c->f[VFS_B], c->red);
+        hipLaunchKernelGGL(k_poisson_rhs_km, dim3(km_blocks(g, kc)), dim3(KM_I * KM_J), 0, st, g, kc, fac, c->f[VFS_UCONT],
+                           c->f[VFS_NVERT], c->f[VFS_AJ], c->f[VFS_B], c->red, sums, red_quiet(c));
     } else {
         hipLaunchKernelGGL(k_poisson_rhs, dim3(RED_BLOCKS), dim3(RED_THREADS), 0, st, g, fac, c->f[VFS_UCONT],
-                           c->f[VFS_NVERT], c->f[VFS_AJ], c->f[VFS_B], c->red);
+                           c->f[VFS_NVERT], c->f[VFS_AJ], c->f[VFS_B], c->red, sums, red_quiet(c));
     }
-    hipLaunchKernelGGL(finish_reduce<OpSum>, dim3(1), dim3(RED_THREADS), 0, st, c->red, nparts, c->red + 2 * RED_BLOCKS);
-    hipLaunchKernelGGL(finish_reduce<OpSum>, dim3(1), dim3(RED_THREADS), 0, st, c->red + RED_BLOCKS, nparts,
-                       c->red + 2 * RED_BLOCKS + 1);
-    hipLaunchKernelGGL(k_null_scale, dim3(blocks_for(g.n, QTPB)), dim3(QTPB), 0, st, g, c->red + 2 * RED_BLOCKS,
-                       c->f[VFS_NVERT], c->f[VFS_AJ], c->f[VFS_B]);
+    hipLaunchKernelGGL(k_null_scale, dim3(blocks_for(g.n, QTPB)), dim3(QTPB), 0, st, g, sums, c->f[VFS_NVERT],
+                       c->f[VFS_AJ], c->f[VFS_B]);
     VFS_LAUNCH_CHECK("poisson rhs");
     return VFS_OK;
 }
@@ -149,41 +155,32 @@ int poisson_rhs(vfs_ctx *c)
 // a13: Convert_Phi2_Phi + UpdatePressure (poisson.c:98-186, 3137-3297)
 // ---------------------------------------------------------------------------
 
-__global__ void k_phi_mask(Grid g, double th, const double *__restrict__ nvert, double *__restrict__ phi)
+// Phi keeps the row values only (Convert_Phi2_Phi), P += Phi in the fluid cells
+// (UpdatePressure), and both get their periodic ghosts: each point that is no
+// periodic ghost also writes those that copy it.  One pass; the mask, the
+// update and a periodic fix of each were four launches.
+__global__ void k_update_p(Grid g, double th, const double *__restrict__ nvert, double *__restrict__ phi, double *__restrict__ p)
 {
     long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x;
     if (t >= g.n) return;
-    const int i = t % g.mx;
-    const long long r = t / g.mx;
-    const int j = r % g.my, k = r / g.my;
-    bool rowc = i >= 1 && i < g.mx - 1 && j >= 1 && j < g.my - 1 && k >= 1 && k < g.mz - 1 && nvert[t] < th;
-    if (!rowc) phi[t] = 0;
-}
-
-__global__ void k_update_p(Grid g, const double *__restrict__ nvert, const double *__restrict__ phi, double *__restrict__ p)
-{
-    long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-    if (t >= g.n) return;
-    const int i = t % g.mx;
-    const long long r = t / g.mx;
-    const int j = r % g.my, k = r / g.my;
-    if (i < 1 || i >= g.mx - 1 || j < 1 || j >= g.my - 1 || k < 1 || k >= g.mz - 1) return;
-    if (nvert[t] < 0.1) p[t] += phi[t];
-    if (nvert[t] > 1.1) p[t] = 0;
+    const int t32 = (int)t, i = t32 % g.mx, r = t32 / g.mx, j = r % g.my, k = r / g.my;
+    if (is_periodic_ghost(g, k, j, i)) return;
+    const bool in = i >= 1 && i < g.mx - 1 && j >= 1 && j < g.my - 1 && k >= 1 && k < g.mz - 1;
+    const double nv = nvert[t], f = in && nv < th ? phi[t] : 0.0;
+    double v = p[t];
+    if (in && nv < 0.1) v += f;
+    if (in && nv > 1.1) v = 0;
+    store_periodic(g, phi, k, j, i, f);
+    store_periodic(g, p, k, j, i, v);
 }
 
 int update_pressure(vfs_ctx *c)
 {
     const Grid &g = c->g;
-    hipStream_t st = c->stream;
-    const unsigned nb = blocks_for(g.n, QTPB);
-    hipLaunchKernelGGL(k_phi_mask, dim3(nb), dim3(QTPB), 0, st, g, c->p.poisson_threshold, c->f[VFS_NVERT], c->f[VFS_PHI]);
-    VFS_LAUNCH_CHECK("phi mask");
-    int rc = periodic_fix_grid(st, g, c->f[VFS_PHI], 1, 0);
-    if (rc) return rc;
-    hipLaunchKernelGGL(k_update_p, dim3(nb), dim3(QTPB), 0, st, g, c->f[VFS_NVERT], c->f[VFS_PHI], c->f[VFS_P]);
+    hipLaunchKernelGGL(k_update_p, dim3(blocks_for(g.n, QTPB)), dim3(QTPB), 0, c->stream, g, c->p.poisson_threshold,
+                       c->f[VFS_NVERT], c->f[VFS_PHI], c->f[VFS_P]);
     VFS_LAUNCH_CHECK("update pressure");
-    return periodic_fix_grid(st, g, c->f[VFS_P], 1, 0);
+    return VFS_OK;
 }
 
 // ---------------------------------------------------------------------------
@@ -341,8 +338,22 @@ int projection(vfs_ctx *c)
 // a15: Divergence (main.c:936-1074)
 // ---------------------------------------------------------------------------
 
+// the block's maximum; without counters (rs.ctr null) a second launch finishes
+// the partials, else the block that ends last
+__device__ inline void divergence_max(double v, double *part, double *out, const RedSync &rs)
+{
+    __shared__ double res[1];
+    v = block_reduce<OpMax>(v);
+    if (!rs.ctr) {
+        if (threadIdx.x == 0) part[blockIdx.x] = v;
+        return;
+    }
+    if (threadIdx.x == 0) red_put(part + blockIdx.x, v);
+    if (red_last(rs, gridDim.x)) red_finish_rows<OpMax>(rs, 1, gridDim.x, part, out, res);
+}
+
 __global__ void k_divergence(Grid g, const double *__restrict__ ucont, const double *__restrict__ aj,
-                             const double *__restrict__ nvert, double *__restrict__ part)
+                             const double *__restrict__ nvert, double *part, double *out, RedSync rs)
 {
     const long long ni = (long long)(g.mx - 2) * (g.my - 2) * (g.mz - 2);
     double v = 0;
@@ -358,15 +369,15 @@ __global__ void k_divergence(Grid g, const double *__restrict__ ucont, const dou
             d = 0.;
         v = fmax(v, d);
     }
-    v = block_reduce<OpMax>(v);
-    if (threadIdx.x == 0) part[blockIdx.x] = v;
+    divergence_max(v, part, out, rs);
 }
 
 // The same with k-marching tiles: ucont.z and nvert of the planes k-1, k,
 // k+1 at the thread's own (i, j) carried in registers
 __global__ void __launch_bounds__(KM_I * KM_J) k_divergence_km(Grid g, int kc, const double *__restrict__ ucont,
                                                               const double *__restrict__ aj,
-                                                              const double *__restrict__ nvert, double *__restrict__ part)
+                                                              const double *__restrict__ nvert, double *part, double *out,
+                                                              RedSync rs)
 {
     double v = 0;
     int i, j, k0, k1;
@@ -384,27 +395,22 @@ __global__ void __launch_bounds__(KM_I * KM_J) k_divergence_km(Grid g, int kc, c
             nv0 = nvp;
         }
     }
-    v = block_reduce<OpMax>(v);
-    if (threadIdx.x == 0) part[blockIdx.x] = v;
+    divergence_max(v, part, out, rs);
 }
 
 int divergence(vfs_ctx *c, double *out)
 {
     hipStream_t st = c->stream;
     const int kc = km_reductions() ? km_chunk(c->g) : 0;
-    int nparts = RED_BLOCKS;
-    if (kc > 0) {
-        nparts = (int)km_blocks(c->g, kc);
-        hipLaunchKernelGGL(k_divergence_km, dim3(nparts), dim3(KM_I * KM_J), 0, st, c->g, kc, c->f[VFS_UCONT], c->f[VFS_AJ],
-                           c->f[VFS_NVERT], c->red);
-    } else {
+    if (kc > 0)
+        hipLaunchKernelGGL(k_divergence_km, dim3(km_blocks(c->g, kc)), dim3(KM_I * KM_J), 0, st, c->g, kc, c->f[VFS_UCONT],
+                           c->f[VFS_AJ], c->f[VFS_NVERT], c->red, c->red + RED_BLOCKS, red_sync(c));
+    else
         hipLaunchKernelGGL(k_divergence, dim3(RED_BLOCKS), dim3(RED_THREADS), 0, st, c->g, c->f[VFS_UCONT], c->f[VFS_AJ],
-                           c->f[VFS_NVERT], c->red);
-    }
-    hipLaunchKernelGGL(finish_reduce<OpMax>, dim3(1), dim3(RED_THREADS), 0, st, c->red, nparts, c->red + RED_BLOCKS);
+                           c->f[VFS_NVERT], c->red, c->red + RED_BLOCKS, red_sync(c));
     VFS_LAUNCH_CHECK("divergence");
-    VFS_HIP(hipMemcpyAsync(c->red_host, c->red + RED_BLOCKS, sizeof(double), hipMemcpyDeviceToHost, st));
-    VFS_HIP(hipStreamSynchronize(st));
+    const int rc = red_wait(c);
+    if (rc) return rc;
     *out = c->red_host[0];
     return VFS_OK;
 }
@@ -460,9 +466,11 @@ int divergence_noalloc(const vfs_params &p, const double *ucont, const double *a
     if (rc) return rc;
     // every block writes its own partial, so nothing needs clearing between calls
     if (kc > 0)
-        hipLaunchKernelGGL(k_divergence_km, dim3((unsigned)nparts), dim3(KM_I * KM_J), 0, st, g, kc, ucont, aj, nvert, part);
+        hipLaunchKernelGGL(k_divergence_km, dim3((unsigned)nparts), dim3(KM_I * KM_J), 0, st, g, kc, ucont, aj, nvert, part, nullptr,
+                           RedSync{});
     else
-        hipLaunchKernelGGL(k_divergence, dim3(RED_BLOCKS), dim3(RED_THREADS), 0, st, g, ucont, aj, nvert, part);
+        hipLaunchKernelGGL(k_divergence, dim3(RED_BLOCKS), dim3(RED_THREADS), 0, st, g, ucont, aj, nvert, part, nullptr,
+                           RedSync{});
     hipLaunchKernelGGL(finish_reduce<OpMax>, dim3(1), dim3(RED_THREADS), 0, st, part, (int)nparts, maxdiv);
     VFS_LAUNCH_CHECK("divergence_noalloc");
     return VFS_OK;

@@ -178,6 +178,7 @@ int vfs_ctx_create(const vfs_params *params, vfs_ctx **out)
     c->face = c->pucont = c->snap = c->fpc = c->red = c->red_host = c->inflow_plane = nullptr;
     c->red_ctr = nullptr;
     c->red_seq = 0;
+    for (hipEvent_t &ev : c->step_ev) ev = nullptr;
     c->ps = nullptr;
     c->cs_mode = vfs::CS_PARAM;
     c->dyn = nullptr;
@@ -247,6 +248,8 @@ int vfs_ctx_destroy(vfs_ctx *c)
     if (c->inflow_plane) hipFree(c->inflow_plane);
     if (c->red_host) hipHostFree(c->red_host);
     if (c->red_ctr) hipFree(c->red_ctr);
+    for (hipEvent_t ev : c->step_ev)
+        if (ev) hipEventDestroy(ev);
     if (c->imp_ws) hipFree(c->imp_ws);
     if (c->dyn) hipFree(c->dyn);
     if (c->ev_pool) {
@@ -453,21 +456,24 @@ int vfs::runge_kutta(vfs_ctx *c, bool lazy_ucat)
     int rc = vfs::inflow_flux(c, nullptr);  // rhs.c:1612
     if (!rc) rc = vfs::form_bcs(c, 0);
     if (rc) return rc;
-    const size_t n3 = 3 * (size_t)c->g.n;
-    VFS_HIP(hipMemcpyAsync(c->pucont, c->f[VFS_UCONT], n3 * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
-    for (int s = 0; s < 4; s++) {
+    // pUcont stays in VFS_UCONT's own buffer: the first three stages write and
+    // read a second buffer that stands in for it, the last writes back over pUcont
+    // point by point.  (A copy of Ucont instead took 130 us at 256x192x256.)
+    double *const own = c->f[VFS_UCONT];
+    rc = vfs::c2c(c);
+    for (int s = 0; s < 4 && !rc; s++) {
         // the reference calls Contra2Cart at the start of every stage
         // (rhs.c:1642); from the second stage on Ucont is unchanged since the
         // previous stage's closing call and Contra2Cart is idempotent, so
         // that call would rewrite the same Ucat
-        if (s == 0) rc = vfs::c2c(c);
-        if (rc) return rc;
         // Rhs = 0; Formfunction_2(Rhs, 1); Rhs -= dP; Ucont = a*Rhs + pUcont  (rhs.c:1647-1658)
-        rc = vfs::formfunction2(c, 1.0, c->pucont, alfa[s] * c->p.dt * c->p.st, c->f[VFS_UCONT]);
-        if (rc) return rc;
-        if (s < 3 || !lazy) rc = vfs::c2c(c);
-        if (rc) return rc;
+        double *const out = s < 3 ? c->pucont : own;
+        rc = vfs::formfunction2(c, 1.0, own, alfa[s] * c->p.dt * c->p.st, out);
+        c->f[VFS_UCONT] = out;
+        if (!rc && (s < 3 || !lazy)) rc = vfs::c2c(c);
     }
+    c->f[VFS_UCONT] = own;
+    if (rc) return rc;
     return vfs::form_bcs(c, 1, lazy);
 }
 
@@ -594,13 +600,19 @@ static int step_common(vfs_ctx *c, const vfs_solve_opts *o, const vfs_newton_opt
 {
     using clk = std::chrono::steady_clock;
     auto t0 = clk::now();
+    // the stages' times come from events on the stream, so that the host goes
+    // on enqueuing where it would wait to read a clock
+    for (hipEvent_t &ev : c->step_ev)
+        if (!ev) VFS_HIP(hipEventCreateWithFlags(&ev, hipEventDisableSystemFence));
+    if (st) VFS_HIP(hipEventRecord(c->step_ev[0], c->stream));
     int rc = c->p.pseudo_periodic ? vfs_pseudo_periodic_plane(c) : VFS_OK;  // solvers.c:355-358
-    if (!rc) rc = vfs_calc_k_flux(c, nullptr);              // solvers.c:363
+    if (!rc) rc = vfs::calc_k_flux_start(c);                // solvers.c:363
     if (!rc && c->p.les) rc = vfs::c2c(c);                  // solvers.c:368
     const int freq = c->p.dynamic_freq < 1 ? 1 : c->p.dynamic_freq;  // main.c:1439
     if (!rc && c->p.les && (c->ti % freq == 0 || c->ti == c->tistart))
         rc = vfs::smagorinsky_constant(c, c->ti, c->tistart, c->rstart);  // solvers.c:369
     if (!rc && c->p.les) rc = vfs::eddy_viscosity(c);       // solvers.c:370
+    if (!rc) rc = vfs::calc_k_flux_finish(c, &c->mean_k_flux);
     if (!rc) rc = vfs_pressure_gradient(c);                 // solvers.c:438
     vfs_newton_stats ns;
     std::memset(&ns, 0, sizeof(ns));
@@ -615,15 +627,14 @@ static int step_common(vfs_ctx *c, const vfs_solve_opts *o, const vfs_newton_opt
         }
     }
     if (rc) return rc;
-    VFS_HIP(hipStreamSynchronize(c->stream));
-    auto t1 = clk::now();
+    if (st) VFS_HIP(hipEventRecord(c->step_ev[1], c->stream));
     vfs_solve_stats ps;
     std::memset(&ps, 0, sizeof(ps));
     rc = vfs::poisson_rhs(c);                               // solvers.c:650-655
-    if (!rc) rc = vfs::poisson_solve(c, o, &ps);
+    if (!rc) rc = vfs::poisson_solve(c, o, &ps, false);
     if (rc && rc != VFS_ENOCONV) return rc;
     int conv = rc;
-    auto t2 = clk::now();
+    if (st) VFS_HIP(hipEventRecord(c->step_ev[2], c->stream));
     rc = vfs::update_pressure(c);                           // solvers.c:662
     if (!rc) rc = vfs::projection(c);                       // solvers.c:663
     double md = 0;
@@ -632,11 +643,15 @@ static int step_common(vfs_ctx *c, const vfs_solve_opts *o, const vfs_newton_opt
     auto t3 = clk::now();
     c->ti++;
     if (st) {
+        float ms1 = 0, ms2 = 0;
+        VFS_HIP(hipEventSynchronize(c->step_ev[2]));
+        VFS_HIP(hipEventElapsedTime(&ms1, c->step_ev[0], c->step_ev[1]));
+        VFS_HIP(hipEventElapsedTime(&ms2, c->step_ev[1], c->step_ev[2]));
         st->poisson_iterations = ps.iterations;
         st->poisson_relres = ps.relres;
         st->maxdiv = md;
-        st->ms_momentum = std::chrono::duration<double, std::milli>(t1 - t0).count();
-        st->ms_poisson = std::chrono::duration<double, std::milli>(t2 - t1).count();
+        st->ms_momentum = ms1;
+        st->ms_poisson = ms2;
         st->ms_total = std::chrono::duration<double, std::milli>(t3 - t0).count();
         st->newton_iterations = ns.newton_iterations;
         st->linear_iterations = ns.linear_iterations;

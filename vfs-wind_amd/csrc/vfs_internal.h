@@ -61,6 +61,33 @@ __host__ __device__ inline bool periodic_src(const Grid &g, int k, int j, int i,
     return fi || fj || fk;
 }
 
+// f = v at point (k, j, i), which is no periodic ghost, and at the periodic
+// ghosts that copy it (what a periodic fix afterwards would store there)
+__device__ inline void store_periodic(const Grid &g, double *__restrict__ f, int k, int j, int i, double v)
+{
+    const long long q = ((long long)k * g.my + j) * g.mx + i;
+    f[q] = v;
+    const long long di = !g.pi ? 0 : i == 1 ? g.mx - 2 : i == g.mx - 2 ? 2 - g.mx : 0;
+    const long long dj = !g.pj ? 0 : (long long)g.mx * (j == 1 ? g.my - 2 : j == g.my - 2 ? 2 - g.my : 0);
+    const long long dk = !g.pk ? 0 : g.plane * (k == 1 ? g.mz - 2 : k == g.mz - 2 ? 2 - g.mz : 0);
+    if (di) f[q + di] = v;
+    if (dj) {
+        f[q + dj] = v;
+        if (di) f[q + dj + di] = v;
+    }
+    if (dk) {
+        f[q + dk] = v;
+        if (di) f[q + dk + di] = v;
+        if (dj) f[q + dk + dj] = v;
+        if (dj && di) f[q + dk + dj + di] = v;
+    }
+}
+// whether (k, j, i) is a ghost of a periodic direction
+__device__ inline bool is_periodic_ghost(const Grid &g, int k, int j, int i)
+{
+    return (g.pi && (i == 0 || i == g.mx - 1)) || (g.pj && (j == 0 || j == g.my - 1)) || (g.pk && (k == 0 || k == g.mz - 1));
+}
+
 // the cell metrics of point q into v[0..9]: csi xyz, eta xyz, zet xyz, aj
 __device__ inline void load_cell_metrics(const double *__restrict__ csi, const double *__restrict__ eta,
                                          const double *__restrict__ zet, const double *__restrict__ aj, long long q,
@@ -236,6 +263,7 @@ struct vfs_ctx {
     double *dyn;
     // time-step index of the step drivers (ti, tistart, rstart_flg)
     int ti, tistart, rstart;
+    hipEvent_t step_ev[3];  // the step drivers' momentum and Poisson times (made at the first step)
     // per-kernel timing (vfs_profile): event pairs recorded around launches
     int prof_on;
     unsigned prof_mask;                // kernel ids recorded while prof_on (bit id)
@@ -297,6 +325,8 @@ int pseudo_periodic_plane(vfs_ctx *c);
 int eddy_viscosity(vfs_ctx *c);
 int pressure_gradient(vfs_ctx *c);
 int calc_k_flux(vfs_ctx *c, double *out);
+int calc_k_flux_start(vfs_ctx *c);
+int calc_k_flux_finish(vfs_ctx *c, double *out);
 int mean_k_area(vfs_ctx *c, double *out);
 // FormFunction_SNES's residual (momentum.c:2237-2336) formed in Formfunction_2's
 // cell pass: r = (0 - u/dt + u_o/dt) + scale F(u) + 0.5 RHS_o - dP (+ F_eul),
@@ -318,7 +348,7 @@ bool formfunction2_fused(const vfs_ctx *c);
 int min_dt(vfs_ctx *c, double *out);
 int poisson_rhs(vfs_ctx *c);
 int poisson_apply(vfs_ctx *c, const double *x, double *y);
-int poisson_solve(vfs_ctx *c, const vfs_solve_opts *o, vfs_solve_stats *st);
+int poisson_solve(vfs_ctx *c, const vfs_solve_opts *o, vfs_solve_stats *st, bool sync = true);
 int poisson_solve_learned(vfs_ctx *c, vfs_unet *net, const vfs_solve_opts *o, vfs_solve_stats *st);
 void poisson_free(vfs_ctx *c);
 int update_pressure(vfs_ctx *c);

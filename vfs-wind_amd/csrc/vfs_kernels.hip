@@ -30,10 +30,9 @@ constexpr int TPB = 256;
 // cell's source wraps all periodic directions at once (periodic_src), so it
 // is never a periodic ghost itself and the planes do not depend on each
 // other; a cell on two planes is written twice with the same value.
-__global__ void k_periodic_planes(Grid g, double *__restrict__ f, int nc, int mode)
+// (k, j, i) of the t-th periodic ghost point; false past the last
+__device__ inline bool periodic_ghost(const Grid &g, long long t, int &k, int &j, int &i)
 {
-    long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-    int i, j, k;
     const long long n0 = g.pi ? 2LL * g.my * g.mz : 0, n1 = g.pj ? 2LL * g.mx * g.mz : 0;
     const long long n2 = g.pk ? 2LL * g.mx * g.my : 0;
     if (t < n0) {
@@ -46,9 +45,15 @@ __global__ void k_periodic_planes(Grid g, double *__restrict__ f, int nc, int mo
         i = t % g.mx; long long r = t / g.mx;
         j = r % g.my; int side = (int)(r / g.my); k = side ? g.mz - 1 : 0;
     } else {
-        return;
+        return false;
     }
-    int a, b, c, fi, fj, fk;
+    return true;
+}
+
+__global__ void k_periodic_planes(Grid g, double *__restrict__ f, int nc, int mode)
+{
+    int i, j, k, a, b, c, fi, fj, fk;
+    if (!periodic_ghost(g, blockIdx.x * (long long)blockDim.x + threadIdx.x, k, j, i)) return;
     if (!periodic_src(g, k, j, i, c, b, a, fi, fj, fk)) return;
     long long d = gidx(g, k, j, i), s = gidx(g, c, b, a);
     if (mode == 0) {
@@ -238,17 +243,21 @@ int launch_metrics(vfs_ctx *c, const Grid &g, const double *coor, double *const 
 // a2: Contra2Cart_2 (rhs.c:65-749)
 // ---------------------------------------------------------------------------
 
-// interior Cramer solve, rhs.c:158-247
-__device__ inline void c2c_point(const Grid &g, int k, int j, int i, const double *__restrict__ ucont,
-                                 const double *__restrict__ csi, const double *__restrict__ eta,
-                                 const double *__restrict__ zet, const double *__restrict__ nvert,
-                                 double *__restrict__ ucat)
+// interior Cramer solve, rhs.c:158-247, into u; false where the cell is blanked
+// (its Ucat stays).  The faces at index 0 of a periodic direction are read from
+// the interior faces their ghosts copy, so the ghosts need not be filled first.
+__device__ inline bool c2c_value(const Grid &g, int k, int j, int i, const double *ucont, const double *__restrict__ csi,
+                                 const double *__restrict__ eta, const double *__restrict__ zet,
+                                 const double *__restrict__ nvert, double u[3])
 {
-    const long long q = gidx(g, k, j, i);
-    if (nvert && nvert[q] >= 0.1) return;  // nvert == nullptr: no point is blanked
-    double q0 = 0.5 * (ucont[3 * gidx(g, k, j, i - 1) + 0] + ucont[3 * q + 0]);
-    double q1 = 0.5 * (ucont[3 * gidx(g, k, j - 1, i) + 1] + ucont[3 * q + 1]);
-    double q2 = 0.5 * (ucont[3 * gidx(g, k - 1, j, i) + 2] + ucont[3 * q + 2]);
+    const long long q = ((long long)k * g.my + j) * g.mx + i;
+    if (nvert && nvert[q] >= 0.1) return false;  // nvert == nullptr: no point is blanked
+    const long long qi = g.pi && i == 1 ? q + g.mx - 3 : q - 1;
+    const long long qj = g.pj && j == 1 ? q + (long long)(g.my - 3) * g.mx : q - g.mx;
+    const long long qk = g.pk && k == 1 ? q + (long long)(g.mz - 3) * g.plane : q - g.plane;
+    double q0 = 0.5 * (ucont[3 * qi + 0] + ucont[3 * q + 0]);
+    double q1 = 0.5 * (ucont[3 * qj + 1] + ucont[3 * q + 1]);
+    double q2 = 0.5 * (ucont[3 * qk + 2] + ucont[3 * q + 2]);
     const double m00 = csi[3 * q], m01 = csi[3 * q + 1], m02 = csi[3 * q + 2];
     const double m10 = eta[3 * q], m11 = eta[3 * q + 1], m12 = eta[3 * q + 2];
     const double m20 = zet[3 * q], m21 = zet[3 * q + 1], m22 = zet[3 * q + 2];
@@ -256,25 +265,60 @@ __device__ inline void c2c_point(const Grid &g, int k, int j, int i, const doubl
     double det0 = q0 * (m11 * m22 - m12 * m21) - q1 * (m01 * m22 - m02 * m21) + q2 * (m01 * m12 - m02 * m11);
     double det1 = -q0 * (m10 * m22 - m12 * m20) + q1 * (m00 * m22 - m02 * m20) - q2 * (m00 * m12 - m02 * m10);
     double det2 = q0 * (m10 * m21 - m11 * m20) - q1 * (m00 * m21 - m01 * m20) + q2 * (m00 * m11 - m01 * m10);
-    ucat[3 * q + 0] = det0 / det;
-    ucat[3 * q + 1] = det1 / det;
-    ucat[3 * q + 2] = det2 / det;
+    u[0] = det0 / det;
+    u[1] = det1 / det;
+    u[2] = det2 / det;
+    return true;
+}
+__device__ inline void c2c_point(const Grid &g, int k, int j, int i, const double *ucont, const double *__restrict__ csi,
+                                 const double *__restrict__ eta, const double *__restrict__ zet,
+                                 const double *__restrict__ nvert, double *__restrict__ ucat)
+{
+    double u[3];
+    if (!c2c_value(g, k, j, i, ucont, csi, eta, zet, nvert, u)) return;
+    const long long q = gidx(g, k, j, i);
+    for (int c = 0; c < 3; c++) ucat[3 * q + c] = u[c];
 }
 
-__global__ void k_c2c_interior(Grid g, const double *__restrict__ ucont, const double *__restrict__ csi,
+// ghost points of the periodic directions (both planes of each in turn)
+__host__ __device__ inline long long periodic_ghosts(const Grid &g)
+{
+    return (g.pi ? 2LL * g.my * g.mz : 0) + (g.pj ? 2LL * g.mx * g.mz : 0) + (g.pk ? 2LL * g.mx * g.my : 0);
+}
+
+// Blocks of the first `zint` z layers take the interior cells; the others take
+// the periodic ghost points, where they copy Ucont (rhs.c:129-156) and form the
+// Ucat of the cell the ghost stands for (rhs.c:254-291) from Ucont again, since
+// that cell's own thread is writing it.  Separate periodic passes before and after
+// the interior one cost a launch each.
+__global__ void k_c2c_interior(Grid g, int zint, double *ucont, const double *__restrict__ csi,
                                const double *__restrict__ eta, const double *__restrict__ zet,
                                const double *__restrict__ nvert, double *__restrict__ ucat)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
-    const int j = blockIdx.y + 1, k = blockIdx.z + 1;
-    if (i >= g.mx - 1) return;
-    c2c_point(g, k, j, i, ucont, csi, eta, zet, nvert, ucat);
+    if ((int)blockIdx.z < zint) {
+        const int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
+        const int j = blockIdx.y + 1, k = blockIdx.z + 1;
+        if (i >= g.mx - 1) return;
+        c2c_point(g, k, j, i, ucont, csi, eta, zet, nvert, ucat);
+        return;
+    }
+    const long long blk = ((long long)(blockIdx.z - zint) * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
+    int k, j, i, c, b, a, fi, fj, fk;
+    if (!periodic_ghost(g, blk * blockDim.x + threadIdx.x, k, j, i)) return;
+    if (!periodic_src(g, k, j, i, c, b, a, fi, fj, fk)) return;
+    const long long d = gidx(g, k, j, i), s = gidx(g, c, b, a);
+    for (int q = 0; q < 3; q++) ucont[3 * d + q] = ucont[3 * s + q];
+    double u[3];
+    const bool in = a >= 1 && a <= g.mx - 2 && b >= 1 && b <= g.my - 2 && c >= 1 && c <= g.mz - 2;
+    if (!in || !c2c_value(g, c, b, a, ucont, csi, eta, zet, nvert, u))
+        for (int q = 0; q < 3; q++) u[q] = ucat[3 * s + q];
+    for (int q = 0; q < 3; q++) ucat[3 * d + q] = u[q];
 }
 
 // the interior cells whose Contra2Cart inputs k_wall_flux may change: the
 // planes i = 1 / i = mx-2 / j = 1 / j = my-2 next to a wall face (bc 1 or 10)
 __device__ inline bool wall_face(const Grid &g, int side) { return g.bc[side] == 1 || g.bc[side] == 10; }
-__global__ void k_c2c_walls(Grid g, const double *__restrict__ ucont, const double *__restrict__ csi,
+__global__ void k_c2c_walls(Grid g, const double *ucont, const double *__restrict__ csi,
                             const double *__restrict__ eta, const double *__restrict__ zet,
                             const double *__restrict__ nvert, double *__restrict__ ucat)
 {
@@ -319,33 +363,40 @@ __device__ inline void slip_fill(const Grid &g, const double *csi, const double 
 }
 
 // ghost-cell BC fill, rhs.c:300-680, for the boundary planes of the
-// non-periodic directions.  Each ghost cell is visited by exactly one thread
-// (planes of a later axis skip cells owned by an earlier axis).
-__global__ void k_c2c_bc(Grid g, int axis, const double *__restrict__ L2, const double *__restrict__ uold,
+// non-periodic directions, all in one launch.  Each ghost cell is visited by
+// exactly one thread (planes of a later axis skip cells owned by an earlier
+// axis) and no rule reads what another cell's writes (L2 is a snapshot where one
+// would).  On a plane, a ghost of the periodic directions evaluates the rules of
+// the point it stands for, whose value the periodic fix at the end of
+// Contra2Cart (rhs.c:712-748) would copy to it.
+__global__ void k_c2c_bc(Grid g, const double *L2, const double *__restrict__ uold,
                          const double *__restrict__ csi, const double *__restrict__ eta,
-                         const double *__restrict__ zet, const double *__restrict__ nvert, double *__restrict__ ucat)
+                         const double *__restrict__ zet, const double *__restrict__ nvert, double *ucat)
 {
     long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x;
+    const long long n0 = g.pi ? 0 : 2LL * g.my * g.mz, n1 = g.pj ? 0 : 2LL * g.mx * g.mz, n2 = g.pk ? 0 : 2LL * g.mx * g.my;
     int i, j, k;
-    if (axis == 0) {
-        if (t >= 2LL * g.my * g.mz) return;
+    if (t < n0) {
         int side = t & 1; long long r = t >> 1;
         j = r % g.my; k = r / g.my; i = side ? g.mx - 1 : 0;
-    } else if (axis == 1) {
-        if (t >= 2LL * g.mx * g.mz) return;
+    } else if ((t -= n0) < n1) {
         i = t % g.mx; long long r = t / g.mx;
         int side = r & 1; k = r >> 1; j = side ? g.my - 1 : 0;
         if (!g.pi && (i == 0 || i == g.mx - 1)) return;
     } else {
-        if (t >= 2LL * g.mx * g.my) return;
+        if ((t -= n1) >= n2) return;
         i = t % g.mx; long long r = t / g.mx;
         j = r % g.my; int side = (int)(r / g.my); k = side ? g.mz - 1 : 0;
         if (!g.pi && (i == 0 || i == g.mx - 1)) return;
         if (!g.pj && (j == 0 || j == g.my - 1)) return;
     }
     const int *bc = g.bc;
-    const long long q = gidx(g, k, j, i);
-    double u[3] = {ucat[3 * q], ucat[3 * q + 1], ucat[3 * q + 2]};
+    const long long q = gidx(g, k, j, i);  // the ghost this thread writes
+    {
+        int c_, b_, a_, fi, fj, fk;
+        if (periodic_src(g, k, j, i, c_, b_, a_, fi, fj, fk)) { k = c_; j = b_; i = a_; }
+    }
+    double u[3] = {0, 0, 0};
     bool touched = false;
     int solid_flag = 0;
     const int mx = g.mx, my = g.my, mz = g.mz;
@@ -478,8 +529,6 @@ int c2c(vfs_ctx *c)
     hipStream_t st = c->stream;
     if (c->ucat_fresh) return VFS_OK;  // would rewrite the same values
     double *ucont = c->f[VFS_UCONT], *ucat = c->f[VFS_UCAT];
-    int rc = periodic_fix(c, ucont, 3, 0);  // rhs.c:129-156
-    if (rc) return rc;
     // The interior cells are a pointwise function of Ucont, the metrics and
     // nvert; where they are known to hold that function already, only the
     // cells whose inputs changed are recomputed.  The ghost-cell passes below
@@ -488,48 +537,49 @@ int c2c(vfs_ctx *c)
     const char *pe = std::getenv("VFS_C2C_PARTIAL");
     const int part = pe && pe[0] == '0' ? (int)UCAT_STALE : c->ucat_part;
     bool nb = false;
-    rc = nvert_all_zero(c, &nb);
+    int rc = nvert_all_zero(c, &nb);
     if (rc) return rc;
     const double *nvi = nb ? nullptr : c->f[VFS_NVERT];  // interior passes skip the blanking test
+    const bool full = part != UCAT_WALLS && part != UCAT_INTERIOR;
     if (part == UCAT_WALLS) {
         const long long ni = (long long)(g.my - 2) * (g.mz - 2), nj = (long long)(g.mx - 2) * (g.mz - 2);
         hipLaunchKernelGGL(k_c2c_walls, dim3(blocks_for(4 * (ni > nj ? ni : nj), TPB)), dim3(TPB), 0, st, g, ucont,
                            c->f[VFS_CSI], c->f[VFS_ETA], c->f[VFS_ZET], nvi, ucat);
         VFS_LAUNCH_CHECK("c2c walls");
-    } else if (part != UCAT_INTERIOR) {
-        dim3 blk(TPB), grd(blocks_for(g.mx - 2, TPB), g.my - 2, g.mz - 2);
-        prof_begin(c, K_C2C);
-        hipLaunchKernelGGL(k_c2c_interior, grd, blk, 0, st, g, ucont, c->f[VFS_CSI], c->f[VFS_ETA], c->f[VFS_ZET], nvi,
-                           ucat);
-        prof_end(c);
+    }
+    const long long ng = periodic_ghosts(g);
+    if (full || ng > 0) {
+        // interior layers (none where the interior stands) and, after them, the
+        // periodic ghosts
+        const int zint = full ? g.mz - 2 : 0;
+        const unsigned gx = blocks_for(g.mx - 2, TPB), gy = g.my - 2;
+        const unsigned gz = (unsigned)((ng + (long long)gx * gy * TPB - 1) / ((long long)gx * gy * TPB));
+        if (full) prof_begin(c, K_C2C);
+        hipLaunchKernelGGL(k_c2c_interior, dim3(gx, gy, zint + gz), dim3(TPB), 0, st, g, zint, ucont, c->f[VFS_CSI],
+                           c->f[VFS_ETA], c->f[VFS_ZET], nvi, ucat);
+        if (full) prof_end(c);
         VFS_LAUNCH_CHECK("c2c interior");
     }
-    rc = periodic_fix(c, ucat, 3, 0);  // rhs.c:254-291
-    if (rc) return rc;
     const double *L2 = ucat;
     const bool corner = corner_rule_active(g);
     if (bc_needs_snapshot(g) || corner) {
         VFS_HIP(hipMemcpyAsync(c->snap, ucat, 3 * (size_t)g.n * sizeof(double), hipMemcpyDeviceToDevice, st));
         L2 = c->snap;
     }
-    const int per[3] = {g.pi, g.pj, g.pk};
-    const long long np[3] = {2LL * g.my * g.mz, 2LL * g.mx * g.mz, 2LL * g.mx * g.my};
-    for (int a = 0; a < 3; a++) {
-        if (per[a]) continue;
-        hipLaunchKernelGGL(k_c2c_bc, dim3(blocks_for(np[a], TPB)), dim3(TPB), 0, st, g, a, L2, c->f[VFS_UCAT_OLD],
+    const long long nb_pts = (g.pi ? 0 : 2LL * g.my * g.mz) + (g.pj ? 0 : 2LL * g.mx * g.mz) + (g.pk ? 0 : 2LL * g.mx * g.my);
+    if (nb_pts > 0)
+        hipLaunchKernelGGL(k_c2c_bc, dim3(blocks_for(nb_pts, TPB)), dim3(TPB), 0, st, g, L2, c->f[VFS_UCAT_OLD],
                            c->f[VFS_CSI], c->f[VFS_ETA], c->f[VFS_ZET], c->f[VFS_NVERT], ucat);
-    }
     VFS_LAUNCH_CHECK("c2c bc");
     if (corner) {
         hipLaunchKernelGGL(k_c2c_corner, dim3(blocks_for(g.mz, TPB)), dim3(TPB), 0, st, g, ucat);
         VFS_LAUNCH_CHECK("c2c corner");
+        rc = periodic_fix(c, ucat, 3, 0);  // rhs.c:712-748 (otherwise the passes above have filled those ghosts)
+        if (rc) return rc;
     }
-    rc = periodic_fix(c, ucat, 3, 0);  // rhs.c:712-748
-    if (!rc) {
-        c->ucat_fresh = true;
-        c->ucat_part = UCAT_STALE;
-    }
-    return rc;
+    c->ucat_fresh = true;
+    c->ucat_part = UCAT_STALE;
+    return VFS_OK;
 }
 
 // ---------------------------------------------------------------------------
@@ -538,8 +588,9 @@ int c2c(vfs_ctx *c)
 
 // outlet plane sums: FluxOut and the area (bcs.c:2127-2175)
 __global__ void k_outlet_sums(Grid g, const double *__restrict__ ucont, const double *__restrict__ zet,
-                              const double *__restrict__ nvert, double *__restrict__ part)
+                              const double *__restrict__ nvert, double *part, double *out, RedSync rs)
 {
+    __shared__ double res[2];
     const int k = g.mz - 1;
     const long long n = (long long)(g.mx - 2) * (g.my - 2);
     double flux = 0, area = 0;
@@ -553,7 +604,11 @@ __global__ void k_outlet_sums(Grid g, const double *__restrict__ ucont, const do
     }
     flux = block_reduce<OpSum>(flux);
     area = block_reduce<OpSum>(area);
-    if (threadIdx.x == 0) { part[blockIdx.x] = flux; part[RED_BLOCKS + blockIdx.x] = area; }
+    if (threadIdx.x == 0) {
+        red_put(part + blockIdx.x, flux);
+        red_put(part + RED_BLOCKS + blockIdx.x, area);
+    }
+    if (red_last(rs, gridDim.x)) red_finish_rows<OpSum>(rs, 2, gridDim.x, part, out, res);
 }
 
 __global__ void k_outlet_scale(Grid g, double flux_in, const double *__restrict__ sums, const double *__restrict__ zet,
@@ -649,8 +704,9 @@ __global__ void k_inflow(Grid g, int mode, int profile, int plane, double inlet_
                          const double *__restrict__ sums, const double *__restrict__ coor,
                          const double *__restrict__ pl, const double *__restrict__ csi, const double *__restrict__ eta,
                          const double *__restrict__ zet, const double *__restrict__ nvert, double *__restrict__ ucont,
-                         double *__restrict__ ucat, double *__restrict__ part)
+                         double *__restrict__ ucat, double *part, double *out, RedSync rs)
 {
+    __shared__ double res[1];
     const long long n = (long long)(g.mx - 2) * (g.my - 2);
     double s = 0;
     for (long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x; t < n; t += (long long)gridDim.x * blockDim.x) {
@@ -707,7 +763,8 @@ __global__ void k_inflow(Grid g, int mode, int profile, int plane, double inlet_
         }
     }
     s = block_reduce<OpSum>(s);
-    if (threadIdx.x == 0) part[blockIdx.x] = s;
+    if (threadIdx.x == 0) red_put(part + blockIdx.x, s);
+    if (red_last(rs, gridDim.x)) red_finish_rows<OpSum>(rs, 1, gridDim.x, part, out, res);
 }
 
 // pseudo_periodic_BC (bcs.c:29-95): plane := ucat(kplane), kplane = (6 mz) / 10
@@ -741,26 +798,19 @@ int inflow_flux(vfs_ctx *c, double *flux_in)
     const double inlet_flux = c->p.inlet_flux;
     // device scalars: sums[0] = flux of the set inlet (flux1), sums[1] = inletArea, sums[2] = FluxIn
     double *sums = c->red + 2 * RED_BLOCKS;
-    hipLaunchKernelGGL(k_inflow, dim3(RED_BLOCKS), dim3(RED_THREADS), 0, st, g, 0, profile, plane, inlet_flux, 0.0,
-                       (const double *)nullptr, c->f[VFS_COOR], c->inflow_plane, c->f[VFS_CSI], c->f[VFS_ETA],
-                       c->f[VFS_ZET], c->f[VFS_NVERT], c->f[VFS_UCONT], c->f[VFS_UCAT], c->red);
-    hipLaunchKernelGGL(finish_reduce<OpSum>, dim3(1), dim3(RED_THREADS), 0, st, c->red, RED_BLOCKS, sums + 1);
-    hipLaunchKernelGGL(k_inflow, dim3(RED_BLOCKS), dim3(RED_THREADS), 0, st, g, 1, profile, plane, inlet_flux, 0.0,
-                       (const double *)sums, c->f[VFS_COOR], c->inflow_plane, c->f[VFS_CSI], c->f[VFS_ETA], c->f[VFS_ZET],
-                       c->f[VFS_NVERT], c->f[VFS_UCONT], c->f[VFS_UCAT], c->red);
-    hipLaunchKernelGGL(finish_reduce<OpSum>, dim3(1), dim3(RED_THREADS), 0, st, c->red, RED_BLOCKS, sums);
-    double *result = sums;
-    if (held && inlet_flux > 0) {
-        hipLaunchKernelGGL(k_inflow, dim3(RED_BLOCKS), dim3(RED_THREADS), 0, st, g, 2, profile, plane, inlet_flux, inlet_flux,
-                           (const double *)sums, c->f[VFS_COOR], c->inflow_plane, c->f[VFS_CSI], c->f[VFS_ETA],
-                           c->f[VFS_ZET], c->f[VFS_NVERT], c->f[VFS_UCONT], c->f[VFS_UCAT], c->red);
-        hipLaunchKernelGGL(finish_reduce<OpSum>, dim3(1), dim3(RED_THREADS), 0, st, c->red, RED_BLOCKS, sums + 2);
-        result = sums + 2;
-    }
+    const bool hold = held && inlet_flux > 0;
+    auto pass = [&](int mode, double flux0, double *out, const RedSync &rs) {
+        hipLaunchKernelGGL(k_inflow, dim3(reduce_blocks((long long)(g.mx - 2) * (g.my - 2))), dim3(RED_THREADS), 0, st, g, mode,
+                           profile, plane, inlet_flux, flux0, (const double *)sums, c->f[VFS_COOR], c->inflow_plane, c->f[VFS_CSI],
+                           c->f[VFS_ETA], c->f[VFS_ZET], c->f[VFS_NVERT], c->f[VFS_UCONT], c->f[VFS_UCAT], c->red, out, rs);
+    };
+    pass(0, 0.0, sums + 1, red_quiet(c));
+    pass(1, 0.0, sums, hold ? red_quiet(c) : red_sync(c));
+    if (hold) pass(2, inlet_flux, sums + 2, red_sync(c));
     ucat_stale(c);
     VFS_LAUNCH_CHECK("inflow flux");
-    VFS_HIP(hipMemcpyAsync(c->red_host, result, sizeof(double), hipMemcpyDeviceToHost, st));
-    VFS_HIP(hipStreamSynchronize(st));
+    const int rc = red_wait(c);
+    if (rc) return rc;
     c->p.flux_in_sum = c->red_host[0];  // FluxInSum, read by the outlet balance of FormBCS
     if (flux_in) *flux_in = c->red_host[0];
     return VFS_OK;
@@ -886,6 +936,7 @@ static int form_bcs_open(vfs_ctx *c)
     const double *m_axis[3] = {c->f[VFS_CSI], c->f[VFS_ETA], c->f[VFS_ZET]};
     bool far = false, changed = false;
     for (int f = 0; f < 6; f++) far = far || g.bc[f] == 6;
+    if (!far && g.bc[5] != 8) return VFS_OK;
     VFS_HIP(hipMemsetAsync(scal, 0, 9 * sizeof(double), st));
     if (far) {
         for (int f = 0; f < 6; f++) {
@@ -966,11 +1017,9 @@ int form_bcs(vfs_ctx *c, int outflow_scale, bool lazy_ucat)
     rc = form_bcs_open(c);  // bcs.c:1745-2041
     if (rc) return rc;
     if (g.bc[5] == 4 && !g.pk) {
-        hipLaunchKernelGGL(k_outlet_sums, dim3(RED_BLOCKS), dim3(RED_THREADS), 0, st, g, c->f[VFS_UCONT],
-                           c->f[VFS_ZET], c->f[VFS_NVERT], c->red);
-        hipLaunchKernelGGL(finish_reduce<OpSum>, dim3(1), dim3(RED_THREADS), 0, st, c->red, RED_BLOCKS, c->red + 2 * RED_BLOCKS);
-        hipLaunchKernelGGL(finish_reduce<OpSum>, dim3(1), dim3(RED_THREADS), 0, st, c->red + RED_BLOCKS, RED_BLOCKS,
-                           c->red + 2 * RED_BLOCKS + 1);
+        if (outflow_scale)  // (nothing else reads the sums)
+            hipLaunchKernelGGL(k_outlet_sums, dim3(reduce_blocks((long long)(g.mx - 2) * (g.my - 2))), dim3(RED_THREADS), 0, st, g,
+                               c->f[VFS_UCONT], c->f[VFS_ZET], c->f[VFS_NVERT], c->red, c->red + 2 * RED_BLOCKS, red_quiet(c));
         VFS_LAUNCH_CHECK("outlet sums");
         if (outflow_scale) {
             long long n = (long long)(g.mx - 2) * (g.my - 2);
@@ -1062,6 +1111,7 @@ __global__ void k_eddy(Grid g, double cs2, const double *__restrict__ csf, const
 // get nu_t = 0 from k_zero_ghosts.
 // NB: no point is blanked (every nvert 0): the blanking tests fold away;
 // CSF: lCs is the per-point array csf (dynamic model), else the scalar cs2
+// A value is also stored at the periodic ghosts that copy its point.
 template <bool NB, bool CSF>
 __global__ void __launch_bounds__(KM_I * KM_J) k_eddy_km(Grid g, int kc, double cs2, const double *__restrict__ csf,
                                                         const double *__restrict__ ucat,
@@ -1082,7 +1132,7 @@ __global__ void __launch_bounds__(KM_I * KM_J) k_eddy_km(Grid g, int kc, double 
         for (int c = 0; c < 3; c++) up[c] = ucat[3 * (q + P) + c];
         const double nvp = NVR(q + P);
         if (nv0 > 1.1) {
-            nut[q] = 0;
+            store_periodic(g, nut, k, j, i, 0.0);
         } else {
             const double nve = NVR(q + 1), nvw = NVR(q - 1), nvn = NVR(q + g.mx), nvs = NVR(q - g.mx);
             double dd[3][3];
@@ -1100,7 +1150,7 @@ __global__ void __launch_bounds__(KM_I * KM_J) k_eddy_km(Grid g, int kc, double 
                 else if (nvm > SOL || (!g.pk && k == 0)) dd[c][2] = (up[c] - u0[c]);
                 else dd[c][2] = (up[c] - um[c]) * 0.5;
             }
-            nut[q] = smagorinsky(CSF ? csf[q] : cs2, dd, csi + 3 * q, eta + 3 * q, zet + 3 * q, aj[q]);
+            store_periodic(g, nut, k, j, i, smagorinsky(CSF ? csf[q] : cs2, dd, csi + 3 * q, eta + 3 * q, zet + 3 * q, aj[q]));
         }
         for (int c = 0; c < 3; c++) { um[c] = u0[c]; u0[c] = up[c]; }
         nvm = nv0;
@@ -1167,7 +1217,7 @@ int eddy_viscosity(vfs_ctx *c)
     }
     prof_end(c);
     VFS_LAUNCH_CHECK("eddy viscosity");
-    return periodic_fix(c, c->f[VFS_NU_T], 1, 0);
+    return e && e[0] == '0' ? periodic_fix(c, c->f[VFS_NU_T], 1, 0) : VFS_OK;
 }
 
 // ---------------------------------------------------------------------------
@@ -1178,8 +1228,9 @@ int eddy_viscosity(vfs_ctx *c)
 // |1/(ucont.c * aj)| over interior cells (Calc_Minimum_dt, momentum.c:157-161)
 __global__ void k_interior_reduce(Grid g, int mode, const double *__restrict__ ucont, const double *__restrict__ zet,
                                   const double *__restrict__ aj, const double *__restrict__ nvert,
-                                  double *__restrict__ part)
+                                  double *part, double *out, RedSync rs)
 {
+    __shared__ double res[1];
     const long long ni = (long long)(g.mx - 2) * (g.my - 2) * (g.mz - 2);
     double v = mode == 2 ? 1.e7 : 0.0;
     for (long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x; t < ni; t += (long long)gridDim.x * blockDim.x) {
@@ -1196,21 +1247,38 @@ __global__ void k_interior_reduce(Grid g, int mode, const double *__restrict__ u
         }
     }
     v = mode == 2 ? block_reduce<OpMin>(v) : block_reduce<OpSum>(v);
-    if (threadIdx.x == 0) part[blockIdx.x] = v;
+    if (threadIdx.x == 0) red_put(part + blockIdx.x, v);
+    if (!red_last(rs, gridDim.x)) return;
+    if (mode == 2) red_finish_rows<OpMin>(rs, 1, gridDim.x, part, out, res);
+    else red_finish_rows<OpSum>(rs, 1, gridDim.x, part, out, res);
+}
+
+static int interior_reduce_start(vfs_ctx *c, int mode, int at = 0)
+{
+    const Grid &g = c->g;
+    hipLaunchKernelGGL(k_interior_reduce, dim3(reduce_blocks((long long)(g.mx - 2) * (g.my - 2) * (g.mz - 2))), dim3(RED_THREADS), 0,
+                       c->stream, g, mode, c->f[VFS_UCONT], c->f[VFS_ZET], c->f[VFS_AJ], c->f[VFS_NVERT], c->red,
+                       c->red + RED_BLOCKS, red_sync(c, at));
+    VFS_LAUNCH_CHECK("interior reduce");
+    return VFS_OK;
 }
 
 static int interior_reduce(vfs_ctx *c, int mode, double *out)
 {
-    hipStream_t st = c->stream;
-    hipLaunchKernelGGL(k_interior_reduce, dim3(RED_BLOCKS), dim3(RED_THREADS), 0, st, c->g, mode, c->f[VFS_UCONT],
-                       c->f[VFS_ZET], c->f[VFS_AJ], c->f[VFS_NVERT], c->red);
-    if (mode == 2) hipLaunchKernelGGL(finish_reduce<OpMin>, dim3(1), dim3(RED_THREADS), 0, st, c->red, RED_BLOCKS, c->red + RED_BLOCKS);
-    else hipLaunchKernelGGL(finish_reduce<OpSum>, dim3(1), dim3(RED_THREADS), 0, st, c->red, RED_BLOCKS, c->red + RED_BLOCKS);
-    VFS_LAUNCH_CHECK("interior reduce");
-    VFS_HIP(hipMemcpyAsync(c->red_host, c->red + RED_BLOCKS, sizeof(double), hipMemcpyDeviceToHost, st));
-    VFS_HIP(hipStreamSynchronize(st));
-    *out = c->red_host[0];
-    return VFS_OK;
+    int rc = interior_reduce_start(c, mode);
+    if (!rc) rc = red_wait(c);
+    if (!rc) *out = c->red_host[0];
+    return rc;
+}
+
+// Calc_k_Flux in two halves, so that other work can be enqueued between them
+constexpr int KFLUX_AT = 256;  // (no other result goes there)
+int calc_k_flux_start(vfs_ctx *c) { return interior_reduce_start(c, 0, KFLUX_AT); }
+int calc_k_flux_finish(vfs_ctx *c, double *out)
+{
+    const int rc = red_wait(c);
+    if (!rc) *out = c->red_host[KFLUX_AT] / (c->g.mz - 2);
+    return rc;
 }
 
 int calc_k_flux(vfs_ctx *c, double *out)

@@ -203,17 +203,10 @@ constexpr int KRYLOV_MAXV = 33;                    // basis vectors plus one
 constexpr int KRYLOV_R = KRYLOV_MAXV * RED_BLOCKS; // results in the reduction scratch, after the partials
 constexpr int KRYLOV_H2 = KRYLOV_R + KRYLOV_MAXV + 1;
 
-// blocks of a Gram-Schmidt sweep: no more than have elements
-inline unsigned krylov_blocks(long long n)
-{
-    const long long b = (n + RED_THREADS - 1) / RED_THREADS;
-    return (unsigned)(b < RED_BLOCKS ? b : RED_BLOCKS);
-}
-
 // <w, V_v> (v < nv) and <w, w> into scratch[KRYLOV_R ..]; rs tells the host
 inline void launch_multidot(hipStream_t st, long long n, int nv, const double *V, const double *w, double *scratch, const RedSync &rs)
 {
-    const dim3 gb(krylov_blocks(n)), tb(RED_THREADS);
+    const dim3 gb(reduce_blocks(n)), tb(RED_THREADS);
     auto k = nv <= 4 ? k_multidot<4, 4> : nv <= 8 ? k_multidot<8, 4> : nv <= 16 ? k_multidot<16, 2> : k_multidot<KRYLOV_MAXV - 1, 1>;
     hipLaunchKernelGGL(k, gb, tb, 0, st, n, nv, V, n, w, scratch, scratch + KRYLOV_R, rs);
 }
@@ -230,7 +223,7 @@ inline void launch_gram_schmidt(hipStream_t st, long long n, int nv, const doubl
     RedSync quiet = rs;
     quiet.host = nullptr;
     launch_multidot(st, n, nv, V, w, scratch, quiet);
-    const dim3 gb(krylov_blocks(n)), tb(RED_THREADS);
+    const dim3 gb(reduce_blocks(n)), tb(RED_THREADS);
     double *h = scratch + KRYLOV_R, *h2 = scratch + KRYLOV_H2;
     auto a = nv <= 4 ? k_multiaxpy<4, 4> : nv <= 8 ? k_multiaxpy<8, 4> : nv <= 16 ? k_multiaxpy<16, 2> : k_multiaxpy<KRYLOV_MAXV - 1, 1>;
     hipLaunchKernelGGL(a, gb, tb, 0, st, n, nv, (const double *)h, V, n, w, scratch, h2, rs);

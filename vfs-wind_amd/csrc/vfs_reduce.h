@@ -13,6 +13,13 @@ namespace vfs {
 constexpr int RED_THREADS = 256;
 constexpr int RED_BLOCKS = 1024;  // partials per reduction (fits ctx->red)
 
+// blocks of a reduction over n elements: no more than have one each thread
+inline unsigned reduce_blocks(long long n)
+{
+    const long long b = (n + RED_THREADS - 1) / RED_THREADS;
+    return (unsigned)(b < 1 ? 1 : b < RED_BLOCKS ? b : RED_BLOCKS);
+}
+
 struct OpSum {
     __device__ static double init() { return 0.0; }
     __device__ static double op(double a, double b) { return a + b; }
