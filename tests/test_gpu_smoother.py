@@ -216,3 +216,19 @@ def test_deep_level_sweeps(monkeypatch):
         assert not np.array_equal(out[0][1], out[1][1])
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("ny", [4, 8, 9, 15, 17, 57])
+def test_short_segments_padding_bitwise(monkeypatch, ny):
+    """The one-pass form loads every point of a segment without a test and pads
+    short segments: against the two-pass form, at line lengths of one segment,
+    of full segments and of segments short by up to seven points, on a grid
+    whose lines do not fill the last block."""
+    out = []
+    for fused in ("1", "0"):
+        monkeypatch.setenv("VFS_ZEBRA_FUSED", fused)
+        st, phi, res = _solve(monkeypatch, {"VFS_SMOOTH_COMPACT": "1", "VFS_MG_TAIL": "0"}, (18, ny, 14))
+        assert res <= 1.01e-8
+        out.append((st.iterations, phi))
+    assert out[0][0] == out[1][0]
+    assert np.array_equal(out[0][1], out[1][1])

@@ -829,8 +829,8 @@ __global__ void __launch_bounds__(1024) k_zebra_line_c4(Grid g, ZGrid z, int c, 
     const long long sstride = 2 * z.cplane;
     const long long base = (long long)kk * z.njI * z.nh + h;  // + jj * nh
     const long long cb = c * z.cplane + base;
-    const float *lo = sf + cb, *mm = sf + sstride + cb, *cp = sf + 2 * sstride + cb;
     const long long nh = z.nh;
+    if (!act) i = 1;
     const int I[3] = {canon(i - 1, g.mx, g.pi), i, canon(i + 1, g.mx, g.pi)};
     const int K[3] = {canon(k - 1, g.mz, g.pk), k, canon(k + 1, g.mz, g.pk)};
     // SPL: b and x in the S layout.  The neighbours are of the other colour
@@ -840,41 +840,91 @@ __global__ void __launch_bounds__(1024) k_zebra_line_c4(Grid g, ZGrid z, int c, 
     const int q = 1 - c;
     const bool okw = I[0] >= 1 && I[0] <= g.mx - 2, oke = I[2] >= 1 && I[2] <= g.mx - 2;
     const bool okb = K[0] >= 1 && K[0] <= g.mz - 2, okt = K[2] >= 1 && K[2] <= g.mz - 2;
-    const long long hw = okw ? (I[0] - zebra_i0(k, q)) >> 1 : 0, he = oke ? (I[2] - zebra_i0(k, q)) >> 1 : 0;
+    const long long hw = okw && act ? (I[0] - zebra_i0(k, q)) >> 1 : 0, he = oke && act ? (I[2] - zebra_i0(k, q)) >> 1 : 0;
     const long long rowq = q * z.cplane, nrow = (long long)z.njI * z.nh;
     const long long sw = rowq + kk * nrow + hw, se = rowq + kk * nrow + he;
     const long long sbt = rowq + (okb ? K[0] - 1 : 0) * nrow + h, stp = rowq + (okt ? K[2] - 1 : 0) * nrow + h;
+    // Segments of up to 8 points load everything first and unconditionally (a
+    // point past the segment's end reads the segment's first, a neighbour past
+    // the grid's edge some other point's value), so that all loads are in flight
+    // together; the 16-point form would hold more than its registers and loads
+    // point by point.  A padded point hands its carry on unchanged (factors
+    // -1, 1, -1 and right-hand side 0), which keeps the recurrences free of
+    // tests.  Waiting for one point's loads after another's took 6.9 us per
+    // half-sweep at 64x48x64 and 6.5 on the 48x32x40 level of a 96x64x80 grid,
+    // together 4.8 and 4.2; at 160x96x192 both 12 (4.4 TB/s).
+    const int np = act ? j1 - j0 : 0;
+    const float *lo = sf + cb, *mm = sf + sstride + cb, *cp = sf + 2 * sstride + cb;
     float r[SLM], l[SLM], m[SLM], u[SLM];
+    if constexpr (SLM <= 8) {
+        h4_t w[SLM];
+        float dd[SLM], xe[SLM], xw[SLM], xt[SLM], xb[SLM];
 #pragma unroll
-    for (int v = 0; v < SLM; v++) {
-        const int jj = j0 + v;
-        if (act && jj < j1) {
-            const long long o = jj * nh;
-            const float bq = SPL ? b[cb + o] : b[((long long)k * g.my + jj + 1) * g.mx + i];
-            // XZ: the iterate is zero on entry (the first half-sweep of a
-            // V-cycle level): the same sum over zero neighbours, without reading them
-            if constexpr (XZ)
-                r[v] = c4_sum(sh[cb + o], sd[cb + o], 0.f, 0.f, 0.f, 0.f, bq);
-            else if constexpr (SPL)
-                r[v] = c4_sum(sh[cb + o], sd[cb + o], oke ? x[se + o] : 0.f, okw ? x[sw + o] : 0.f, okt ? x[stp + o] : 0.f,
-                              okb ? x[sbt + o] : 0.f, bq);
-            else
-                r[v] = c4_rhs(g, I, K, jj + 1, sh[cb + o], sd[cb + o], x, bq);
+        for (int v = 0; v < SLM; v++) {
+            const int jj = np > 0 ? j0 + (v < np ? v : 0) : 0;
+            const long long o = jj * nh, row0 = (long long)(jj + 1) * g.mx;
+            w[v] = sh[cb + o];
+            dd[v] = sd[cb + o];
+            r[v] = SPL ? b[cb + o] : b[(long long)k * g.plane + row0 + i];
+            // XZ: the iterate is zero on entry (the first half-sweep of a V-cycle
+            // level): the same sum over zero neighbours, without reading them
+            if constexpr (XZ) {
+                xe[v] = xw[v] = xt[v] = xb[v] = 0.f;
+            } else if constexpr (SPL) {
+                xe[v] = x[se + o];
+                xw[v] = x[sw + o];
+                xt[v] = x[stp + o];
+                xb[v] = x[sbt + o];
+            } else {
+                xe[v] = x[(long long)K[1] * g.plane + row0 + I[2]];
+                xw[v] = x[(long long)K[1] * g.plane + row0 + I[0]];
+                xt[v] = x[(long long)K[2] * g.plane + row0 + I[1]];
+                xb[v] = x[(long long)K[0] * g.plane + row0 + I[1]];
+            }
             l[v] = lo[o];
             m[v] = mm[o];
             u[v] = cp[o];
-        } else {
-            r[v] = 0; l[v] = 0; m[v] = 0; u[v] = 0;
+        }
+#pragma unroll
+        for (int v = 0; v < SLM; v++) {
+            const float rv = c4_sum(w[v], dd[v], SPL && !oke ? 0.f : xe[v], SPL && !okw ? 0.f : xw[v], SPL && !okt ? 0.f : xt[v],
+                                    SPL && !okb ? 0.f : xb[v], r[v]);
+            r[v] = v < np ? rv : 0.f;
+            if (v >= np) {
+                l[v] = u[v] = -1.f;
+                m[v] = 1.f;
+            }
+        }
+    } else {
+#pragma unroll
+        for (int v = 0; v < SLM; v++) {
+            r[v] = 0.f;
+            l[v] = u[v] = -1.f;
+            m[v] = 1.f;
+            if (v < np) {
+                const int jj = j0 + v;
+                const long long o = jj * nh;
+                const float bq = SPL ? b[cb + o] : b[((long long)k * g.my + jj + 1) * g.mx + i];
+                if constexpr (XZ)
+                    r[v] = c4_sum(sh[cb + o], sd[cb + o], 0.f, 0.f, 0.f, 0.f, bq);
+                else if constexpr (SPL)
+                    r[v] = c4_sum(sh[cb + o], sd[cb + o], oke ? x[se + o] : 0.f, okw ? x[sw + o] : 0.f, okt ? x[stp + o] : 0.f,
+                                  okb ? x[sbt + o] : 0.f, bq);
+                else
+                    r[v] = c4_rhs(g, I, K, jj + 1, sh[cb + o], sd[cb + o], x, bq);
+                l[v] = lo[o];
+                m[v] = mm[o];
+                u[v] = cp[o];
+            }
         }
     }
     // forward map of the segment: d_out = A d_in + B
     float A = 1, B = 0;
 #pragma unroll
-    for (int v = 0; v < SLM; v++)
-        if (j0 + v < j1) {
-            B = (r[v] - l[v] * B) * m[v];
-            A = (-l[v] * A) * m[v];
-        }
+    for (int v = 0; v < SLM; v++) {
+        B = (r[v] - l[v] * B) * m[v];
+        A = (-l[v] * A) * m[v];
+    }
     const int me = seg * LL + ln;
     sA[me] = A;
     sB[me] = B;
@@ -882,35 +932,31 @@ __global__ void __launch_bounds__(1024) k_zebra_line_c4(Grid g, ZGrid z, int c, 
     float d = 0;
     for (int s = 0; s < seg; s++) d = sA[s * LL + ln] * d + sB[s * LL + ln];
 #pragma unroll
-    for (int v = 0; v < SLM; v++)
-        if (j0 + v < j1) {
-            d = (r[v] - l[v] * d) * m[v];
-            r[v] = d;
-        }
+    for (int v = 0; v < SLM; v++) {
+        d = (r[v] - l[v] * d) * m[v];
+        r[v] = v < np ? d : 0.f;
+    }
     __syncthreads();
     // backward map of the segment: x_first = A x_above + B
     A = 1;
     B = 0;
 #pragma unroll
-    for (int v = SLM - 1; v >= 0; v--)
-        if (j0 + v < j1) {
-            B = r[v] - u[v] * B;
-            A = -u[v] * A;
-        }
+    for (int v = SLM - 1; v >= 0; v--) {
+        B = r[v] - u[v] * B;
+        A = -u[v] * A;
+    }
     sA[me] = A;
     sB[me] = B;
     __syncthreads();
     float xl = 0;
     for (int s = nseg - 1; s > seg; s--) xl = sA[s * LL + ln] * xl + sB[s * LL + ln];
-    if (act) {
 #pragma unroll
-        for (int v = SLM - 1; v >= 0; v--) {
+    for (int v = SLM - 1; v >= 0; v--) {
+        xl = r[v] - u[v] * xl;
+        if (v < np) {
             const int jj = j0 + v;
-            if (jj < j1) {
-                xl = r[v] - u[v] * xl;
-                if (SPL) x[cb + jj * nh] = xl;
-                else x[((long long)k * g.my + jj + 1) * g.mx + i] = xl;
-            }
+            if (SPL) x[cb + jj * nh] = xl;
+            else x[(long long)k * g.plane + (long long)(jj + 1) * g.mx + i] = xl;
         }
     }
 }
@@ -2226,10 +2272,9 @@ static LinePlan line_plan(const PLevel &L)
     // on the finest level the one-pass kernel takes 16-point segments and 64
     // lines per block up to 256-point lines (a segment row is a whole
     // wavefront; the coarse levels, which fill fewer blocks, keep 8 and 32)
-    // where that leaves two blocks per CU: 52 against 54 us per half-sweep at
+    // where that leaves two blocks per CU: 48 against 57 us per half-sweep at
     // 256x192x256, but with fewer lines the shorter, more numerous blocks of
-    // the coarse levels are faster (11 against 8 us at 64x48x64; whole solves
-    // 2.73 -> 2.48 ms there, 10.2 -> 9.7 ms at 192x144x192)
+    // the coarse levels are faster (11 against 5 us at 64x48x64)
     if (fusable && L.finest && L.z.njI <= line_slm<float>() * 16 && (long long)L.z.nkI * L.z.nh >= 64 * 512) p.short_seg = false;
     if (force == 1) p.short_seg = sizeof(T) == 4;
     if (force == 2) p.short_seg = false;
