@@ -197,3 +197,43 @@ def test_turbine_angvel_against_oracle(mode):
         st[2] = -alm.loads()[7]  # Torque_aero = -M_Sum
     alm.close()
     ctx.close()
+
+
+@pytest.mark.parametrize("nodes_per_blade,cells,radius,off", [
+    (2, (12, 9, 14), 3.0, 0.0),       # one element per blade, boxes clipped on every side
+    (41, (22, 37, 70), 9.0, 6.5),     # blades that leave the box: clipped and empty boxes, a ragged union box
+    (300, (30, 28, 26), 7.0, 0.0),    # more elements than one list of a brick holds
+], ids=["one-element", "leaving", "897-elements"])
+def test_alm_bricks_and_searches(nodes_per_blade, cells, radius, off):
+    """The nearest-node search, the sampled velocity, the polar search and the
+    spreading at their edges, on the oracle's chain of the same stages."""
+    vfs = importlib.import_module("vfs-wind_amd")
+    cases = importlib.import_module("vfs-wind_amd.cases")
+    nx, ny, nz = cells
+    b = cases.box(nx, ny, nz, h=1.0, bump=0.3)
+    per, bc = (0, 0, 0), (10, 10, 10, 10, 5, 4)
+    hub = (nx / 2 + 0.13 + off, ny / 2 - 0.21, nz / 2 + 0.37)
+    ts = cases.synthetic_turbine(radius, hub, nodes_per_blade=nodes_per_blade)
+    o = po.Oracle(po.make_params(*b["da"], per=per, bctype=bc, les=0), b["coor"])
+    o.set("ucat", b["ucat"])
+    t = po.make_turbine(ts.nx, ts.ny, ts.nz, ts.xc, ts.yc, ts.zc, ts.angvel, ts.pitch, ts.r_nacelle, ts.refangle)
+    with vfs.Context(vfs.make_params(*b["da"], per=per, bctype=bc, les=0)) as ctx:
+        ctx.upload("COOR", b["coor"])
+        ctx.form_metrics()
+        ctx.upload("UCAT", b["ucat"])
+        alm = vfs.ALM(ctx, ts.turbine_struct(vfs), ts.nodes, ts.foils)
+        try:
+            alm.step(0.03)
+            box, rbox = o.alm_preprocess(alm.get("CENT")), o.alm_preprocess(alm.get("REF_CENT"))
+            assert np.array_equal(alm.get("BOX").astype(np.int32), box)
+            assert np.array_equal(alm.get("REF_BOX").astype(np.int32), rbox)
+            ul = alm.get("U_LAGR")
+            assert relerr(ul, o.alm_ulagr(alm.get("REF_CENT"), rbox)) <= TOL
+            f, aoa, cl, cd = po.alm_flagr(t, *ts.nodes.shape[:2], alm.get("CENT"), ul, alm.get("NODE_VEL"), alm.get("TWIST"),
+                                          alm.get("CHORD"), po.Foils(ts.foils))
+            assert relerr(alm.get("CL"), cl) <= TOL and relerr(alm.get("F_LAGR"), f) <= TOL
+            want = o.alm_feul(alm.get("CENT"), box, alm.get("F_LAGR"), alm.get("DA"), df=7, halfwidth=2.0)
+            assert np.abs(want).max() > 0
+            assert relerr(ctx.download("FEUL"), want) <= TOL
+        finally:
+            alm.close()

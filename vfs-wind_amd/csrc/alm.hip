@@ -5,16 +5,17 @@
 // lengths, twist/chord by radius) touch a few hundred numbers and run on the
 // host in FP64; everything that reads or writes the Eulerian grid runs on the
 // device:
-//   k_alm_nearest   Pre_process      nearest grid node along the first
-//                                    interior grid lines, +-6 cell box
+//   k_alm_nearest   Pre_process      one wavefront per element and grid
+//                                    direction: nearest grid node along the
+//                                    first interior grid lines, +-6 cell box
 //   k_alm_ulagr     Calc_U_lagr      one block per element, dfunc_s3h-weighted
 //                                    sum of ucat over its box (tree reduction)
-//   k_alm_flagr     Calc_F_lagr_ACL  one thread per element
-//   k_alm_feul      Calc_F_eul       one thread per cell of the union of the
-//                                    element boxes, gathering every element
-//                                    whose box holds the cell in element
-//                                    order, so each cell sums its terms in
-//                                    the reference's order; then the
+//   k_alm_flagr     Calc_F_lagr_ACL  one wavefront per element
+//   k_alm_feul      Calc_F_eul       one block per brick of 64 cells of the
+//                                    union of the element boxes, gathering
+//                                    every element whose box holds the cell in
+//                                    element order, so each cell sums its
+//                                    terms in the reference's order; then the
 //                                    blanking / boundary-layer zeroing.
 #include <hip/hip_runtime.h>
 
@@ -96,24 +97,46 @@ struct GridMet {
 
 __device__ inline double CO(const GridMet &m, int c, int k, int j, int i) { return m.coor[3 * gidx(m.g, k, j, i) + c]; }
 
-// Pre_process, rotor_model.c:1880-1995 (one rank)
-__global__ void k_alm_nearest(GridMet m, int n, const double *__restrict__ cent, int *__restrict__ box)
+// Pre_process, rotor_model.c:1880-1995 (one rank).  A block per element, a
+// wavefront per grid direction, a lane per 64th node of its line: one thread
+// per element walked up to mx + my + mz nodes, one load after another, 66 us
+// at 96x64x80 and 222 us at 384x192x256 for 120 elements; now 7 and 10 us for
+// twice as many, the reference line's (model 6) following in the same launch.
+// The first of equally near nodes is taken, as by a scan in order.
+constexpr int ALM_NEAREST_TPB = 192;
+__global__ void __launch_bounds__(ALM_NEAREST_TPB) k_alm_nearest(GridMet m, int n1, const double *__restrict__ cent1,
+                                                                 int *__restrict__ box1, const double *__restrict__ cent2,
+                                                                 int *__restrict__ box2)
 {
-    const int l = blockIdx.x * blockDim.x + threadIdx.x;
-    if (l >= n) return;
+    const bool second = (int)blockIdx.x >= n1;
+    const int l = second ? blockIdx.x - n1 : blockIdx.x;
+    const double *cent = second ? cent2 : cent1;
+    int *box = second ? box2 : box1;
     const Grid &g = m.g;
     const int lo[3] = {1, 1, 1}, hi[3] = {g.mx - 1, g.my - 1, g.mz - 1};
     const double cx = cent[3 * l], cy = cent[3 * l + 1], cz = cent[3 * l + 2];
-    int cc[3] = {0, 0, 0};
-    for (int d = 0; d < 3; d++) {
+    __shared__ int near_[3];
+    {
+        const int d = threadIdx.x / 64, lane = threadIdx.x % 64;
+        const int end = d == 0 ? hi[0] : d == 1 ? hi[1] : hi[2];
         double dmin = 1.e6;
-        for (int s = lo[d]; s < hi[d]; s++) {
+        int at = 0;
+        for (int s = 1 + lane; s < end; s += 64) {
             const int i = d == 0 ? s : lo[0] + 1, j = d == 1 ? s : lo[1] + 1, k = d == 2 ? s : lo[2] + 1;
             const double r1 = cx - CO(m, 0, k, j, i), r2 = cy - CO(m, 1, k, j, i), r3 = cz - CO(m, 2, k, j, i);
             const double d1 = sqrt(r1 * r1 + r2 * r2 + r3 * r3);
-            if (d1 < dmin) { dmin = d1; cc[d] = s; }
+            if (d1 < dmin) { dmin = d1; at = s; }
         }
+        for (int o = 32; o > 0; o >>= 1) {  // a lane without a node in reach has at = 0 and dmin = 1e6
+            const double od = __shfl_xor(dmin, o, 64);
+            const int oa = __shfl_xor(at, o, 64);
+            if (oa && (!at || od < dmin || (od == dmin && oa < at))) { dmin = od; at = oa; }
+        }
+        if (lane == 0) near_[d] = at;
     }
+    __syncthreads();
+    if (threadIdx.x) return;
+    int cc[3] = {near_[0], near_[1], near_[2]};
     const double r1 = cx - CO(m, 0, cc[2], cc[1], cc[0]), r2 = cy - CO(m, 1, cc[2], cc[1], cc[0]),
                  r3 = cz - CO(m, 2, cc[2], cc[1], cc[0]);
     const double dmin = sqrt(r1 * r1 + r2 * r2 + r3 * r3);
@@ -131,17 +154,24 @@ __global__ void k_alm_nearest(GridMet m, int n, const double *__restrict__ cent,
     }
 }
 
-// Calc_U_lagr, rotor_model.c:2977-3036: one block per element
-__global__ void __launch_bounds__(ALM_TPB) k_alm_ulagr(GridMet m, const double *__restrict__ ucat, int n,
-                                                       const double *__restrict__ cent, const int *__restrict__ box,
-                                                       double *__restrict__ ulagr)
+// Calc_U_lagr, rotor_model.c:2977-3036: one block per element.  A cell's
+// weight (three normals, three arcsines) is a long serial computation and there
+// are only as many blocks as elements, so the block is as large as it can be
+// and a thread has at most two of the box's up to 1728 cells; the terms meet
+// in LDS and are summed by ALM_TPB threads, each its cells in steps of
+// ALM_TPB, and a tree: 31 -> 24 us for 120 elements, bound by the divisions
+// of the metrics on the 120 CUs that have a block.
+constexpr int ALM_UTPB = 1024, ALM_UCELLS = 8 * ALM_BOX * ALM_BOX * ALM_BOX;
+__global__ void __launch_bounds__(ALM_UTPB) k_alm_ulagr(GridMet m, const double *__restrict__ ucat, int n,
+                                                        const double *__restrict__ cent, const int *__restrict__ box,
+                                                        double *__restrict__ ulagr)
 {
     const int l = blockIdx.x;
     if (l >= n) return;
     const int *b = box + 6 * l;
     const int ni = b[1] - b[0], nj = b[3] - b[2], nk = b[5] - b[4];
     const int cells = ni > 0 && nj > 0 && nk > 0 ? ni * nj * nk : 0;
-    double u[3] = {0, 0, 0};
+    __shared__ double term[3][ALM_UCELLS];
     for (int t = threadIdx.x; t < cells; t += blockDim.x) {
         const int i = b[0] + t % ni, j = b[2] + (t / ni) % nj, k = b[4] + t / (ni * nj);
         double xc[3];
@@ -158,10 +188,16 @@ __global__ void __launch_bounds__(ALM_TPB) k_alm_ulagr(GridMet m, const double *
         const double r2 = (rx * nn[1][0] + ry * nn[1][1] + rz * nn[1][2]) / hy;
         const double r3 = (rx * nn[2][0] + ry * nn[2][1] + rz * nn[2][2]) / hz;
         const double df = dfunc_s3h(r1) * dfunc_s3h(r2) * dfunc_s3h(r3);
-        for (int c = 0; c < 3; c++) u[c] += ucat[3 * q + c] * df;
+        for (int c = 0; c < 3; c++) term[c][t] = ucat[3 * q + c] * df;
     }
+    __syncthreads();
+    double u[3] = {0, 0, 0};
+    if (threadIdx.x < ALM_TPB)
+        for (int t = threadIdx.x; t < cells; t += ALM_TPB)
+            for (int c = 0; c < 3; c++) u[c] += term[c][t];
     __shared__ double red[3][ALM_TPB];
-    for (int c = 0; c < 3; c++) red[c][threadIdx.x] = u[c];
+    if (threadIdx.x < ALM_TPB)
+        for (int c = 0; c < 3; c++) red[c][threadIdx.x] = u[c];
     __syncthreads();
     for (int s = ALM_TPB / 2; s > 0; s >>= 1) {
         if ((int)threadIdx.x < s)
@@ -182,15 +218,19 @@ struct Polars {
 __device__ inline double polar(double aoa, int nq, const double *ang, const double *val, double lim, bool lift, double v)
 {
     const double pi = 3.141592653589793;
-    bool inrange = false;
-    for (int j = 0; j < nq - 1; j++)
-        if (aoa >= ang[j] && aoa <= ang[j + 1]) {
-            const double fac1 = (ang[j + 1] - aoa) / (ang[j + 1] - ang[j]);
-            const double fac2 = (-ang[j] + aoa) / (ang[j + 1] - ang[j]);
-            v = fac1 * val[j] + fac2 * val[j + 1];
-            inrange = true;
-        }
-    if (!inrange) {
+    // the last interval that holds aoa, 64 intervals at a time (the whole
+    // wavefront has the same aoa)
+    int at = -1;
+    for (int j0 = 0; j0 < nq - 1; j0 += 64) {
+        const int j = j0 + threadIdx.x % 64;
+        const unsigned long long hit = __ballot(j < nq - 1 && aoa >= ang[j] && aoa <= ang[j + 1]);
+        if (hit) at = j0 + 63 - __clzll(hit);
+    }
+    if (at >= 0) {
+        const double fac1 = (ang[at + 1] - aoa) / (ang[at + 1] - ang[at]);
+        const double fac2 = (-ang[at] + aoa) / (ang[at + 1] - ang[at]);
+        v = fac1 * val[at] + fac2 * val[at + 1];
+    } else {
         if (aoa < ang[0] && aoa > -45.0) v = (-lim - val[0]) * (aoa - ang[0]) / (-45.0 - ang[0]) + val[0];
         if (aoa <= -45.0 && aoa >= -90.0) v = lift ? lim * sin(2.0 * aoa * pi / 180.0) : -lim;
         if (aoa < -90.0) v = lift ? 0.0 : -lim;
@@ -241,15 +281,17 @@ __device__ inline double tip_loss(const TurbineDev &t, double r, double aoa, dou
 
 // Calc_F_lagr_ACL, rotor_model.c:2384-2597 (rotor_model 3/6): blade-element
 // forces with the selected tip-loss factor and 3D lift correction; the
-// nacelle zeroing here unless the force smoothing runs first
-__global__ void k_alm_flagr(TurbineDev t, Polars P, const double *__restrict__ cent, const double *__restrict__ ulagr,
+// nacelle zeroing here unless the force smoothing runs first.  A wavefront per
+// element: its lanes search the polar tables together (polar) and are
+// otherwise alike; one thread per element walked the tables entry by entry.
+// For 120 elements and tables of 181 entries 39 -> 10 us.
+__global__ void __launch_bounds__(64) k_alm_flagr(TurbineDev t, Polars P, const double *__restrict__ cent, const double *__restrict__ ulagr,
                             const double *__restrict__ unode, const double *__restrict__ twist,
                             const double *__restrict__ chord, double *__restrict__ aoa, double *__restrict__ cl,
                             double *__restrict__ cd, double *__restrict__ flagr)
 {
     const int ne = t.nvb - 1;
-    const int l = blockIdx.x * blockDim.x + threadIdx.x;
-    if (l >= t.nb * ne) return;
+    const int l = blockIdx.x;
     const double pi = 3.141592653589793;
     const int n1 = (l / ne) * t.nvb + l % ne, n2 = n1 + 1;
     const double rx = cent[3 * l] - t.xc, ry = cent[3 * l + 1] - t.yc, rz = cent[3 * l + 2] - t.zc;
@@ -270,7 +312,8 @@ __global__ void k_alm_flagr(TurbineDev t, Polars P, const double *__restrict__ c
     double tmp = -nrel[0] * nrot[0] - nrel[1] * nrot[1] - nrel[2] * nrot[2];
     tmp /= (1 + 1e-9);
     const double a = acos(tmp) * 180.0 / pi - twist[l] - t.pitch;
-    aoa[l] = a;
+    const bool writer = threadIdx.x == 0;
+    if (writer) aoa[l] = a;
     double nL[3] = {nrel[1] * nbl[2] - nrel[2] * nbl[1], nrel[2] * nbl[0] - nrel[0] * nbl[2], nrel[0] * nbl[1] - nrel[1] * nbl[0]};
     tmp = t.nx * nL[0] + t.ny * nL[1] + t.nz * nL[2];
     if (tmp < 0.0) { nL[0] = -nL[0]; nL[1] = -nL[1]; nL[2] = -nL[2]; }
@@ -283,8 +326,8 @@ __global__ void k_alm_flagr(TurbineDev t, Polars P, const double *__restrict__ c
             vcl = polar(a, o[2], P.tab + o[3], P.tab + o[3] + o[2], 1.05, true, vcl);
         }
     }
-    cl[l] = vcl;
-    cd[l] = vcd;
+    if (writer) cl[l] = vcl;
+    if (writer) cd[l] = vcd;
     const double factor = chord[l];
     double F[3];
     for (int c = 0; c < 3; c++) F[c] = -0.5 * uref * uref * fabs(vcd) * nrel[c] * factor;
@@ -300,6 +343,7 @@ __global__ void k_alm_flagr(TurbineDev t, Polars P, const double *__restrict__ c
         F[2] += Fc * t.nz;
     }
     const double rn = sqrt(rx * rx + ry * ry + rz * rz);
+    if (!writer) return;
     for (int c = 0; c < 3; c++) flagr[3 * l + c] = t.nacelle_here && rn < t.r_nacelle ? 0.0 : F[c];
 }
 
@@ -329,54 +373,96 @@ __global__ void k_alm_nacelle(TurbineDev t, const double *__restrict__ cent, dou
     if (sqrt(rx * rx + ry * ry + rz * rz) < t.r_nacelle) flagr[3 * l] = flagr[3 * l + 1] = flagr[3 * l + 2] = 0.0;
 }
 
-// Calc_F_eul, rotor_model.c:3738-3830, gathered per cell over the union box
-__global__ void k_alm_feul(GridMet m, int n, const double *__restrict__ cent, const int *__restrict__ box,
-                           const double *__restrict__ flagr, const double *__restrict__ dA, int df, double hw, int ui0,
-                           int uj0, int uk0, int uni, int unj, int unk, double *__restrict__ feul)
+// Calc_F_eul, rotor_model.c:3738-3830, gathered per cell over the union box.
+// A term is some 800 FP64 instructions (nine distances, nine kernels) and a
+// cell near the hub has a term of nearly every element, while the union box is
+// only some hundred wavefronts of cells; with one thread per cell the chip was
+// idle but for their serial chains.  So a block takes a brick of 64 cells:
+// the elements whose boxes meet the brick are listed in order, FEUL_WAVES of
+// them at a time are taken by one wavefront each (lane = cell), and the terms
+// meet in LDS, where one wavefront per component adds them to the cells' sums in
+// element order: the sums of a serial loop (a missing term adds a zero to a sum
+// that is never -0).  120 elements: 282 -> 60 us at a radius of 12 cells,
+// 255 -> 59 at 32; the bricks at the hub take the longest.
+constexpr int FEUL_WAVES = 8, FEUL_LIST = 64 * FEUL_WAVES;
+constexpr int FEUL_BI = 8, FEUL_BJ = 4, FEUL_BK = 2;  // brick; 12-cell boxes meet 2.1 bricks' worth of cells per cell
+__global__ void __launch_bounds__(FEUL_LIST) k_alm_feul(GridMet m, int n, const double *__restrict__ cent,
+                                                        const int *__restrict__ box, const double *__restrict__ flagr,
+                                                        const double *__restrict__ dA, int df, double hw, int ui0, int uj0,
+                                                        int uk0, int uni, int unj, int unk, double *__restrict__ feul)
 {
-    const long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-    if (t >= (long long)uni * unj * unk) return;
-    const int i = ui0 + t % uni, j = uj0 + (t / uni) % unj, k = uk0 + t / ((long long)uni * unj);
-    const long long q = gidx(m.g, k, j, i);
+    __shared__ int list[FEUL_LIST], count[FEUL_WAVES];
+    __shared__ double term[FEUL_WAVES][3][64];
+    const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
+    const int nbi = (uni + FEUL_BI - 1) / FEUL_BI, nbj = (unj + FEUL_BJ - 1) / FEUL_BJ;
+    const int i0 = ui0 + (int)(blockIdx.x % nbi) * FEUL_BI, j0 = uj0 + (int)(blockIdx.x / nbi % nbj) * FEUL_BJ,
+              k0 = uk0 + (int)(blockIdx.x / (nbi * nbj)) * FEUL_BK;
+    const int i = i0 + lane % FEUL_BI, j = j0 + lane / FEUL_BI % FEUL_BJ, k = k0 + lane / (FEUL_BI * FEUL_BJ);
+    const bool in = i < ui0 + uni && j < uj0 + unj && k < uk0 + unk;
+    const long long q = in ? gidx(m.g, k, j, i) : gidx(m.g, k0, j0, i0);
     bool geo = false;
-    double ri0[3], rj0[3], rk0[3], nn[3][3], hx = 0, hy = 0, hz = 0, vol = 0;
-    double acc[3] = {feul[3 * q], feul[3 * q + 1], feul[3 * q + 2]};
-    for (int l = 0; l < n; l++) {
-        const int *b = box + 6 * l;
-        if (i < b[0] || i >= b[1] || j < b[2] || j >= b[3] || k < b[4] || k >= b[5]) continue;
-        if (!geo) {
-            for (int c = 0; c < 3; c++) {
-                ri0[c] = (CO(m, c, k, j, i) + CO(m, c, k - 1, j, i) + CO(m, c, k, j - 1, i) + CO(m, c, k - 1, j - 1, i)) * 0.25;
-                rj0[c] = (CO(m, c, k, j, i) + CO(m, c, k - 1, j, i) + CO(m, c, k, j, i - 1) + CO(m, c, k - 1, j, i - 1)) * 0.25;
-                rk0[c] = (CO(m, c, k, j, i) + CO(m, c, k, j - 1, i) + CO(m, c, k, j, i - 1) + CO(m, c, k, j - 1, i - 1)) * 0.25;
+    double ri0[3], rj0[3], rk0[3], nn[3][3], h[3] = {0, 0, 0}, vol = 0;
+    double acc = wave < 3 ? feul[3 * q + wave] : 0.0;
+    for (int l0 = 0; l0 < n; l0 += FEUL_LIST) {
+        const int le = l0 + (int)threadIdx.x;
+        const int *b = box + 6 * (le < n ? le : n - 1);
+        const bool meets = le < n && b[0] < i0 + FEUL_BI && b[1] > i0 && b[2] < j0 + FEUL_BJ && b[3] > j0 &&
+                           b[4] < k0 + FEUL_BK && b[5] > k0;
+        const unsigned long long hit = __ballot(meets);
+        if (lane == 0) count[wave] = __popcll(hit);
+        __syncthreads();
+        int at = __popcll(hit & ((1ull << lane) - 1)), total = 0;
+        for (int w = 0; w < FEUL_WAVES; w++) {
+            if (w < wave) at += count[w];
+            total += count[w];
+        }
+        if (meets) list[at] = le;
+        __syncthreads();
+        for (int e0 = 0; e0 < total; e0 += FEUL_WAVES) {
+            if (e0 + wave < total) {
+                const int l = list[e0 + wave];
+                const int *bl = box + 6 * l;
+                double t[3] = {0, 0, 0};
+                if (in && i >= bl[0] && i < bl[1] && j >= bl[2] && j < bl[3] && k >= bl[4] && k < bl[5]) {
+                    if (!geo) {
+                        for (int c = 0; c < 3; c++) {
+                            ri0[c] = (CO(m, c, k, j, i) + CO(m, c, k - 1, j, i) + CO(m, c, k, j - 1, i) + CO(m, c, k - 1, j - 1, i)) * 0.25;
+                            rj0[c] = (CO(m, c, k, j, i) + CO(m, c, k - 1, j, i) + CO(m, c, k, j, i - 1) + CO(m, c, k - 1, j, i - 1)) * 0.25;
+                            rk0[c] = (CO(m, c, k, j, i) + CO(m, c, k, j - 1, i) + CO(m, c, k, j, i - 1) + CO(m, c, k, j - 1, i - 1)) * 0.25;
+                        }
+                        cell_normals(m.csi, m.eta, m.zet, q, nn);
+                        cell_spacing(m.csi, m.eta, m.zet, m.aj, q, h[0], h[1], h[2]);
+                        vol = 1.0 / (h[0] * h[1] * h[2]);
+                        geo = true;
+                    }
+                    const double *ce = cent + 3 * l;
+                    const double *fc[3] = {ri0, rj0, rk0};
+                    double dfun[3];
+#pragma unroll
+                    for (int f = 0; f < 3; f++) {
+                        const double rr[3] = {fc[f][0] - ce[0], fc[f][1] - ce[1], fc[f][2] - ce[2]};
+                        double r[3];
+                        for (int d = 0; d < 3; d++) r[d] = fabs(rr[0] * nn[d][0] + rr[1] * nn[d][1] + rr[2] * nn[d][2]) / h[d];
+                        if (df == 0) dfun[f] = vol * dfunc_2h(r[0]) * dfunc_2h(r[1]) * dfunc_2h(r[2]);
+                        else if (df == 7) dfun[f] = vol * dfunc_exp(r[0], hw) * dfunc_exp(r[1], hw) * dfunc_exp(r[2], hw);
+                        else dfun[f] = vol * dfunc_s4h(r[0]) * dfunc_s4h(r[1]) * dfunc_s4h(r[2]);
+                    }
+                    const double Fx = flagr[3 * l], Fy = flagr[3 * l + 1], Fz = flagr[3 * l + 2], a = dA[l];
+                    const double *mt[3] = {m.csi + 3 * q, m.eta + 3 * q, m.zet + 3 * q};
+                    for (int f = 0; f < 3; f++)
+                        t[f] = Fx * dfun[f] * a * mt[f][0] + Fy * dfun[f] * a * mt[f][1] + Fz * dfun[f] * a * mt[f][2];
+                }
+                for (int f = 0; f < 3; f++) term[wave][f][lane] = t[f];
             }
-            cell_normals(m.csi, m.eta, m.zet, q, nn);
-            cell_spacing(m.csi, m.eta, m.zet, m.aj, q, hx, hy, hz);
-            vol = 1.0 / (hx * hy * hz);
-            geo = true;
+            __syncthreads();
+            if (wave < 3) {
+                const int ew = total - e0 < FEUL_WAVES ? total - e0 : FEUL_WAVES;
+                for (int w = 0; w < ew; w++) acc += term[w][wave][lane];
+            }
+            __syncthreads();
         }
-        const double *ce = cent + 3 * l;
-        const double ri[3] = {ri0[0] - ce[0], ri0[1] - ce[1], ri0[2] - ce[2]};
-        const double rj[3] = {rj0[0] - ce[0], rj0[1] - ce[1], rj0[2] - ce[2]};
-        const double rk[3] = {rk0[0] - ce[0], rk0[1] - ce[1], rk0[2] - ce[2]};
-        double r[3][3];  // [face][direction]
-        const double *rr[3] = {ri, rj, rk};
-        const double h[3] = {hx, hy, hz};
-        for (int f = 0; f < 3; f++)
-            for (int d = 0; d < 3; d++)
-                r[f][d] = fabs(rr[f][0] * nn[d][0] + rr[f][1] * nn[d][1] + rr[f][2] * nn[d][2]) / h[d];
-        double dfun[3];
-        for (int f = 0; f < 3; f++) {
-            if (df == 0) dfun[f] = vol * dfunc_2h(r[f][0]) * dfunc_2h(r[f][1]) * dfunc_2h(r[f][2]);
-            else if (df == 7) dfun[f] = vol * dfunc_exp(r[f][0], hw) * dfunc_exp(r[f][1], hw) * dfunc_exp(r[f][2], hw);
-            else dfun[f] = vol * dfunc_s4h(r[f][0]) * dfunc_s4h(r[f][1]) * dfunc_s4h(r[f][2]);
-        }
-        const double Fx = flagr[3 * l], Fy = flagr[3 * l + 1], Fz = flagr[3 * l + 2], a = dA[l];
-        const double *mt[3] = {m.csi + 3 * q, m.eta + 3 * q, m.zet + 3 * q};
-        for (int f = 0; f < 3; f++)
-            acc[f] += Fx * dfun[f] * a * mt[f][0] + Fy * dfun[f] * a * mt[f][1] + Fz * dfun[f] * a * mt[f][2];
     }
-    for (int c = 0; c < 3; c++) feul[3 * q + c] = acc[c];
+    if (wave < 3 && in) feul[3 * q + wave] = acc;
 }
 
 // zeroing after the spread, rotor_model.c:3836-3929, over the union box
@@ -668,9 +754,9 @@ int vfs_alm_preprocess(vfs_alm *a)
     vfs_ctx *c = a->ctx;
     const int ne = a->nb * a->ne;
     GridMet m = gridmet(c);
-    hipLaunchKernelGGL(k_alm_nearest, dim3(blocks_for(ne, 64)), dim3(64), 0, c->stream, m, ne, a->d_cent, a->d_box);
-    if (a->t.rotor_model == 6)
-        hipLaunchKernelGGL(k_alm_nearest, dim3(blocks_for(ne, 64)), dim3(64), 0, c->stream, m, ne, a->d_refcent, a->d_refbox);
+    const int sets = a->t.rotor_model == 6 ? 2 : 1;
+    hipLaunchKernelGGL(k_alm_nearest, dim3(sets * ne), dim3(ALM_NEAREST_TPB), 0, c->stream, m, ne, a->d_cent, a->d_box,
+                       a->d_refcent, a->d_refbox);
     VFS_LAUNCH_CHECK("alm nearest");
     a->box_host.resize(6 * ne);
     VFS_HIP(hipMemcpyAsync(a->box_host.data(), a->d_box, 6 * ne * sizeof(int), hipMemcpyDeviceToHost, c->stream));
@@ -684,7 +770,7 @@ int vfs_alm_u_lagr(vfs_alm *a)
     vfs_ctx *c = a->ctx;
     const int ne = a->nb * a->ne;
     const bool ref = a->t.rotor_model == 6;  // model 6 samples on the reference line (solvers.c:543-555)
-    hipLaunchKernelGGL(k_alm_ulagr, dim3(ne), dim3(ALM_TPB), 0, c->stream, gridmet(c), (const double *)c->f[VFS_UCAT], ne,
+    hipLaunchKernelGGL(k_alm_ulagr, dim3(ne), dim3(ALM_UTPB), 0, c->stream, gridmet(c), (const double *)c->f[VFS_UCAT], ne,
                        ref ? a->d_refcent : a->d_cent, ref ? a->d_refbox : a->d_box, a->d_ulagr);
     VFS_LAUNCH_CHECK("alm u_lagr");
     return VFS_OK;
@@ -701,7 +787,7 @@ int vfs_alm_f_lagr(vfs_alm *a)
                   T.correction3d_cl, T.num_blade, smooth ? 0 : 1, T.r_rotor, T.tsr, T.a_shen, T.b_shen, T.c_shen,
                   T.correction_shen1, T.c0_cl};
     Polars P{(int)a->foil_rbeg.size(), a->d_off, a->d_tab};
-    hipLaunchKernelGGL(k_alm_flagr, dim3(blocks_for(ne, 64)), dim3(64), 0, c->stream, td, P, a->d_cent, a->d_ulagr, a->d_unode,
+    hipLaunchKernelGGL(k_alm_flagr, dim3(ne), dim3(64), 0, c->stream, td, P, a->d_cent, a->d_ulagr, a->d_unode,
                        a->d_twist, a->d_chord, a->d_aoa, a->d_cl, a->d_cd, a->d_flagr);
     if (smooth) {
         // smoothforce_AL + 1 passes (the reference's do-while), then the nacelle zeroing
@@ -822,7 +908,8 @@ int vfs_alm_f_eul(vfs_alm *a)
     const int uni = hi[0] - lo[0], unj = hi[1] - lo[1], unk = hi[2] - lo[2];
     const long long cells = (long long)uni * unj * unk;
     GridMet m = gridmet(c);
-    hipLaunchKernelGGL(k_alm_feul, dim3(blocks_for(cells, ALM_TPB)), dim3(ALM_TPB), 0, c->stream, m, ne, a->d_cent, a->d_box,
+    const unsigned bricks = (unsigned)((uni + FEUL_BI - 1) / FEUL_BI) * ((unj + FEUL_BJ - 1) / FEUL_BJ) * ((unk + FEUL_BK - 1) / FEUL_BK);
+    hipLaunchKernelGGL(k_alm_feul, dim3(bricks), dim3(FEUL_LIST), 0, c->stream, m, ne, a->d_cent, a->d_box,
                        a->d_flagr, a->d_dA, a->t.deltafunc, a->t.halfwidth, lo[0], lo[1], lo[2], uni, unj, unk,
                        c->f[VFS_FEUL]);
     hipLaunchKernelGGL(k_alm_feul_zero, dim3(blocks_for(cells, ALM_TPB)), dim3(ALM_TPB), 0, c->stream, m, lo[0], lo[1], lo[2],
@@ -903,7 +990,8 @@ int vfs_alm_set_disk(vfs_alm *a, int n, const double *cent, const double *dA)
     VFS_HIP(hipMalloc((void **)&a->d_dbox, 6 * n * sizeof(int)));
     VFS_HIP(hipMemcpy(a->d_dcent, cent, 3 * n * 8, hipMemcpyHostToDevice));
     VFS_HIP(hipMemcpy(a->d_dA_disk, dA, n * 8, hipMemcpyHostToDevice));
-    hipLaunchKernelGGL(k_alm_nearest, dim3(blocks_for(n, 64)), dim3(64), 0, c->stream, gridmet(c), n, a->d_dcent, a->d_dbox);
+    hipLaunchKernelGGL(k_alm_nearest, dim3(n), dim3(ALM_NEAREST_TPB), 0, c->stream, gridmet(c), n, a->d_dcent, a->d_dbox,
+                       (const double *)nullptr, (int *)nullptr);
     VFS_LAUNCH_CHECK("alm disk nearest");
     VFS_HIP(hipStreamSynchronize(c->stream));
     return VFS_OK;
@@ -915,7 +1003,7 @@ int vfs_alm_uref(vfs_alm *a, double *uref)
     if (!a || !uref || a->n_disk < 1) return set_error(VFS_EINVAL, "vfs_alm_uref: no reference disk (vfs_alm_set_disk)");
     vfs_ctx *c = a->ctx;
     const int n = a->n_disk;
-    hipLaunchKernelGGL(k_alm_ulagr, dim3(n), dim3(ALM_TPB), 0, c->stream, gridmet(c), (const double *)c->f[VFS_UCAT], n,
+    hipLaunchKernelGGL(k_alm_ulagr, dim3(n), dim3(ALM_UTPB), 0, c->stream, gridmet(c), (const double *)c->f[VFS_UCAT], n,
                        a->d_dcent, a->d_dbox, a->d_ulagr_disk);
     VFS_LAUNCH_CHECK("alm disk u_lagr");
     std::vector<double> u(3 * n);
