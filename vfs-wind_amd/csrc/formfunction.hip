@@ -52,17 +52,18 @@ struct FaceArgs {
 // integers) is kept as float in LDS, which represents them exactly.
 constexpr int FT_I = 32, FT_J = 16;
 
-template <bool SO>
+template <bool SO, int FJ = FT_J>
 struct TileDims {
-    static constexpr int HI = FT_I + (SO ? 2 : 3), HJ = FT_J + (SO ? 2 : 3), HP = HI * HJ;
+    static constexpr int HI = FT_I + (SO ? 2 : 3), HJ = FJ + (SO ? 2 : 3), HP = HI * HJ;
 };
 
 // NB: no point of the grid is blanked (every nvert is 0), so NV is the
 // constant 0 and every blanking test folds away at compile time; the tests
 // then take the branches they take for nvert = 0, so the result is the same.
-template <bool SO, bool NB = false>
+template <bool SO_, bool NB_ = false, int FJ = FT_J>
 struct TileAcc {
-    using D = TileDims<SO>;
+    static constexpr bool SO = SO_, NB = NB_, ORDERED = false;
+    using D = TileDims<SO, FJ>;
     const FaceArgs *a;
     const double *ux, *uy, *uz, *nt;
     const float *nv;
@@ -97,30 +98,6 @@ struct TileAcc {
     }
 };
 
-// viscous face flux, momentum.c:682-696 and 863-902 (and the j/k twins)
-__device__ inline void visc_face(const double cs[3], const double et[3], const double ze[3], const double nrm[3],
-                                 double ajc, const double d[3][3], double nu, double nu_t, int les, int laplacian,
-                                 double out[3])
-{
-    double g11 = cs[0] * nrm[0] + cs[1] * nrm[1] + cs[2] * nrm[2];
-    double g21 = et[0] * nrm[0] + et[1] * nrm[1] + et[2] * nrm[2];
-    double g31 = ze[0] * nrm[0] + ze[1] * nrm[1] + ze[2] * nrm[2];
-    double r[3][3];
-    for (int c = 0; c < 3; c++)
-        for (int q = 0; q < 3; q++) r[c][q] = d[c][0] * cs[q] + d[c][1] * et[q] + d[c][2] * ze[q];
-    for (int c = 0; c < 3; c++) out[c] = 0;
-    if (les)
-        for (int c = 0; c < 3; c++)
-            out[c] = (g11 * d[c][0] + g21 * d[c][1] + g31 * d[c][2] + r[0][c] * nrm[0] + r[1][c] * nrm[1] +
-                      r[2][c] * nrm[2]) * ajc * (nu_t);
-    if (laplacian)
-        for (int c = 0; c < 3; c++)
-            for (int q = 0; q < 3; q++) r[c][q] = 0.;
-    for (int c = 0; c < 3; c++)
-        out[c] += (g11 * d[c][0] + g21 * d[c][1] + g31 * d[c][2] + r[0][c] * nrm[0] + r[1][c] * nrm[1] +
-                   r[2][c] * nrm[2]) * ajc * (nu);
-}
-
 // the 10 metric values (csi, eta, zet, aj) of point q of one family
 __device__ inline void load_metrics(const Metrics9 &m, long long q, double v[10])
 {
@@ -133,175 +110,231 @@ __device__ inline void load_metrics(const Metrics9 &m, long long q, double v[10]
     v[9] = m.aj[q];
 }
 
-// convective and viscous flux of the i face of point (i,j,k)
-// (momentum.c:668-928): i in [0,mx-2], j,k interior; zero elsewhere
-template <bool SO, bool NB = false>
-__device__ inline void flux_i(const FaceArgs &a, const TileAcc<SO, NB> &T, int i, int j, int k, const double *Mf, double ucf,
+// Loads of the point `off` of the plane whose first point is the uniform q0 go
+// by scalar base addresses and a 32-bit byte offset (a plane's 24 bytes a point
+// stay far below 4 GB).  lane_offset makes the offset a new value to the
+// compiler, which would else keep a pointer for each array across the planes.
+__device__ inline unsigned lane_offset(unsigned byte)
+{
+    asm volatile("" : "+v"(byte));
+    return byte;
+}
+__device__ inline double at_byte(const double *base, unsigned byte)
+{
+    return *reinterpret_cast<const double *>(reinterpret_cast<const char *>(base) + byte);
+}
+__device__ inline void load_metrics(const Metrics9 &m, long long q0, unsigned off, double v[10])
+{
+    const unsigned b3 = lane_offset(24 * off);
+    const double *c = m.csi + 3 * q0, *e = m.eta + 3 * q0, *z = m.zet + 3 * q0;
+    v[0] = at_byte(c, b3); v[1] = at_byte(c + 1, b3); v[2] = at_byte(c + 2, b3);
+    v[3] = at_byte(e, b3); v[4] = at_byte(e + 1, b3); v[5] = at_byte(e + 2, b3);
+    v[6] = at_byte(z, b3); v[7] = at_byte(z + 1, b3); v[8] = at_byte(z + 2, b3);
+    v[9] = at_byte(m.aj + q0, lane_offset(8 * off));
+}
+
+// The metrics of the face between two cells as the face functions take them:
+// twice the mean area vectors and a quarter of the mean Jacobian
+// (rhs2.c:595-647).  The viscous flux is quadratic in the vectors and linear in
+// the Jacobian, so the powers of two cancel and a face's flux has the bits it
+// has with the stored means (face_mean) themselves; a[9] and b[9] are the
+// reciprocal Jacobians, which a cell's faces share.
+__device__ inline void face_sum(const double a[10], const double b[10], double f[10])
+{
+#pragma unroll
+    for (int c = 0; c < 9; c++) f[c] = a[c] + b[c];
+    f[9] = 0.5 / (a[9] + b[9]);
+}
+
+// Viscous face flux, momentum.c:682-696 and 863-902 (and the j/k twins), of
+// the face whose normal is area vector F of M (csi, eta, zet): component c is
+// (g_m du_c/dm + (du_q/dm M_mc) n_q) ajc (nu + nu_t), summed over m and q, with
+// g_m = M_m . n.  d[c][m] is du_c along direction m without the factor s[m] of
+// its difference.  The second sum is taken as M_mc (du_q/dm n_q), which needs
+// 18 products instead of 36, and the products accumulate in fused
+// multiply-adds: 45 FP64 instructions where the sums term by term, rounded
+// product by product, were 143.  Each sum still has its nine triple products.
+template <int F>
+__device__ inline void visc_face(const double M[10], const double d[3][3], const double s[3], double nu, double nu_t, int les,
+                                 int laplacian, double out[3])
+{
+    const double *n = M + 3 * F;
+    double gm[3], w[3];
+#pragma unroll
+    for (int m = 0; m < 3; m++) {
+        gm[m] = __builtin_fma(M[3 * m + 2], n[2], __builtin_fma(M[3 * m + 1], n[1], M[3 * m] * n[0]));
+        w[m] = __builtin_fma(d[2][m], n[2], __builtin_fma(d[1][m], n[1], d[0][m] * n[0]));
+        if (m != F) {  // (the difference across the face itself has no factor)
+            gm[m] *= s[m];
+            w[m] *= s[m];
+        }
+    }
+    double V[3], S[3];
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+        V[c] = __builtin_fma(gm[2], d[c][2], __builtin_fma(gm[1], d[c][1], gm[0] * d[c][0]));
+        S[c] = __builtin_fma(M[6 + c], w[2], __builtin_fma(M[3 + c], w[1], __builtin_fma(M[c], w[0], V[c])));
+    }
+    if (laplacian) {  // the molecular part keeps the first sum only
+        const double at = les ? M[9] * nu_t : 0.0, an = M[9] * nu;
+#pragma unroll
+        for (int c = 0; c < 3; c++) out[c] = __builtin_fma(S[c], at, V[c] * an);
+    } else {
+        const double at = M[9] * (les ? nu_t + nu : nu);
+#pragma unroll
+        for (int c = 0; c < 3; c++) out[c] = S[c] * at;
+    }
+}
+
+// convective and viscous flux of the i face of point (i,j,k) (momentum.c:668-928),
+// i in [0,mx-2] and the other two indices interior
+template <class Tile>
+__device__ inline void face_i(const FaceArgs &a, const Tile &T, int i, int j, int k, const double *M, double uc,
                               double dv[3], double vs[3])
 {
     const Grid &g = a.g;
-    const int mx = g.mx, my = g.my, mz = g.mz;
     const double SOL = 0.1;  // k-omega.c:19
-    (void)SOL; (void)my; (void)mz;
-    for (int c = 0; c < 3; c++) dv[c] = vs[c] = 0;
-    if (i < mx - 1 && j >= 1 && j < my - 1 && k >= 1 && k < mz - 1) {
-        const double cs[3] = {Mf[0], Mf[1], Mf[2]};
-        const double et[3] = {Mf[3], Mf[4], Mf[5]};
-        const double ze[3] = {Mf[6], Mf[7], Mf[8]};
-        double d[3][3];
-        // Compute_du_i, k-omega.c:56-116
-        for (int c = 0; c < 3; c++) {
-            d[c][0] = T.U(c, k, j, i + 1) - T.U(c, k, j, i);
-            if (T.NV(k, j + 1, i) > SOL || T.NV(k, j + 1, i + 1) > SOL)
-                d[c][1] = (T.U(c, k, j, i + 1) + T.U(c, k, j, i) - T.U(c, k, j - 1, i + 1) - T.U(c, k, j - 1, i)) * 0.5;
-            else if (T.NV(k, j - 1, i) > SOL || T.NV(k, j - 1, i + 1) > SOL)
-                d[c][1] = (T.U(c, k, j + 1, i + 1) + T.U(c, k, j + 1, i) - T.U(c, k, j, i + 1) - T.U(c, k, j, i)) * 0.5;
-            else
-                d[c][1] = (T.U(c, k, j + 1, i + 1) + T.U(c, k, j + 1, i) - T.U(c, k, j - 1, i + 1) - T.U(c, k, j - 1, i)) * 0.25;
-            if (T.NV(k + 1, j, i) > SOL || T.NV(k + 1, j, i + 1) > SOL)
-                d[c][2] = (T.U(c, k, j, i + 1) + T.U(c, k, j, i) - T.U(c, k - 1, j, i + 1) - T.U(c, k - 1, j, i)) * 0.5;
-            else if (T.NV(k - 1, j, i) > SOL || T.NV(k - 1, j, i + 1) > SOL)
-                d[c][2] = (T.U(c, k + 1, j, i + 1) + T.U(c, k + 1, j, i) - T.U(c, k, j, i + 1) - T.U(c, k, j, i)) * 0.5;
-            else
-                d[c][2] = (T.U(c, k + 1, j, i + 1) + T.U(c, k + 1, j, i) - T.U(c, k - 1, j, i + 1) - T.U(c, k - 1, j, i)) * 0.25;
-        }
+    // Compute_du_i, k-omega.c:56-116: one-sided next to a blanked cell
+    int jp = j + 1, jm = j - 1;
+    int kp = k + 1, km = k - 1;
+    double s[3] = {1.0, 0.25, 0.25};
+    if (T.NV(k, j + 1, i) > SOL || T.NV(k, j + 1, i + 1) > SOL) jp = j, s[1] = 0.5;
+    else if (T.NV(k, j - 1, i) > SOL || T.NV(k, j - 1, i + 1) > SOL) jm = j, s[1] = 0.5;
+    if (T.NV(k + 1, j, i) > SOL || T.NV(k + 1, j, i + 1) > SOL) kp = k, s[2] = 0.5;
+    else if (T.NV(k - 1, j, i) > SOL || T.NV(k - 1, j, i + 1) > SOL) km = k, s[2] = 0.5;
+    double d[3][3];
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+        const double u0 = T.U(c, k, j, i), u1 = T.U(c, k, j, i + 1);
+        d[c][0] = u1 - u0;
+        d[c][1] = T.U(c, k, jp, i + 1) + T.U(c, k, jp, i) - T.U(c, k, jm, i + 1) - T.U(c, k, jm, i);
+        d[c][2] = T.U(c, kp, j, i + 1) + T.U(c, kp, j, i) - T.U(c, km, j, i + 1) - T.U(c, km, j, i);
+        if (Tile::SO) dv[c] = -uc * 0.5 * (u0 + u1);
+        if (Tile::ORDERED) { asm volatile("" ::: "memory"); __builtin_amdgcn_sched_barrier(0); }
+    }
+    if (!Tile::SO) {
         int iL = i - 1, iR = i + 2;
-        if (i == 0 || i == mx - 2) {
-            if (g.pi && i == mx - 2) iR = mx + 2;
+        if (i == 0 || i == g.mx - 2) {
+            if (g.pi && i == g.mx - 2) iR = g.mx + 2;
             else if (g.pi && i == 0) iL = -3;
             else iL = i, iR = i + 1;
         } else if (T.NV(k, j, iL) + T.NV(k, j, iR) > 0.1) iL = i, iR = i + 1;
-        if (SO) iL = i, iR = i + 1;
-        const double uc = ucf;
-        for (int c = 0; c < 3; c++) {
-            if (SO) dv[c] = -uc * 0.5 * (T.U(c, k, j, i) + T.U(c, k, j, i + 1));
-            else dv[c] = -uc * 0.0625 * (-T.U(c, k, j, iL) + 9. * T.U(c, k, j, i) + 9. * T.U(c, k, j, i + 1) - T.U(c, k, j, iR));
-        }
-        if (T.NV(k, j, i) + T.NV(k, j, i + 1) > 0.1) dv[0] = dv[1] = dv[2] = 0;
-        double nut = 0;
-        if (a.les) {
-            if ((i == 0 && !g.pi) || T.NV(k, j, i) > 0.1) nut = T.NT(k, j, i + 1);
-            else if ((i == mx - 2 && !g.pi) || T.NV(k, j, i + 1) > 0.1) nut = T.NT(k, j, i);
-            else nut = 0.5 * (T.NT(k, j, i) + T.NT(k, j, i + 1));
-        }
-        visc_face(cs, et, ze, cs, Mf[9], d, a.nu, nut, a.les, a.laplacian, vs);
+#pragma unroll
+        for (int c = 0; c < 3; c++)
+            dv[c] = -uc * 0.0625 * (-T.U(c, k, j, iL) + 9. * T.U(c, k, j, i) + 9. * T.U(c, k, j, i + 1) - T.U(c, k, j, iR));
     }
+    if (T.NV(k, j, i) + T.NV(k, j, i + 1) > 0.1) dv[0] = dv[1] = dv[2] = 0;
+    double nut = 0;
+    if (a.les) {
+        const double n0 = T.NT(k, j, i), n1 = T.NT(k, j, i + 1);
+        if ((i == 0 && !g.pi) || T.NV(k, j, i) > 0.1) nut = n1;
+        else if ((i == g.mx - 2 && !g.pi) || T.NV(k, j, i + 1) > 0.1) nut = n0;
+        else nut = 0.5 * (n0 + n1);
+    }
+    visc_face<0>(M, d, s, a.nu, nut, a.les, a.laplacian, vs);
 }
 
-// convective and viscous flux of the j face of point (i,j,k)
-// (momentum.c:930-1211): j in [0,my-2], i,k interior; zero elsewhere
-template <bool SO, bool NB = false>
-__device__ inline void flux_j(const FaceArgs &a, const TileAcc<SO, NB> &T, int i, int j, int k, const double *Mf, double ucf,
+// convective and viscous flux of the j face of point (i,j,k) (momentum.c:930-1211),
+// j in [0,my-2] and the other two indices interior
+template <class Tile>
+__device__ inline void face_j(const FaceArgs &a, const Tile &T, int i, int j, int k, const double *M, double uc,
                               double dv[3], double vs[3])
 {
     const Grid &g = a.g;
-    const int mx = g.mx, my = g.my, mz = g.mz;
     const double SOL = 0.1;  // k-omega.c:19
-    (void)SOL; (void)my; (void)mz;
-    for (int c = 0; c < 3; c++) dv[c] = vs[c] = 0;
-    if (i >= 1 && i < mx - 1 && j < my - 1 && k >= 1 && k < mz - 1) {
-        const double cs[3] = {Mf[0], Mf[1], Mf[2]};
-        const double et[3] = {Mf[3], Mf[4], Mf[5]};
-        const double ze[3] = {Mf[6], Mf[7], Mf[8]};
-        double d[3][3];
-        // Compute_du_j, k-omega.c:141-200
-        for (int c = 0; c < 3; c++) {
-            if (T.NV(k, j, i + 1) > SOL || T.NV(k, j + 1, i + 1) > SOL)
-                d[c][0] = (T.U(c, k, j + 1, i) + T.U(c, k, j, i) - T.U(c, k, j + 1, i - 1) - T.U(c, k, j, i - 1)) * 0.5;
-            else if (T.NV(k, j, i - 1) > SOL || T.NV(k, j + 1, i - 1) > SOL)
-                d[c][0] = (T.U(c, k, j + 1, i + 1) + T.U(c, k, j, i + 1) - T.U(c, k, j + 1, i) - T.U(c, k, j, i)) * 0.5;
-            else
-                d[c][0] = (T.U(c, k, j + 1, i + 1) + T.U(c, k, j, i + 1) - T.U(c, k, j + 1, i - 1) - T.U(c, k, j, i - 1)) * 0.25;
-            d[c][1] = T.U(c, k, j + 1, i) - T.U(c, k, j, i);
-            if (T.NV(k + 1, j, i) > SOL || T.NV(k + 1, j + 1, i) > SOL)
-                d[c][2] = (T.U(c, k, j + 1, i) + T.U(c, k, j, i) - T.U(c, k - 1, j + 1, i) - T.U(c, k - 1, j, i)) * 0.5;
-            else if (T.NV(k - 1, j, i) > SOL || T.NV(k - 1, j + 1, i) > SOL)
-                d[c][2] = (T.U(c, k + 1, j + 1, i) + T.U(c, k + 1, j, i) - T.U(c, k, j + 1, i) - T.U(c, k, j, i)) * 0.5;
-            else
-                d[c][2] = (T.U(c, k + 1, j + 1, i) + T.U(c, k + 1, j, i) - T.U(c, k - 1, j + 1, i) - T.U(c, k - 1, j, i)) * 0.25;
-        }
+    // Compute_du_j, k-omega.c:141-200: one-sided next to a blanked cell
+    int ip = i + 1, im = i - 1;
+    int kp = k + 1, km = k - 1;
+    double s[3] = {0.25, 1.0, 0.25};
+    if (T.NV(k, j, i + 1) > SOL || T.NV(k, j + 1, i + 1) > SOL) ip = i, s[0] = 0.5;
+    else if (T.NV(k, j, i - 1) > SOL || T.NV(k, j + 1, i - 1) > SOL) im = i, s[0] = 0.5;
+    if (T.NV(k + 1, j, i) > SOL || T.NV(k + 1, j + 1, i) > SOL) kp = k, s[2] = 0.5;
+    else if (T.NV(k - 1, j, i) > SOL || T.NV(k - 1, j + 1, i) > SOL) km = k, s[2] = 0.5;
+    double d[3][3];
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+        const double u0 = T.U(c, k, j, i), u1 = T.U(c, k, j + 1, i);
+        d[c][1] = u1 - u0;
+        d[c][0] = T.U(c, k, j + 1, ip) + T.U(c, k, j, ip) - T.U(c, k, j + 1, im) - T.U(c, k, j, im);
+        d[c][2] = T.U(c, kp, j + 1, i) + T.U(c, kp, j, i) - T.U(c, km, j + 1, i) - T.U(c, km, j, i);
+        if (Tile::SO) dv[c] = -uc * 0.5 * (u0 + u1);
+        if (Tile::ORDERED) { asm volatile("" ::: "memory"); __builtin_amdgcn_sched_barrier(0); }
+    }
+    if (!Tile::SO) {
         int jL = j - 1, jR = j + 2;
-        if (j == 0 || j == my - 2) {
-            if (g.pj && j == my - 2) jR = my + 2;
+        if (j == 0 || j == g.my - 2) {
+            if (g.pj && j == g.my - 2) jR = g.my + 2;
             else if (g.pj && j == 0) jL = -3;
             else jL = j, jR = j + 1;
         } else if (T.NV(k, jL, i) + T.NV(k, jR, i) > 0.1) jL = j, jR = j + 1;
-        if (SO) jL = j, jR = j + 1;
-        const double uc = ucf;
-        for (int c = 0; c < 3; c++) {
-            if (SO) dv[c] = -uc * 0.5 * (T.U(c, k, j, i) + T.U(c, k, j + 1, i));
-            else dv[c] = -uc * 0.0625 * (-T.U(c, k, jL, i) + 9. * T.U(c, k, j, i) + 9. * T.U(c, k, j + 1, i) - T.U(c, k, jR, i));
-        }
-        if (T.NV(k, j, i) + T.NV(k, j + 1, i) > 0.1) dv[0] = dv[1] = dv[2] = 0;
-        double nut = 0;
-        if (a.les) {
-            if ((j == 0 && !g.pj) || T.NV(k, j, i) > 0.1) nut = T.NT(k, j + 1, i);
-            else if ((j == my - 2 && !g.pj) || T.NV(k, j + 1, i) > 0.1) nut = T.NT(k, j, i);
-            else nut = 0.5 * (T.NT(k, j, i) + T.NT(k, j + 1, i));
-        }
-        visc_face(cs, et, ze, et, Mf[9], d, a.nu, nut, a.les, a.laplacian, vs);
+#pragma unroll
+        for (int c = 0; c < 3; c++)
+            dv[c] = -uc * 0.0625 * (-T.U(c, k, jL, i) + 9. * T.U(c, k, j, i) + 9. * T.U(c, k, j + 1, i) - T.U(c, k, jR, i));
     }
+    if (T.NV(k, j, i) + T.NV(k, j + 1, i) > 0.1) dv[0] = dv[1] = dv[2] = 0;
+    double nut = 0;
+    if (a.les) {
+        const double n0 = T.NT(k, j, i), n1 = T.NT(k, j + 1, i);
+        if ((j == 0 && !g.pj) || T.NV(k, j, i) > 0.1) nut = n1;
+        else if ((j == g.my - 2 && !g.pj) || T.NV(k, j + 1, i) > 0.1) nut = n0;
+        else nut = 0.5 * (n0 + n1);
+    }
+    visc_face<1>(M, d, s, a.nu, nut, a.les, a.laplacian, vs);
 }
 
-// convective and viscous flux of the k face of point (i,j,k)
-// (momentum.c:1212-1451): k in [0,mz-2], i,j interior; zero elsewhere
-template <bool SO, bool NB = false>
-__device__ inline void flux_k(const FaceArgs &a, const TileAcc<SO, NB> &T, int i, int j, int k, const double *Mf, double ucf,
+// convective and viscous flux of the k face of point (i,j,k) (momentum.c:1212-1451),
+// k in [0,mz-2] and the other two indices interior
+template <class Tile>
+__device__ inline void face_k(const FaceArgs &a, const Tile &T, int i, int j, int k, const double *M, double uc,
                               double dv[3], double vs[3])
 {
     const Grid &g = a.g;
-    const int mx = g.mx, my = g.my, mz = g.mz;
     const double SOL = 0.1;  // k-omega.c:19
-    (void)SOL; (void)my; (void)mz;
-    for (int c = 0; c < 3; c++) dv[c] = vs[c] = 0;
-    if (i >= 1 && i < mx - 1 && j >= 1 && j < my - 1 && k < mz - 1) {
-        const double cs[3] = {Mf[0], Mf[1], Mf[2]};
-        const double et[3] = {Mf[3], Mf[4], Mf[5]};
-        const double ze[3] = {Mf[6], Mf[7], Mf[8]};
-        double d[3][3];
-        // Compute_du_k, k-omega.c:227-288
-        for (int c = 0; c < 3; c++) {
-            if (T.NV(k, j, i + 1) > SOL || T.NV(k + 1, j, i + 1) > SOL)
-                d[c][0] = (T.U(c, k + 1, j, i) + T.U(c, k, j, i) - T.U(c, k + 1, j, i - 1) - T.U(c, k, j, i - 1)) * 0.5;
-            else if (T.NV(k, j, i - 1) > SOL || T.NV(k + 1, j, i - 1) > SOL)
-                d[c][0] = (T.U(c, k + 1, j, i + 1) + T.U(c, k, j, i + 1) - T.U(c, k + 1, j, i) - T.U(c, k, j, i)) * 0.5;
-            else
-                d[c][0] = (T.U(c, k + 1, j, i + 1) + T.U(c, k, j, i + 1) - T.U(c, k + 1, j, i - 1) - T.U(c, k, j, i - 1)) * 0.25;
-            if (T.NV(k, j + 1, i) > SOL || T.NV(k + 1, j + 1, i) > SOL)
-                d[c][1] = (T.U(c, k + 1, j, i) + T.U(c, k, j, i) - T.U(c, k + 1, j - 1, i) - T.U(c, k, j - 1, i)) * 0.5;
-            else if (T.NV(k, j - 1, i) > SOL || T.NV(k + 1, j - 1, i) > SOL)
-                d[c][1] = (T.U(c, k + 1, j + 1, i) + T.U(c, k, j + 1, i) - T.U(c, k + 1, j, i) - T.U(c, k, j, i)) * 0.5;
-            else
-                d[c][1] = (T.U(c, k + 1, j + 1, i) + T.U(c, k, j + 1, i) - T.U(c, k + 1, j - 1, i) - T.U(c, k, j - 1, i)) * 0.25;
-            d[c][2] = T.U(c, k + 1, j, i) - T.U(c, k, j, i);
-        }
+    // Compute_du_k, k-omega.c:227-288: one-sided next to a blanked cell
+    int ip = i + 1, im = i - 1;
+    int jp = j + 1, jm = j - 1;
+    double s[3] = {0.25, 0.25, 1.0};
+    if (T.NV(k, j, i + 1) > SOL || T.NV(k + 1, j, i + 1) > SOL) ip = i, s[0] = 0.5;
+    else if (T.NV(k, j, i - 1) > SOL || T.NV(k + 1, j, i - 1) > SOL) im = i, s[0] = 0.5;
+    if (T.NV(k, j + 1, i) > SOL || T.NV(k + 1, j + 1, i) > SOL) jp = j, s[1] = 0.5;
+    else if (T.NV(k, j - 1, i) > SOL || T.NV(k + 1, j - 1, i) > SOL) jm = j, s[1] = 0.5;
+    double d[3][3];
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+        const double u0 = T.U(c, k, j, i), u1 = T.U(c, k + 1, j, i);
+        d[c][2] = u1 - u0;
+        d[c][0] = T.U(c, k + 1, j, ip) + T.U(c, k, j, ip) - T.U(c, k + 1, j, im) - T.U(c, k, j, im);
+        d[c][1] = T.U(c, k + 1, jp, i) + T.U(c, k, jp, i) - T.U(c, k + 1, jm, i) - T.U(c, k, jm, i);
+        if (Tile::SO) dv[c] = -uc * 0.5 * (u0 + u1);
+        if (Tile::ORDERED) { asm volatile("" ::: "memory"); __builtin_amdgcn_sched_barrier(0); }
+    }
+    if (!Tile::SO) {
         int kL = k - 1, kR = k + 2;
-        if (k == 0 || k == mz - 2) {
-            if (g.pk && k == mz - 2) kR = mz + 2;
+        if (k == 0 || k == g.mz - 2) {
+            if (g.pk && k == g.mz - 2) kR = g.mz + 2;
             else if (g.pk && k == 0) kL = -3;
             else kL = k, kR = k + 1;
         } else if (T.NV(kL, j, i) + T.NV(kR, j, i) > 0.1) kL = k, kR = k + 1;
-        if (SO) kL = k, kR = k + 1;
-        const double uc = ucf;
-        for (int c = 0; c < 3; c++) {
-            if (SO) dv[c] = -uc * 0.5 * (T.U(c, k, j, i) + T.U(c, k + 1, j, i));
-            else dv[c] = -uc * 0.0625 * (-T.U(c, kL, j, i) + 9. * T.U(c, k, j, i) + 9. * T.U(c, k + 1, j, i) - T.U(c, kR, j, i));
-        }
-        if (T.NV(k, j, i) + T.NV(k + 1, j, i) > 0.1) dv[0] = dv[1] = dv[2] = 0;
-        double nut = 0;
-        if (a.les) {
-            if ((k == 0 && !g.pk) || T.NV(k, j, i) > 0.1) nut = T.NT(k + 1, j, i);
-            else if ((k == mz - 2 && !g.pk) || T.NV(k + 1, j, i) > 0.1) nut = T.NT(k, j, i);
-            else nut = 0.5 * (T.NT(k, j, i) + T.NT(k + 1, j, i));
-        }
-        visc_face(cs, et, ze, ze, Mf[9], d, a.nu, nut, a.les, a.laplacian, vs);
+#pragma unroll
+        for (int c = 0; c < 3; c++)
+            dv[c] = -uc * 0.0625 * (-T.U(c, kL, j, i) + 9. * T.U(c, k, j, i) + 9. * T.U(c, k + 1, j, i) - T.U(c, kR, j, i));
     }
+    if (T.NV(k, j, i) + T.NV(k + 1, j, i) > 0.1) dv[0] = dv[1] = dv[2] = 0;
+    double nut = 0;
+    if (a.les) {
+        const double n0 = T.NT(k, j, i), n1 = T.NT(k + 1, j, i);
+        if ((k == 0 && !g.pk) || T.NV(k, j, i) > 0.1) nut = n1;
+        else if ((k == g.mz - 2 && !g.pk) || T.NV(k + 1, j, i) > 0.1) nut = n0;
+        else nut = 0.5 * (n0 + n1);
+    }
+    visc_face<2>(M, d, s, a.nu, nut, a.les, a.laplacian, vs);
 }
 
 // the 18 face fluxes of point (i,j,k) (momentum.c:668-1451); SO selects the
 // second-order convection at compile time (a.second_order is then 1).  With
 // DER the face metrics are rebuilt from the cell metrics: `cur` holds the
-// point's own cell metrics and `nk` those of cell k+1.
+// point's own cell metrics and `nk` those of cell k+1 (both with the reciprocal
+// Jacobian).
 template <bool SO, bool DER>
 __device__ inline void face_point(const FaceArgs &a, const TileAcc<SO> &T, int i, int j, int k, const double *cur,
                                   const double *nk)
@@ -310,7 +343,6 @@ __device__ inline void face_point(const FaceArgs &a, const TileAcc<SO> &T, int i
     const long long q = ((long long)k * g.my + j) * g.mx + i;
     const long long n = g.n;
     const int mx = g.mx, my = g.my, mz = g.mz;
-    const double SOL = 0.1;  // k-omega.c:19
     // the point's three face-metric families and fluxes, loaded together up
     // front (q is a valid point for every face, used or not) so that the 33
     // HBM loads are in flight at once
@@ -323,21 +355,23 @@ __device__ inline void face_point(const FaceArgs &a, const TileAcc<SO> &T, int i
         double ni[10], nj[10];
         load_metrics(a.cell, i < mx - 1 ? q + 1 : q, ni);
         load_metrics(a.cell, j < my - 1 ? q + mx : q, nj);
-        face_mean(cur, ni, M[0]);
-        face_mean(cur, nj, M[1]);
-        face_mean(cur, nk, M[2]);
+        ni[9] = 1. / ni[9];
+        nj[9] = 1. / nj[9];
+        face_sum(cur, ni, M[0]);
+        face_sum(cur, nj, M[1]);
+        face_sum(cur, nk, M[2]);
     } else {
         load_metrics(a.fi, q, M[0]);
         load_metrics(a.fj, q, M[1]);
         load_metrics(a.fk, q, M[2]);
     }
-
-    double dv[3], vs[3];
-    flux_i<SO>(a, T, i, j, k, M[0], UC[0], dv, vs);
-    for (int c = 0; c < 3; c++) { a.out[(0 + c) * n + q] = dv[c]; a.out[(9 + c) * n + q] = vs[c]; }
-    flux_j<SO>(a, T, i, j, k, M[1], UC[1], dv, vs);
-    for (int c = 0; c < 3; c++) { a.out[(3 + c) * n + q] = dv[c]; a.out[(12 + c) * n + q] = vs[c]; }
-    flux_k<SO>(a, T, i, j, k, M[2], UC[2], dv, vs);
+    const bool ii = i >= 1 && i < mx - 1, jj = j >= 1 && j < my - 1, kk = k >= 1 && k < mz - 1;
+    double dv[3] = {0, 0, 0}, vs[3] = {0, 0, 0};
+    if (i < mx - 1 && jj && kk) face_i(a, T, i, j, k, M[0], UC[0], dv, vs);
+    for (int c = 0; c < 3; c++) { a.out[(0 + c) * n + q] = dv[c]; a.out[(9 + c) * n + q] = vs[c]; dv[c] = vs[c] = 0; }
+    if (ii && j < my - 1 && kk) face_j(a, T, i, j, k, M[1], UC[1], dv, vs);
+    for (int c = 0; c < 3; c++) { a.out[(3 + c) * n + q] = dv[c]; a.out[(12 + c) * n + q] = vs[c]; dv[c] = vs[c] = 0; }
+    if (ii && jj && k < mz - 1) face_k(a, T, i, j, k, M[2], UC[2], dv, vs);
     for (int c = 0; c < 3; c++) { a.out[(6 + c) * n + q] = dv[c]; a.out[(15 + c) * n + q] = vs[c]; }
 }
 
@@ -392,8 +426,12 @@ __global__ void __launch_bounds__(FT_I * FT_J) k_face_fluxes(FaceArgs a, int kc)
         if (i < g.mx && j < g.my) {
             if (DER) {
                 const long long q = ((long long)k * g.my + j) * g.mx + i;
-                if (!have) load_metrics(a.cell, q, cur);
+                if (!have) {
+                    load_metrics(a.cell, q, cur);
+                    cur[9] = 1. / cur[9];
+                }
                 load_metrics(a.cell, k < g.mz - 1 ? q + g.plane : q, nk);
+                nk[9] = 1. / nk[9];
             }
             TileAcc<SO> T{&a, sx, sy, sz, st, sn, i0, j0, k, slot0};
             face_point<SO, DER>(a, T, i, j, k, cur, nk);
@@ -410,7 +448,7 @@ __global__ void __launch_bounds__(FT_I * FT_J) k_face_fluxes(FaceArgs a, int kc)
 
 // The face pass fused with the flux divergence (momentum.c:1548-1678) for
 // second-order convection with the face metrics rebuilt from the cell
-// metrics.  A block owns an FT_I x FT_J column and marches in k as
+// metrics.  A block owns an FT_I x FP_J column and marches in k as
 // k_face_fluxes does; on each plane the i- and j-face fluxes of its points go
 // to LDS together with one extra column (the i face at i0-1) and one extra row
 // (the j face at j0-1), and the k-face flux of the plane below stays in
@@ -428,184 +466,251 @@ __global__ void __launch_bounds__(FT_I * FT_J) k_face_fluxes(FaceArgs a, int kc)
 // Contra2Cart, the eddy viscosity, Formfunction_2's own Ucont fix and
 // FormMetrics leave them) the faces at index 0 computed here are bitwise
 // those copies, so that fix is not applied.
-constexpr int FX_J = FT_J + 1;
-static_assert(FT_I == 32, "a row of the tile is half a wavefront (the i-face exchange shuffles within it)");
+// Eight rows of points a block: two blocks fit a CU's LDS and, at 208 registers
+// a lane, its register files, so one block's loads and barriers overlap with
+// the other's arithmetic.  What bounds it is the wait for those loads with two
+// wavefronts per SIMD (the VALU is busy for a third of the time).  With the
+// faces' FP64 work at 90 instead of 187 instructions each, no face behind a
+// test, constant LDS offsets and scalar base addresses (600 instructions a point
+// instead of 1000; before, one block of 16 rows per CU): 766 -> 638 us at
+// 256x192x256, 1184 -> 965 at 384x192x256, 39 -> 30 at 96x64x80, 24 -> 17 at
+// 64x48x64, 14 -> 9 at 16x12x16.  Sixteen rows: 640, 923, 34, 21, 11; three
+// blocks per CU (168 registers) spill and take twice as long, and so does any
+// load of the next plane into registers that spill for it.
+constexpr int FP_J = 8;
+constexpr int FP_T = FT_I * FP_J;
+constexpr int FP_WAVES = 2;  // wavefronts per SIMD, which is also blocks per CU
+static_assert(FT_I == 32, "a row of the tile is half a wavefront (the i-face exchange stays within it)");
 constexpr int HX_T0 = 64;  // first thread of the second wavefront
-static_assert(FT_I * FT_J >= HX_T0 + FT_J && FT_J * 2 <= 64, "halo lanes of the i faces");
+static_assert(FP_T >= HX_T0 + FP_J && FP_J <= 64, "halo lanes of the i faces");
 inline long long face_fp_tiles(const Grid &g)
 {
-    return (long long)((g.mx - 2 + FT_I - 1) / FT_I) * ((g.my - 2 + FT_J - 1) / FT_J);
+    return (long long)((g.mx - 2 + FT_I - 1) / FT_I) * ((g.my - 2 + FP_J - 1) / FP_J);
 }
-template <bool NB>
-__global__ void __launch_bounds__(FT_I * FT_J) __attribute__((amdgpu_waves_per_eu(2))) k_face_fp(FaceArgs a, int kc, double *__restrict__ fp)
+// the value of the lane before (0 in the wavefront's first lane)
+__device__ inline double lane_before(double v)
 {
-    using D = TileDims<true>;
-    __shared__ double sx[3 * D::HP], sy[3 * D::HP], sz[3 * D::HP], st[3 * D::HP];
-    __shared__ float sn[3 * D::HP];
-    __shared__ double fxj[6][FX_J][FT_I];  // j-face div xyz, visc xyz; row 0 = face j0-1
-    __shared__ double hx[6][FT_J];         // i-face div xyz, visc xyz at i0-1 of each row
+    const long long b = __double_as_longlong(v);
+    const unsigned l = (unsigned)__builtin_amdgcn_mov_dpp((int)b, 0x138, 0xf, 0xf, true);  // wave_shr:1
+    const unsigned h = (unsigned)__builtin_amdgcn_mov_dpp((int)(b >> 32), 0x138, 0xf, 0xf, true);
+    return __longlong_as_double((long long)((unsigned long long)h << 32 | l));
+}
+// TileAcc of k_face_fp, for the faces of one point: the tile's four quantities
+// are one array and b[] holds, for the planes k-1, k and k+1, the index of the
+// tile point at (j-1, i-1), so that every read is one of three registers and a
+// constant offset.
+template <bool NB_>
+struct PointTile {
+    static constexpr bool SO = true, NB = NB_, ORDERED = true;
+    using D = TileDims<true, FP_J>;
+    const double *u;
+    const float *nv;
+    int i, j, k, b1, dn, up;
+    __device__ inline int at(int kk, int jj, int ii) const
+    {
+        int p = b1;
+        if (kk != k) p += kk > k ? up : dn;
+        return p + (jj - j + 1) * D::HI + (ii - i + 1);
+    }
+    __device__ inline double U(int c, int kk, int jj, int ii) const { return u[c * 3 * D::HP + at(kk, jj, ii)]; }
+    __device__ inline double NT(int kk, int jj, int ii) const { return u[9 * D::HP + at(kk, jj, ii)]; }
+    __device__ inline double NV(int kk, int jj, int ii) const { return NB ? 0.0 : (double)nv[at(kk, jj, ii)]; }
+};
+// The faces of a point share most of the 19 points of the tile that they read:
+// reading them again for each face is cheap, while kept from one face to the
+// next they take 114 registers.
+__device__ inline void reread_tile() { asm volatile("" ::: "memory"); }
+template <bool NB>
+__global__ void __launch_bounds__(FP_T) __attribute__((amdgpu_waves_per_eu(FP_WAVES))) k_face_fp(FaceArgs a, int kc, double *__restrict__ fp)
+{
+    using D = TileDims<true, FP_J>;
+    // ucat and nu_t of the tile's planes first: their offsets fit the LDS instructions
+    __shared__ struct {
+        double u[4][3 * D::HP];
+        double fxj[6][FP_J + 1][FT_I];   // j-face div xyz, visc xyz; row 0 = face j0-1
+        double hx[6][FP_J];              // i-face div xyz, visc xyz at i0-1 of each row
+        float nv[NB ? 1 : 3 * D::HP];
+    } S;
+    auto &fxj = S.fxj;
+    auto &hx = S.hx;
     const Grid &g = a.g;
     // The tiles cover the interior points (1 .. m-2 on each axis; kc planes a
     // block): the faces at index 0 are the halo faces of the first tiles, and
     // the ghost points' projections are not written (zero at the non-periodic
-    // ghosts since allocation; the cell pass does not read the periodic ones).  Tiles are taken in XCD order, so the tiles that share a
-    // halo run on one XCD's L2.
-    const int nbi = (g.mx - 2 + FT_I - 1) / FT_I, nbj = (g.my - 2 + FT_J - 1) / FT_J;
+    // ghosts since allocation; the cell pass does not read the periodic ones).
+    // Tiles are taken in XCD order, so the tiles that share a halo run on one
+    // XCD's L2.  A lane beyond the last interior point computes that point's
+    // faces again and stores nothing, so no face is behind a test.
+    const int nbi = (g.mx - 2 + FT_I - 1) / FT_I, nbj = (g.my - 2 + FP_J - 1) / FP_J;
     int b = (int)xcd_block1();
     const int bi = b % nbi;
     b /= nbi;
     const int bj = b % nbj, bk = b / nbj;
-    const int i0 = 1 + bi * FT_I, j0 = 1 + bj * FT_J, k0 = 1 + bk * kc;
+    const int i0 = 1 + bi * FT_I, j0 = 1 + bj * FP_J, k0 = 1 + bk * kc;
     const int k1 = k0 + kc < g.mz - 1 ? k0 + kc : g.mz - 1;
     const int tx = threadIdx.x % FT_I, ty = threadIdx.x / FT_I;
-    const int i = i0 + tx, j = j0 + ty;
-    const bool inb = i < g.mx && j < g.my;
+    const bool inb = i0 + tx < g.mx - 1 && j0 + ty < g.my - 1;
+    const int i = i0 + tx < g.mx - 1 ? i0 + tx : g.mx - 2, j = j0 + ty < g.my - 1 ? j0 + ty : g.my - 2;
     const long long n = g.n;
     const bool les = a.les != 0;
     // A tile plane is fetched into registers one plane ahead and written to
     // LDS at the top of the next iteration, so the global loads of plane k+2
-    // are in flight while plane k is computed.  Each thread owns tile points
-    // tid and tid + FT_I*FT_J.
-    constexpr int TPP = (D::HP + FT_I * FT_J - 1) / (FT_I * FT_J);  // tile points per thread
+    // are in flight while plane k is computed.
+    // Each thread owns tile points tid and tid + FP_T of ucat, nu_t and nvert; a
+    // point the grid does not have (beyond the last tile) reads the plane's
+    // first: no face that is stored uses it.
+    constexpr int TPP = (D::HP + FP_T - 1) / FP_T;  // tile points per thread
     double rv[TPP][4];
     float rn[TPP];
-    auto fetch_plane = [&](int kk) {
-        const int wk = wrapi(kk, g.mz, g.pk);
+    unsigned tof[TPP];  // the tile point's offset in its plane
 #pragma unroll
-        for (int r = 0; r < TPP; r++) {
-            const int p = threadIdx.x + r * FT_I * FT_J;
-            rv[r][0] = rv[r][1] = rv[r][2] = rv[r][3] = 0;
-            rn[r] = 0;
-            if (p < D::HP) {
-                const int di = p % D::HI, dj = p / D::HI;
-                const int wi = wrapi(i0 - 1 + di, g.mx, g.pi), wj = wrapi(j0 - 1 + dj, g.my, g.pj);
-                if (wi >= 0 && wi < g.mx && wj >= 0 && wj < g.my && wk >= 0 && wk < g.mz) {
-                    const long long q = ((long long)wk * g.my + wj) * g.mx + wi;
-                    rv[r][0] = a.ucat[3 * q]; rv[r][1] = a.ucat[3 * q + 1]; rv[r][2] = a.ucat[3 * q + 2];
-                    if (!NB) rn[r] = (float)a.nvert[q];
-                    if (les) rv[r][3] = a.nut[q];
-                }
+    for (int r = 0; r < TPP; r++) {
+        const int p = threadIdx.x + r * FP_T, dj = p / D::HI;
+        const int wi = wrapi(i0 - 1 + p % D::HI, g.mx, g.pi), wj = wrapi(j0 - 1 + dj, g.my, g.pj);
+        tof[r] = p < D::HP && wi >= 0 && wi < g.mx && wj >= 0 && wj < g.my ? (unsigned)(wj * g.mx + wi) : 0;
+        rv[r][3] = 0;
+    }
+    auto fetch_plane = [&](int kk) {
+        const long long q = (long long)wrapi(kk, g.mz, g.pk) * g.plane;
+        const double *u = a.ucat + 3 * q;
+#pragma unroll
+        for (int r = 0; r < TPP; r++)
+            if ((r + 1) * FP_T <= D::HP || threadIdx.x + r * FP_T < D::HP) {
+                const unsigned b3 = lane_offset(24 * tof[r]), b1 = lane_offset(8 * tof[r]);
+                rv[r][0] = at_byte(u, b3); rv[r][1] = at_byte(u + 1, b3); rv[r][2] = at_byte(u + 2, b3);
+                if (!NB) rn[r] = (float)at_byte(a.nvert + q, b1);
+                if (les) rv[r][3] = at_byte(a.nut + q, b1);
             }
-        }
     };
     auto store_plane = [&](int slot) {
 #pragma unroll
         for (int r = 0; r < TPP; r++) {
-            const int p = threadIdx.x + r * FT_I * FT_J;
-            if (p < D::HP) {
+            const int p = threadIdx.x + r * FP_T;
+            if ((r + 1) * FP_T <= D::HP || p < D::HP) {
                 const int l = slot * D::HP + p;
-                sx[l] = rv[r][0]; sy[l] = rv[r][1]; sz[l] = rv[r][2]; st[l] = rv[r][3];
-                if (!NB) sn[l] = rn[r];
+#pragma unroll
+                for (int c = 0; c < 4; c++) S.u[c][l] = rv[r][c];
+                if (!NB) S.nv[l] = rn[r];
             }
         }
     };
     const int kstart = k0 - 1;
-    fetch_plane(kstart - 1);
-    store_plane(0);
+    long long q0 = (long long)kstart * g.plane;  // the plane's first point
     fetch_plane(kstart);
-    store_plane(1);
+    store_plane(1);  // (plane kstart - 1, slot 0, is never read)
     fetch_plane(kstart + 1);
     int slot0 = 0;
+    // cell metrics of the point (cur) and of the cell above it (nk), which the
+    // next plane takes over; [9] the reciprocal Jacobian
     double cur[10], nk[10], kprev[6];
     for (int c = 0; c < 6; c++) kprev[c] = 0;
-    bool have = false;
-    for (int k = kstart; k < k1; k++) {
+    const unsigned off = (unsigned)(j * g.mx + i);
+    load_metrics(a.cell, q0, off, cur);
+    cur[9] = 1. / cur[9];
+    for (int k = kstart; k < k1; k++, q0 += g.plane) {
         int s2 = slot0 + 2;
         if (s2 >= 3) s2 -= 3;
         store_plane(s2);  // plane k+1
         __syncthreads();
         if (k + 1 < k1) fetch_plane(k + 2);
-        TileAcc<true, NB> T{&a, sx, sy, sz, st, sn, i0, j0, k, slot0};
+        const int s1 = slot0 + 1 < 3 ? slot0 + 1 : 0;
+        auto tile = [&](int ii, int jj) {
+            const int p = (int)lane_offset((unsigned)((jj - j0) * D::HI + (ii - i0)));
+            return PointTile<NB>{&S.u[0][0], S.nv, ii, jj, k, s1 * D::HP + p, (slot0 - s1) * D::HP, (s2 - s1) * D::HP};
+        };
         const bool full = k >= k0;  // the plane below the block: its k face only
-        const long long q = ((long long)k * g.my + j) * g.mx + i;
-        if (inb && !have) load_metrics(a.cell, q, cur);
+        double kf[6], M[10];
         double di[6] = {0, 0, 0, 0, 0, 0};  // i-face differences, div xyz and visc xyz
         if (full) {
+            double nb[10], f6[6];
             // i faces: this point's face i+1/2 and, from the lane before it
             // in the row (a row of FT_I points is FT_I consecutive lanes of
             // one wavefront), the face i-1/2; the row's first lane takes the
             // face i0-1/2 from LDS after the barrier.
-            double f6[6] = {0, 0, 0, 0, 0, 0};
-            if (inb) {
-                double nb_[10], M[10];
-                load_metrics(a.cell, i < g.mx - 1 ? q + 1 : q, nb_);
-                face_mean(cur, nb_, M);
-                flux_i<true, NB>(a, T, i, j, k, M, a.ucont[3 * q + 0], f6, f6 + 3);
+            load_metrics(a.cell, q0 + 1, off, nb);
+            double u = at_byte(a.ucont + 3 * q0, lane_offset(24 * off));
+            nb[9] = 1. / nb[9];
+            face_sum(cur, nb, M);
+            __builtin_amdgcn_sched_barrier(0);
+            face_i(a, tile(i, j), i, j, k, M, u, f6, f6 + 3);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int c = 0; c < 6; c++) {
+                const double fl = lane_before(f6[c]);
+                di[c] = tx == 0 ? f6[c] : f6[c] - fl;
             }
-            double fl[6];
-            for (int c = 0; c < 6; c++) fl[c] = __shfl_up(f6[c], 1, FT_I);
-            for (int c = 0; c < 6; c++) di[c] = tx == 0 ? f6[c] : f6[c] - fl[c];
-            for (int c = 0; c < 6; c++) f6[c] = 0;
-            if (inb) {
-                double nb_[10], M[10];
-                load_metrics(a.cell, j < g.my - 1 ? q + g.mx : q, nb_);
-                face_mean(cur, nb_, M);
-                flux_j<true, NB>(a, T, i, j, k, M, a.ucont[3 * q + 1], f6, f6 + 3);
-            }
+            reread_tile();
+            load_metrics(a.cell, q0 + g.mx, off, nb);
+            u = at_byte(a.ucont + 3 * q0 + 1, lane_offset(24 * off));
+            nb[9] = 1. / nb[9];
+            face_sum(cur, nb, M);
+            __builtin_amdgcn_sched_barrier(0);
+            face_j(a, tile(i, j), i, j, k, M, u, f6, f6 + 3);
+#pragma unroll
             for (int c = 0; c < 6; c++) fxj[c][ty + 1][tx] = f6[c];
+            reread_tile();
             if (ty == 0) {  // j face at j0-1 of this column
-                for (int c = 0; c < 6; c++) f6[c] = 0;
-                if (j0 >= 1 && i < g.mx) {
-                    const long long p = q - g.mx;
-                    double cp[10], M[10];
-                    load_metrics(a.cell, p, cp);
-                    face_mean(cp, cur, M);
-                    flux_j<true, NB>(a, T, i, j0 - 1, k, M, a.ucont[3 * p + 1], f6, f6 + 3);
-                }
+                load_metrics(a.cell, q0 - g.mx, off, nb);
+                u = at_byte(a.ucont + 3 * (q0 - g.mx) + 1, lane_offset(24 * off));
+                nb[9] = 1. / nb[9];
+                face_sum(nb, cur, M);
+                __builtin_amdgcn_sched_barrier(0);
+                face_j(a, tile(i, j0 - 1), i, j0 - 1, k, M, u, f6, f6 + 3);
+#pragma unroll
                 for (int c = 0; c < 6; c++) fxj[c][0][tx] = f6[c];
             }
             // the face i0-1/2 of each row, on lanes of the second wavefront
             // (the first one computes the faces j0-1/2), so that no
             // wavefront evaluates more than one halo face
             const int r = (int)threadIdx.x - HX_T0;
-            if (r >= 0 && r < FT_J) {
-                const int jr = j0 + r;
-                for (int c = 0; c < 6; c++) f6[c] = 0;
-                if (i0 >= 1 && jr < g.my) {
-                    const long long p = ((long long)k * g.my + jr) * g.mx + (i0 - 1);
-                    double cp[10], cn[10], M[10];
-                    load_metrics(a.cell, p, cp);
-                    load_metrics(a.cell, p + 1, cn);
-                    face_mean(cp, cn, M);
-                    flux_i<true, NB>(a, T, i0 - 1, jr, k, M, a.ucont[3 * p + 0], f6, f6 + 3);
-                }
+            if (r >= 0 && r < FP_J) {
+                const int jr = j0 + r < g.my - 1 ? j0 + r : g.my - 2;
+                const unsigned oh = (unsigned)(jr * g.mx + i0 - 1);
+                double nc[10];
+                load_metrics(a.cell, q0, oh, nb);
+                load_metrics(a.cell, q0 + 1, oh, nc);
+                u = at_byte(a.ucont + 3 * q0, lane_offset(24 * oh));
+                nb[9] = 1. / nb[9];
+                nc[9] = 1. / nc[9];
+                face_sum(nb, nc, M);
+                __builtin_amdgcn_sched_barrier(0);
+                face_i(a, tile(i0 - 1, jr), i0 - 1, jr, k, M, u, f6, f6 + 3);
+#pragma unroll
                 for (int c = 0; c < 6; c++) hx[c][r] = f6[c];
             }
         }
-        double kf[6] = {0, 0, 0, 0, 0, 0};
-        if (inb) {
-            load_metrics(a.cell, k < g.mz - 1 ? q + g.plane : q, nk);
-            double M[10];
-            face_mean(cur, nk, M);
-            flux_k<true, NB>(a, T, i, j, k, M, a.ucont[3 * q + 2], kf, kf + 3);
-        }
+        reread_tile();
+        load_metrics(a.cell, q0 + g.plane, off, nk);
+        const double u = at_byte(a.ucont + 3 * q0 + 2, lane_offset(24 * off));
+        nk[9] = 1. / nk[9];
+        face_sum(cur, nk, M);
+        __builtin_amdgcn_sched_barrier(0);
+        face_k(a, tile(i, j), i, j, k, M, u, kf, kf + 3);
         __syncthreads();
         if (full && inb) {
-            double f[3] = {0, 0, 0};
-            double pr[3] = {0, 0, 0};
+            double f[3];
             if (tx == 0)
+#pragma unroll
                 for (int c = 0; c < 6; c++) di[c] = di[c] - hx[c][ty];
-            if (i >= 1 && i < g.mx - 1 && j >= 1 && j < g.my - 1 && k >= 1 && k < g.mz - 1) {
-                for (int c = 0; c < 3; c++) {
-                    f[c] = di[c] + fxj[c][ty + 1][tx] - fxj[c][ty][tx] + kf[c] - kprev[c];
-                    f[c] += (di[3 + c] + fxj[3 + c][ty + 1][tx] - fxj[3 + c][ty][tx] + kf[3 + c] - kprev[3 + c]) / 1.0;
-                }
-                // csi.Fp, eta.Fp, zet.Fp of this cell
-                for (int r = 0; r < 3; r++) pr[r] = cur[3 * r] * f[0] + cur[3 * r + 1] * f[1] + cur[3 * r + 2] * f[2];
+#pragma unroll
+            for (int c = 0; c < 3; c++) {
+                f[c] = di[c] + fxj[c][ty + 1][tx] - fxj[c][ty][tx] + kf[c] - kprev[c];
+                f[c] += (di[3 + c] + fxj[3 + c][ty + 1][tx] - fxj[3 + c][ty][tx] + kf[3 + c] - kprev[3 + c]) / 1.0;
             }
-            for (int r = 0; r < 3; r++) fp[r * n + q] = pr[r];
+            // csi.Fp, eta.Fp, zet.Fp of this cell
+#pragma unroll
+            for (int r = 0; r < 3; r++) fp[r * n + q0 + off] = cur[3 * r] * f[0] + cur[3 * r + 1] * f[1] + cur[3 * r + 2] * f[2];
         }
+#pragma unroll
         for (int c = 0; c < 6; c++) kprev[c] = kf[c];
-        if (inb) {
-            for (int c = 0; c < 10; c++) cur[c] = nk[c];
-            have = true;
-        }
+#pragma unroll
+        for (int c = 0; c < 10; c++) cur[c] = nk[c];
         // No barrier here: the next store_plane overwrites the slot of plane
         // k-1, which only the flux evaluations read (all done before the
         // barrier above), and fxj / hx are next written after the next
         // iteration's first barrier, which every wavefront reaches only once
         // it has finished reading them here.
-        slot0 = slot0 + 1 < 3 ? slot0 + 1 : 0;
+        slot0 = s1;
     }
 }
 
@@ -1023,20 +1128,22 @@ int nvert_all_zero(vfs_ctx *c, bool *zero)
 // one of their streams only: nothing is gained beyond this).
 constexpr int CELL_K = 16;
 
-// Planes a block of a face pass marches.  Its registers and LDS leave one
-// block per CU, so a pass takes ceil(blocks / CUs) turns of kc planes, the
-// `extra` planes it computes a second time and the three plane loads before
-// the first one: the run that makes this shortest is taken.  Against runs of
-// 16 planes everywhere: k_face_fp 100 -> 14 us on 16x12x16 cells, 105 -> 24 us
-// on 64x48x64, 107 -> 39 us on 96x64x80, 797 -> 777 us on 256x192x256 (runs of
-// 32); fourth-order k_face_fluxes 372 -> 316 us on 136x104x88.
-static int face_planes(long long tiles, int nk, int extra)
+// Planes a block of a face pass marches.  Its registers and LDS leave per_cu
+// blocks on a CU, so a pass takes ceil(blocks / (CUs * per_cu)) turns of kc
+// planes, the `extra` planes it computes a second time and the plane loads
+// before the first one: the run that makes this shortest is taken.  Against
+// runs of 16 planes everywhere (with one block of 16 rows per CU): k_face_fp
+// 100 -> 14 us on 16x12x16 cells, 105 -> 24 us on 64x48x64, 107 -> 39 us on
+// 96x64x80, 797 -> 777 us on 256x192x256 (runs of 32); fourth-order
+// k_face_fluxes 372 -> 316 us on 136x104x88.
+static int face_planes(long long tiles, int nk, int extra, int per_cu)
 {
-    constexpr int CUS = 256, FILL = 3, LONGEST = 64;
+    constexpr int FILL = 3, LONGEST = 64;
+    const int slots = 256 * per_cu;
     int best = 1;
     long long cost = -1;
     for (int kc = 1; kc <= LONGEST && kc <= nk; kc++) {
-        const long long turns = (tiles * ((nk + kc - 1) / kc) + CUS - 1) / CUS, t = turns * (kc + extra + FILL);
+        const long long turns = (tiles * ((nk + kc - 1) / kc) + slots - 1) / slots, t = turns * (kc + extra + FILL);
         if (cost < 0 || t < cost) {
             cost = t;
             best = kc;
@@ -1090,11 +1197,11 @@ int formfunction2(vfs_ctx *c, double scale, const double *pucont, double rk_alph
     prof_begin(c, K_FACE);
     if (fused) {
         // a block also computes the k faces below its first plane
-        const int kc = face_planes(face_fp_tiles(g), g.mz - 2, 1);
-        hipLaunchKernelGGL(nb ? k_face_fp<true> : k_face_fp<false>, blocks(face_fp_tiles(g), g.mz - 2, kc), dim3(FT_I * FT_J), 0,
+        const int kc = face_planes(face_fp_tiles(g), g.mz - 2, 1, FP_WAVES);
+        hipLaunchKernelGGL(nb ? k_face_fp<true> : k_face_fp<false>, blocks(face_fp_tiles(g), g.mz - 2, kc), dim3(FP_T), 0,
                            st, fa, kc, c->fpc);
     } else {
-        const int kc = face_planes(tiles, g.mz, 0);
+        const int kc = face_planes(tiles, g.mz, 0, 1);
         auto kern = !fa.second_order ? k_face_fluxes<false, false>
                                      : (c->face_derived ? k_face_fluxes<true, true> : k_face_fluxes<true, false>);
         hipLaunchKernelGGL(kern, blocks(tiles, g.mz, kc), dim3(FT_I * FT_J), 0, st, fa, kc);
