@@ -61,3 +61,21 @@ def test_amg_graph_replays_match_direct_launches(monkeypatch):
     monkeypatch.delenv("VFS_AMG_GRAPH")
     assert out[0][0] == out[1][0] and out[0][0] >= 3
     assert np.array_equal(out[0][1], out[1][1])
+
+
+@pytest.mark.parametrize("size", [(24, 16, 20), (18, 13, 22)], ids=str)
+def test_amg_smoother_layouts_bitwise(monkeypatch, size):
+    """The smoother on the rows laid out by colour (padded to the colour's
+    longest) and on the CSR rows: the same bits over a solve."""
+    out = []
+    for rows in ("padded", "csr"):
+        monkeypatch.setenv("VFS_AMG_ROWS", rows)
+        c, o, ctx = channel_pair(*size, les=0)
+        with ctx:
+            ctx.runge_kutta()
+            ctx.poisson_rhs()
+            ctx.upload("PHI", np.zeros(o.shape))
+            st = ctx.poisson_solve(vfs.default_solve_opts(tol=1e-10, use_guess=0, amg=1, maxit=300))
+            out.append((st.iterations, ctx.download("PHI")))
+    assert out[0][0] == out[1][0]
+    assert np.array_equal(out[0][1], out[1][1])

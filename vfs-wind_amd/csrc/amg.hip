@@ -389,18 +389,62 @@ __global__ void k_csr_mv(int n, int add, const int *__restrict__ ptr, const int 
 
 // Gauss-Seidel on the rows of one colour: x_i = (b_i - sum_{j != i} a_ij x_j) / a_ii.
 // Rows of one colour share no entry, so the pass is race-free and its result
-// does not depend on the thread order.
+// does not depend on the thread order.  A V-cycle is some 300 of these launches,
+// one after the other, and a launch is a chain of dependent loads; from the CSR
+// arrays it was five long (row, its bounds, columns, x, right-hand side) and
+// 3.4 us with 64 lanes per row, 4.5 us with 32.  Here a colour's rows are laid out one after the
+// other at a fixed `width`, so that their entries and row numbers are the first
+// load and x and the right-hand side the second: 2.8 and 3.1 us (a launch that
+// does nothing takes 2.1).
+// Entry q of a row keeps the lane it has in a walk over the CSR row, the
+// diagonal and the padding carry column -1: the same sums, to the bit.
+template <int G, int M>
+__global__ void k_gs_colour(int nrows, int width, const int *__restrict__ rows, const int *__restrict__ col,
+                            const double *__restrict__ val, const double *__restrict__ dinv, const double *__restrict__ b,
+                            double *__restrict__ x)
+{
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    const int k = t / G, lane = t % G;
+    if (k >= nrows) return;
+    const int i = rows[k];
+    const double d = dinv[k];
+    const long long e = (long long)k * width;
+    double s = 0, bi = 0;
+    for (int m0 = 0; m0 < width; m0 += M * G) {  // (once, but for rows of more than 4 G entries)
+        int j[M];
+        double v[M], xv[M];
+#pragma unroll
+        for (int m = 0; m < M; m++) {
+            const int q = lane + m0 + m * G;
+            const long long at = e + (q < width ? q : width - 1);
+            j[m] = q < width ? col[at] : -1;
+            v[m] = val[at];
+        }
+        if (m0 == 0) bi = b[i];
+#pragma unroll
+        for (int m = 0; m < M; m++) xv[m] = x[j[m] < 0 ? i : j[m]];
+#pragma unroll
+        for (int m = 0; m < M; m++)
+            if (j[m] >= 0) s += v[m] * xv[m];
+    }
+#pragma unroll
+    for (int m = G / 2; m > 0; m >>= 1) s += __shfl_xor(s, m, G);
+    if (lane == 0) x[i] = (bi - s) * d;
+}
+
+// The same from the CSR arrays, for colours whose rows differ much in length
+// and are so many that reading the padding would cost more than the chain.
 template <int G>
-__global__ void k_gs_colour(int nrows, const int *__restrict__ rows, const int *__restrict__ ptr,
-                            const int *__restrict__ col, const double *__restrict__ val,
-                            const double *__restrict__ dinv, const double *__restrict__ b, double *__restrict__ x)
+__global__ void k_gs_rows(int nrows, const int *__restrict__ rows, const int *__restrict__ ptr, const int *__restrict__ col,
+                          const double *__restrict__ val, const double *__restrict__ dinv, const double *__restrict__ b,
+                          double *__restrict__ x)
 {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     const int k = t / G, lane = t % G;
     if (k >= nrows) return;
     const int i = rows[k];
     const double s = group_row_dot<G>(i, ptr, col, val, x, i, lane);
-    if (lane == 0) x[i] = (b[i] - s) * dinv[i];
+    if (lane == 0) x[i] = (b[i] - s) * dinv[k];
 }
 
 // x = Inv b on the coarsest level (row-major inverse), one wavefront per row
@@ -437,10 +481,17 @@ __global__ void k_zero_d(long long n, double *__restrict__ x)
 struct AmgLevel {
     int n = 0;
     int *ap = nullptr, *ac = nullptr, *pp = nullptr, *pc = nullptr, *rp = nullptr, *rc = nullptr;
-    double *av = nullptr, *pv = nullptr, *rv = nullptr, *dinv = nullptr;
+    double *av = nullptr, *pv = nullptr, *rv = nullptr;
     double *x = nullptr, *b = nullptr, *r = nullptr;
     int *crows = nullptr;          // rows grouped by colour
     std::vector<int> coff;         // colour offsets into crows (host)
+    // the rows by colour, each colour's at its own width (its longest row's
+    // entries): columns, -1 for the diagonal and the padding, values, and the
+    // inverse diagonals
+    int *ec = nullptr;
+    double *ev = nullptr, *dinv = nullptr;
+    std::vector<int> cwidth;       // per colour: width, 0 = its rows stay in the CSR arrays
+    std::vector<long long> cbase;  // per colour: first entry
     int ga = 1, gp = 1, gr = 1;    // lanes per row of A, P and R
 };
 
@@ -488,8 +539,94 @@ static int lanes_for(const amg::Csr &M)
     }
 VFS_AMG_GROUPED(k_csr_apply)
 VFS_AMG_GROUPED(k_csr_mv)
-VFS_AMG_GROUPED(k_gs_colour)
 #undef VFS_AMG_GROUPED
+
+template <int G>
+static void launch_gs_colour(const AmgLevel &L, int c, hipStream_t st)
+{
+    const int first = L.coff[c], cnt = L.coff[c + 1] - first;
+    const dim3 nb(blocks_for((long long)cnt * G, ATPB));
+    const int w = L.cwidth[c];
+    if (!w) {
+        hipLaunchKernelGGL(k_gs_rows<G>, nb, dim3(ATPB), 0, st, cnt, (const int *)L.crows + first, (const int *)L.ap,
+                           (const int *)L.ac, (const double *)L.av, (const double *)L.dinv + first, (const double *)L.b, L.x);
+        return;
+    }
+    auto k = w <= G ? k_gs_colour<G, 1> : w <= 2 * G ? k_gs_colour<G, 2> : k_gs_colour<G, 4>;
+    hipLaunchKernelGGL(k, nb, dim3(ATPB), 0, st, cnt, w, (const int *)L.crows + first, (const int *)L.ec + L.cbase[c],
+                       (const double *)L.ev + L.cbase[c], (const double *)L.dinv + first, (const double *)L.b, L.x);
+}
+static void relax_colour(const AmgLevel &L, int c, hipStream_t st)
+{
+    switch (L.ga) {
+    case 2: launch_gs_colour<2>(L, c, st); break;
+    case 4: launch_gs_colour<4>(L, c, st); break;
+    case 8: launch_gs_colour<8>(L, c, st); break;
+    case 16: launch_gs_colour<16>(L, c, st); break;
+    case 32: launch_gs_colour<32>(L, c, st); break;
+    default: launch_gs_colour<64>(L, c, st); break;
+    }
+}
+
+// The smoother's layout of a level: rows by colour, padded to the colour's
+// longest row, unless that reads more than half as much again as the rows hold
+// and the colour fills the GPU (COLOUR_FULL lanes: below that a launch waits for
+// its loads, not for their number).  VFS_AMG_ROWS=csr, =padded force one.
+constexpr long long COLOUR_FULL = 256LL * 2048;
+static long long colour_widths(const amg::Csr &M, const std::vector<int> &rows, AmgLevel &L)
+{
+    const char *env = std::getenv("VFS_AMG_ROWS");
+    const int nc = (int)L.coff.size() - 1;
+    L.cwidth.assign(nc, 0);
+    L.cbase.assign(nc, 0);
+    long long total = 0;
+    for (int c = 0; c < nc; c++) {
+        const long long cnt = L.coff[c + 1] - L.coff[c];
+        long long longest = 1, held = 0;
+        for (int k = L.coff[c]; k < L.coff[c + 1]; k++) {
+            const int len = M.ptr[rows[k] + 1] - M.ptr[rows[k]];
+            longest = std::max<long long>(longest, len);
+            held += len;
+        }
+        bool pad = 2 * longest * cnt <= 3 * held || cnt * L.ga < COLOUR_FULL;
+        if (env && env[0] == 'c') pad = false;
+        if (env && env[0] == 'p') pad = true;
+        L.cbase[c] = total;
+        if (!pad) continue;
+        L.cwidth[c] = (int)longest;
+        total += longest * cnt;
+    }
+    return total;
+}
+
+// one colour's rows into that layout (32 lanes a row), and its inverse diagonals
+__global__ void k_colour_layout(int nrows, int width, const int *__restrict__ rows, const int *__restrict__ ptr,
+                                const int *__restrict__ col, const double *__restrict__ val, int *__restrict__ ec,
+                                double *__restrict__ ev, double *__restrict__ dinv)
+{
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    const int k = t / 32, lane = t % 32;
+    if (k >= nrows) return;
+    const int i = rows[k], first = ptr[i], len = ptr[i + 1] - first;
+    const int end = len > width ? len : width;
+    for (int q = lane; q < end; q += 32) {
+        int j = -1;
+        double v = 0;
+        if (q < len) {
+            j = col[first + q];
+            v = val[first + q];
+            if (j == i) {
+                if (v != 0) dinv[k] = 1.0 / v;
+                j = -1;
+                v = 0;
+            }
+        }
+        if (q < width) {
+            ec[(long long)k * width + q] = j;
+            ev[(long long)k * width + q] = v;
+        }
+    }
+}
 
 template <typename T>
 static int dev_copy(AmgDev *a, T **dst, const T *src, size_t count)
@@ -591,18 +728,26 @@ int amg_build(const double *c64_host, const unsigned char *row_host, long long n
         AmgLevel &L = a->L[l];
         const amg::Csr &M = H.A[l];
         L.n = M.n;
-        std::vector<double> dinv(M.n, 0.0);
-        for (int i = 0; i < M.n; i++)
-            for (int q = M.ptr[i]; q < M.ptr[i + 1]; q++)
-                if (M.col[q] == i && M.val[q] != 0) dinv[i] = 1.0 / M.val[q];
         std::vector<int> crows;
-        amg::colouring(M, crows, L.coff);
+        long long entries = 0;
         L.ga = lanes_for(M);
+        if (l + 1 < nl) {  // (the coarsest level is solved, not smoothed)
+            amg::colouring(M, crows, L.coff);
+            entries = colour_widths(M, crows, L);
+        }
+        rc = rc ? rc : dev_copy<int>(a, &L.ec, nullptr, entries);
+        rc = rc ? rc : dev_copy<double>(a, &L.ev, nullptr, entries);
+        rc = rc ? rc : dev_copy<double>(a, &L.dinv, nullptr, M.n);
         rc = rc ? rc : dev_copy(a, &L.crows, crows.data(), crows.size());
         rc = rc ? rc : dev_copy(a, &L.ap, M.ptr.data(), M.ptr.size());
         rc = rc ? rc : dev_copy(a, &L.ac, M.col.data(), M.col.size());
         rc = rc ? rc : dev_copy(a, &L.av, M.val.data(), M.val.size());
-        rc = rc ? rc : dev_copy(a, &L.dinv, dinv.data(), dinv.size());
+        for (size_t c = 0; !rc && c < L.cwidth.size(); c++) {
+            const int first = L.coff[c], cnt = L.coff[c + 1] - first;
+            hipLaunchKernelGGL(k_colour_layout, dim3(blocks_for(32LL * cnt, ATPB)), dim3(ATPB), 0, nullptr, cnt, L.cwidth[c],
+                               (const int *)L.crows + first, (const int *)L.ap, (const int *)L.ac, (const double *)L.av,
+                               L.ec + L.cbase[c], L.ev + L.cbase[c], L.dinv + first);
+        }
         rc = rc ? rc : dev_copy<double>(a, &L.x, nullptr, M.n);
         rc = rc ? rc : dev_copy<double>(a, &L.b, nullptr, M.n);
         rc = rc ? rc : dev_copy<double>(a, &L.r, nullptr, M.n);
@@ -621,6 +766,7 @@ int amg_build(const double *c64_host, const unsigned char *row_host, long long n
     }
     rc = rc ? rc : dev_copy(a, &a->inv, inv.data(), inv.size());
     rc = rc ? rc : dev_copy(a, &a->ridx, pts.data(), pts.size());
+    if (!rc) rc = hipStreamSynchronize(nullptr) == hipSuccess ? VFS_OK : check_hip(hipGetLastError(), "amg layout");
     if (rc) { amg_free(a); return rc; }
     *out = a;
     return VFS_OK;
@@ -635,15 +781,10 @@ static void amg_cycle(hipStream_t st, AmgDev *a, int l)
         return;
     }
     AmgLevel &C = a->L[l + 1];
-    const int ncol = (int)L.coff.size() - 1;
-    auto relax = [&](int c) {
-        const int cnt = L.coff[c + 1] - L.coff[c];
-        launch_k_gs_colour(L.ga, cnt, st, cnt, (const int *)L.crows + L.coff[c], (const int *)L.ap, (const int *)L.ac,
-                           (const double *)L.av, (const double *)L.dinv, (const double *)L.b, L.x);
-    };
     // pre-smoothing (forward colours) from a zero iterate, residual, restriction
     hipLaunchKernelGGL(k_zero_d, dim3(nb), dim3(ATPB), 0, st, (long long)L.n, L.x);
-    for (int c = 0; c < ncol; c++) relax(c);
+    const int ncol = (int)L.coff.size() - 1;
+    for (int c = 0; c < ncol; c++) relax_colour(L, c, st);
     launch_k_csr_apply(L.ga, L.n, st, L.n, (const int *)L.ap, (const int *)L.ac, (const double *)L.av, (const double *)L.x,
                        (const double *)L.b, L.r);
     launch_k_csr_mv(L.gr, C.n, st, C.n, 0, (const int *)L.rp, (const int *)L.rc, (const double *)L.rv,
@@ -652,7 +793,7 @@ static void amg_cycle(hipStream_t st, AmgDev *a, int l)
     // prolongation and post-smoothing (backward colours)
     launch_k_csr_mv(L.gp, L.n, st, L.n, 1, (const int *)L.pp, (const int *)L.pc, (const double *)L.pv,
                     (const double *)C.x, L.x);
-    for (int c = ncol - 1; c >= 0; c--) relax(c);
+    for (int c = ncol - 1; c >= 0; c--) relax_colour(L, c, st);
 }
 
 // z = M^-1 v for DA-layout vectors (n_pts points; zero outside the rows).  The
