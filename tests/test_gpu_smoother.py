@@ -232,3 +232,28 @@ def test_short_segments_padding_bitwise(monkeypatch, ny):
         out.append((st.iterations, phi))
     assert out[0][0] == out[1][0]
     assert np.array_equal(out[0][1], out[1][1])
+
+
+@pytest.mark.parametrize("coarse_sweeps", [4, 5])
+@pytest.mark.parametrize("path", ["short", "long"])
+@pytest.mark.parametrize("cells", [(17, 12, 14), (16, 12, 15), (15, 11, 13), (33, 70, 31)], ids=str)
+def test_odd_periodic_counts_bitwise(monkeypatch, cells, path, coarse_sweeps):
+    """Odd counts along the periodic directions: the one-pass form between two
+    arrays against the two-pass form, at even and odd sweep counts (an odd
+    one's first sweep is the two-pass form's), on whole solves."""
+    out = []
+    monkeypatch.setenv("VFS_LINE_PATH", path)
+    monkeypatch.setenv("VFS_MG_TAIL", "0")
+    monkeypatch.setenv("VFS_SMOOTH_COMPACT", "1")
+    for fused in ("1", "0"):
+        monkeypatch.setenv("VFS_ZEBRA_FUSED", fused)
+        c, o, ctx = channel_pair(*cells, les=0)
+        with ctx:
+            ctx.poisson_rhs()
+            opts = vfs.default_solve_opts(tol=1e-8, use_guess=0, maxit=1500, coarse_sweeps=coarse_sweeps)
+            for _ in range(2):  # the second solve replays what the first captured
+                ctx.upload("PHI", np.zeros(o.shape))
+                st = ctx.poisson_solve(opts)
+            out.append((st.iterations, ctx.download("PHI")))
+    assert out[0][0] == out[1][0]
+    assert np.array_equal(out[0][1], out[1][1])

@@ -509,14 +509,14 @@ __device__ inline float c4_sum(h4_t w, float d, float xe, float xw, float xt, fl
     acc += (float)w.w * xb;
     return bq - d * acc;
 }
-__device__ inline float c4_rhs(const Grid &g, const int I[3], const int K[3], int j, h4_t w, float d, const float *__restrict__ x,
-                               float bq)
+__device__ inline float c4_rhs(const Grid &g, const int I[3], const int K[3], int j, h4_t w, float d, const float *pe,
+                               const float *pw, const float *pt, const float *pb, float bq)
 {
     const long long row0 = (long long)j * g.mx;
-    const float xe = x[(long long)K[1] * g.plane + row0 + I[2]];
-    const float xw = x[(long long)K[1] * g.plane + row0 + I[0]];
-    const float xt = x[(long long)K[2] * g.plane + row0 + I[1]];
-    const float xb = x[(long long)K[0] * g.plane + row0 + I[1]];
+    const float xe = pe[(long long)K[1] * g.plane + row0 + I[2]];
+    const float xw = pw[(long long)K[1] * g.plane + row0 + I[0]];
+    const float xt = pt[(long long)K[2] * g.plane + row0 + I[1]];
+    const float xb = pb[(long long)K[0] * g.plane + row0 + I[1]];
     return c4_sum(w, d, xe, xw, xt, xb, bq);
 }
 
@@ -535,7 +535,7 @@ __global__ void __launch_bounds__(PTPB) k_zebra_rhs_c4(Grid g, ZGrid z, int c, c
     const int I[3] = {canon(i - 1, g.mx, g.pi), i, canon(i + 1, g.mx, g.pi)};
     const int K[3] = {canon(k - 1, g.mz, g.pk), k, canon(k + 1, g.mz, g.pk)};
     const long long cq = c * z.cplane + t;
-    rz[t] = c4_rhs(g, I, K, j, sh[cq], sd[cq], x, b[((long long)k * g.my + j) * g.mx + i]);
+    rz[t] = c4_rhs(g, I, K, j, sh[cq], sd[cq], x, x, x, x, b[((long long)k * g.my + j) * g.mx + i]);
 }
 
 // colour-split off-line coefficients and Thomas factors (lo, 1/pivot,
@@ -802,13 +802,20 @@ __host__ __device__ inline bool zebra_fused_ok(const Grid &g)
     return (!g.pi || ((g.mx - 2) & 1) == 0) && (!g.pk || ((g.mz - 2) & 1) == 0);
 }
 
+// With an odd count along a periodic direction the lines at its two ends are
+// neighbours of one colour, and a line must read the other's value from before
+// this half-sweep (as the two-pass form does).  PP: each colour's values then
+// alternate between two arrays; xo holds the other colour's, xs this colour's
+// current values, and the new ones go to x: on 45x37x51 one launch of 5.6 us
+// instead of two of 7.7 together and the gap between them.
 // LL lines per block (32, or 64 with at most 16 segments per line)
-template <int SLM, bool XZ, bool SPL, int LL>
+template <int SLM, bool XZ, bool SPL, int LL, bool PP = false>
 __global__ void __launch_bounds__(1024) k_zebra_line_c4(Grid g, ZGrid z, int c, int nseg, int sl,
                                                                            const h4_t *__restrict__ sh,
                                                                            const float *__restrict__ sd,
                                                                            const float *__restrict__ b,
-                                                                           const float *__restrict__ sf, float *x)
+                                                                           const float *__restrict__ sf, float *x,
+                                                                           const float *xo, const float *xs)
 {
     static_assert(LL * (LL == 64 ? 16 : LINE_MAXSEG) <= 1024, "threads per block");
     __shared__ float sA[1024], sB[1024];
@@ -854,6 +861,8 @@ __global__ void __launch_bounds__(1024) k_zebra_line_c4(Grid g, ZGrid z, int c, 
     // half-sweep at 64x48x64 and 6.5 on the 48x32x40 level of a 96x64x80 grid,
     // together 4.8 and 4.2; at 160x96x192 both 12 (4.4 TB/s).
     const int np = act ? j1 - j0 : 0;
+    auto from = [&](int ii, int kx) -> const float * { return !PP ? x : ((ii + kx - i - k) & 1) ? xo : xs; };
+    const float *pe = from(I[2], k), *pw = from(I[0], k), *pt = from(i, K[2]), *pb = from(i, K[0]);
     const float *lo = sf + cb, *mm = sf + sstride + cb, *cp = sf + 2 * sstride + cb;
     float r[SLM], l[SLM], m[SLM], u[SLM];
     if constexpr (SLM <= 8) {
@@ -876,10 +885,10 @@ __global__ void __launch_bounds__(1024) k_zebra_line_c4(Grid g, ZGrid z, int c, 
                 xt[v] = x[stp + o];
                 xb[v] = x[sbt + o];
             } else {
-                xe[v] = x[(long long)K[1] * g.plane + row0 + I[2]];
-                xw[v] = x[(long long)K[1] * g.plane + row0 + I[0]];
-                xt[v] = x[(long long)K[2] * g.plane + row0 + I[1]];
-                xb[v] = x[(long long)K[0] * g.plane + row0 + I[1]];
+                xe[v] = pe[(long long)K[1] * g.plane + row0 + I[2]];
+                xw[v] = pw[(long long)K[1] * g.plane + row0 + I[0]];
+                xt[v] = pt[(long long)K[2] * g.plane + row0 + I[1]];
+                xb[v] = pb[(long long)K[0] * g.plane + row0 + I[1]];
             }
             l[v] = lo[o];
             m[v] = mm[o];
@@ -911,7 +920,7 @@ __global__ void __launch_bounds__(1024) k_zebra_line_c4(Grid g, ZGrid z, int c, 
                     r[v] = c4_sum(sh[cb + o], sd[cb + o], oke ? x[se + o] : 0.f, okw ? x[sw + o] : 0.f, okt ? x[stp + o] : 0.f,
                                   okb ? x[sbt + o] : 0.f, bq);
                 else
-                    r[v] = c4_rhs(g, I, K, jj + 1, sh[cb + o], sd[cb + o], x, bq);
+                    r[v] = c4_rhs(g, I, K, jj + 1, sh[cb + o], sd[cb + o], pe, pw, pt, pb, bq);
                 l[v] = lo[o];
                 m[v] = mm[o];
                 u[v] = cp[o];
@@ -1803,6 +1812,9 @@ struct PLevel {
     // the finest level's FP32 iterate and right-hand side in the S layout
     // (the compact one-pass path; finest set on level 0 only)
     float *xs32 = nullptr, *bs32 = nullptr;
+    // the iterate's second array (levels with an odd count along a periodic
+    // direction: the one-pass compact form alternates)
+    float *y32 = nullptr;
     bool finest = false;
     double *x64 = nullptr, *b64 = nullptr, *r64 = nullptr;
     // dense inverse on the coarsest level (nr rows), column-major
@@ -1890,6 +1902,7 @@ static int level_alloc_work(vfs_poisson *ps, PLevel &L)
     const size_t cp = (size_t)L.z.cplane;
     int rc = 0;
     rc = rc ? rc : palloc(ps, (void **)&L.x32, n * 4);
+    if (!zebra_fused_ok(L.g)) rc = rc ? rc : palloc(ps, (void **)&L.y32, n * 4);
     rc = rc ? rc : palloc(ps, (void **)&L.b32, n * 4);
     rc = rc ? rc : palloc(ps, (void **)&L.r32, n * 4);
     rc = rc ? rc : palloc(ps, (void **)&L.x64, n * 8);
@@ -2255,6 +2268,7 @@ struct LinePlan {
     bool split;  // the finest level on the one-pass path: x and b in the S layout
     int nseg, sl;
     int lines;   // lines per block of the one-pass kernel (32 or 64)
+    bool twin;   // the one-pass kernel between two arrays (odd periodic counts)
 };
 template <typename T>
 static LinePlan line_plan(const PLevel &L)
@@ -2268,7 +2282,7 @@ static LinePlan line_plan(const PLevel &L)
     const int force = !lp ? 0 : lp[0] == 's' && lp[1] == 'h' ? 1 : lp[0] == 'l' ? 2 : lp[0] == 's' ? 3 : 0;
     p.short_seg = sizeof(T) == 4 && L.z.njI <= LINE_SLM_SHORT * LINE_MAXSEG;
     const char *fz = std::getenv("VFS_ZEBRA_FUSED");
-    const bool fusable = sizeof(T) == 4 && L.compact && zebra_fused_ok(L.g) && !(fz && fz[0] == '0');
+    const bool compact1 = sizeof(T) == 4 && L.compact && !(fz && fz[0] == '0'), fusable = compact1 && zebra_fused_ok(L.g);
     // on the finest level the one-pass kernel takes 16-point segments and 64
     // lines per block up to 256-point lines (a segment row is a whole
     // wavefront; the coarse levels, which fill fewer blocks, keep 8 and 32)
@@ -2286,6 +2300,7 @@ static LinePlan line_plan(const PLevel &L)
     // the compact form's right-hand sides are formed inside the line solve
     // (k_zebra_line_c4) unless VFS_ZEBRA_FUSED=0 asks for the two-pass form
     p.fused = fusable && p.scan;
+    p.twin = compact1 && !fusable && p.scan && L.y32;
     p.lines = p.fused && !p.short_seg && p.nseg <= 16 ? 64 : 32;
     // VFS_MG_SPLIT=0 keeps the finest level's vectors in the natural layout
     // (as does the stored-residual restriction, VFS_MG_FUSED_RESTRICT=0)
@@ -2326,7 +2341,20 @@ static void smooth(vfs_ctx *c, PLevel &L, int sweeps, bool x_zero = false)
                                           : (xz ? k_zebra_line_c4<LG, true, false, 32> : k_zebra_line_c4<LG, false, false, 32>));
                 const unsigned blocks = (unsigned)((lines + P.lines - 1) / P.lines);
                 hipLaunchKernelGGL(k, dim3(blocks), dim3(P.lines * nseg), 0, st, L.g, L.z, col, nseg, sl, sh4, L.sd32,
-                                   P.split ? L.bs32 : L.b32, L.sc32, P.split ? L.xs32 : L.x32);
+                                   P.split ? L.bs32 : L.b32, L.sc32, P.split ? L.xs32 : L.x32, nullptr, nullptr);
+                if (fine) prof_end(c);
+                continue;
+            }
+            // an even number of sweeps leaves both colours in x32; a first odd
+            // one goes the two-pass way
+            if (P.twin && s >= (sweeps & 1)) {
+                if (fine) prof_begin(c, K_LRELAXC32);
+                float *const X[2] = {L.x32, L.y32};
+                const int own = (s - (sweeps & 1)) & 1, other = col ? 1 - own : own;  // the arrays that hold the colours
+                auto k = short_seg ? k_zebra_line_c4<LINE_SLM_SHORT, false, false, 32, true>
+                                   : k_zebra_line_c4<line_slm<float>(), false, false, 32, true>;
+                hipLaunchKernelGGL(k, dim3(scan_blocks), dim3(LINE_LINES * nseg), 0, st, L.g, L.z, col, nseg, sl, sh4, L.sd32,
+                                   L.b32, L.sc32, X[1 - own], (const float *)X[other], (const float *)X[own]);
                 if (fine) prof_end(c);
                 continue;
             }
