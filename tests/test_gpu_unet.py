@@ -101,6 +101,36 @@ def test_unet_gradients_match_oracle():
     net.close(); ctx.close()
 
 
+@pytest.mark.parametrize("cells,levels,base", [
+    ((20, 12, 28), 2, 16),   # one run along i, shorter than 64 and off the 16-point steps
+    ((68, 8, 20), 2, 16),    # a second run of four points
+    ((72, 64, 20), 2, 32),   # more rows than 64 slices want, two output tiles per layer
+], ids=str)
+def test_unet_weight_gradients_ragged(cells, levels, base):
+    """The weight gradients at runs that end inside a matrix step, at few and
+    many rows per slice, against the oracle (same tolerance as above)."""
+    c, o, ctx = channel_pair(*cells, les=0)
+    with ctx:
+        net = vfs.UNet(ctx, base=base, levels=levels, seed=7)
+        orc = uo.UNetOracle(base, levels)
+        rng = np.random.default_rng(4)
+        b, phi = np.zeros(ctx.field_shape("B")), np.zeros(ctx.field_shape("B"))
+        for f in (b, phi):
+            f[1:-1, 1:-1, 1:-1] = rng.standard_normal(tuple(n - 2 for n in f.shape))
+        ctx.upload("B", b)
+        ctx.upload("PHI", phi)
+        params = net.params(0).astype(np.float64)
+        net.gradients(ctx.device_ptr("B"), ctx.device_ptr("PHI"))
+        g = net.params(1).astype(np.float64)
+        _, go, _ = orc.gradients(params, b[1:-1, 1:-1, 1:-1], phi[1:-1, 1:-1, 1:-1], 1.0, bf16=True)
+        off = 0
+        for sh in orc.shapes():
+            n = int(np.prod(sh))
+            assert _nrel(g[off:off + n], go[off:off + n]) <= 5e-2, sh
+            off += n
+        net.close()
+
+
 def test_unet_training_reduces_loss():
     c, o, ctx, net, orc, b, phi = _setup()
     # a real (b, phi) pair: one Poisson solve of the channel

@@ -171,58 +171,108 @@ __global__ void __launch_bounds__(CV_TPB) k_conv3t(Dims d, int cin, const bf16 *
 
 // Partial weight gradients: block (x, y) sums X[p + tap][ci] G[p][co] over
 // the rows x, x + P, x + 2P, ... (P = gridDim.x; a row is a 64-point run along
-// i) for its (tap, 16-channel ci tile, 16-channel co tile) and writes the tile
-// into slice x of `part` (each slice 27 cin cout floats); k_sum_partials then
-// adds the slices in a fixed order, so the gradient does not depend on timing.
+// i) for the three i taps of its (dk, dj), its 16-channel ci tile and its NTB
+// 16-channel co tiles, and writes them into slice x of `part` (each slice
+// 27 cin cout floats); k_sum_partials then adds the slices in a fixed order, so
+// the gradient does not depend on timing.  The lanes hold channels, the matrix
+// instruction's K index is the point, so operands are gathered value by
+// value, and the loads' number and latency are what it costs: the three taps
+// share six values of X per four points (a tap alone took four) and every value
+// of G, and a row's loads are all issued, untested, before its products.  At
+// 64x48x64, base 16: 105 us a layer before, 54 now on average.
+template <int NTB>
 __global__ void __launch_bounds__(64) k_conv3_wgrad(Dims d, int cin, int cout, const bf16 *__restrict__ X,
                                                     const bf16 *__restrict__ G, float *__restrict__ part)
 {
-    const int CB = cin / 16, NT = cout / 16;
+    const int CB = cin / 16, NG = cout / (16 * NTB);
     int w = blockIdx.y;
-    const int t = w % NT;
-    w /= NT;
-    const int cb = w % CB, tap = w / CB;
-    const int dk = tap / 9 - 1, dj = (tap / 3) % 3 - 1, di = tap % 3 - 1;
+    const int t0 = (w % NG) * NTB;
+    w /= NG;
+    const int cb = w % CB, kj = w / CB;
+    const int dk = kj / 3 - 1, dj = kj % 3 - 1;
     const int lane = threadIdx.x, m = lane & 15, kq = lane >> 4;
     const int nbi = (d.ni + 63) / 64;
     const long long nrows = (long long)nbi * d.nj * d.nk;
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    f32x4 acc[3][NTB];
+#pragma unroll
+    for (int e = 0; e < 3; e++)
+#pragma unroll
+        for (int t = 0; t < NTB; t++) acc[e][t] = {0.f, 0.f, 0.f, 0.f};
     for (long long row = blockIdx.x; row < nrows; row += gridDim.x) {
         const int bi = row % nbi, j = (row / nbi) % d.nj, k = row / ((long long)nbi * d.nj);
         const int jj = j + dj, kk = k + dk;
         const bool rowin = jj >= 0 && jj < d.nj && kk >= 0 && kk < d.nk;
+        const bf16 *Xr = X + (rowin ? ((long long)kk * d.nj + jj) * d.ni : 0) * cin + cb * 16 + m;
+        const bf16 *Gr = G + ((long long)k * d.nj + j) * d.ni * cout + t0 * 16 + m;
+        short xv[4][6], gv[4][NTB][4];
+#pragma unroll
         for (int s = 0; s < 4; s++) {  // 16 points per MFMA step
-            bf16x4 a, b;
+            const int i0 = bi * 64 + s * 16 + 4 * kq;  // the lane's first point
+#pragma unroll
+            for (int r = 0; r < 6; r++) {
+                int ii = i0 + r - 1;
+                ii = ii < 0 ? 0 : (ii < d.ni ? ii : d.ni - 1);
+                xv[s][r] = (short)Xr[(long long)ii * cin];
+            }
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                const int i = bi * 64 + s * 16 + 4 * kq + r;  // K index = point
-                const int ii = i + di;
-                const bool pin = i < d.ni;
-                const bool xin = rowin && pin && ii >= 0 && ii < d.ni;
-                const long long px = ((long long)kk * d.nj + jj) * d.ni + ii;
-                const long long pg = ((long long)k * d.nj + j) * d.ni + i;
-                a[r] = xin ? (short)X[px * cin + cb * 16 + m] : (short)0;
-                b[r] = pin ? (short)G[pg * cout + t * 16 + m] : (short)0;
+                const int i = i0 + r < d.ni ? i0 + r : d.ni - 1;
+#pragma unroll
+                for (int t = 0; t < NTB; t++) gv[s][t][r] = (short)Gr[(long long)i * cout + t * 16];
             }
-            acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc, 0, 0, 0);
+        }
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+            const int i0 = bi * 64 + s * 16 + 4 * kq;
+            bf16x4 b[NTB];
+#pragma unroll
+            for (int t = 0; t < NTB; t++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) b[t][r] = i0 + r < d.ni ? gv[s][t][r] : (short)0;
+#pragma unroll
+            for (int e = 0; e < 3; e++) {  // di = e - 1
+                bf16x4 a;
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const int i = i0 + r, ii = i + e - 1;
+                    a[r] = rowin && i < d.ni && ii >= 0 && ii < d.ni ? xv[s][r + e] : (short)0;
+                }
+#pragma unroll
+                for (int t = 0; t < NTB; t++) acc[e][t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b[t], acc[e][t], 0, 0, 0);
+            }
         }
     }
-    // acc[r] = dW[ci = 4 kq + r][co = m] of this tile
+    // acc[r] = dW[ci = 4 kq + r][co = m] of each tile
     float *slice = part + (long long)blockIdx.x * 27 * cin * cout;
 #pragma unroll
-    for (int r = 0; r < 4; r++) {
-        const int ci = cb * 16 + 4 * kq + r, co = t * 16 + m;
-        slice[((long long)tap * cin + ci) * cout + co] = acc[r];
-    }
+    for (int e = 0; e < 3; e++)
+#pragma unroll
+        for (int t = 0; t < NTB; t++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int ci = cb * 16 + 4 * kq + r, co = (t0 + t) * 16 + m;
+                slice[((long long)(kj * 3 + e) * cin + ci) * cout + co] = acc[e][t][r];
+            }
 }
 
-// out[i] = sum over p = 0 .. P-1, in order, of part[p * stride + i], i < n
+// out[i] = sum over p = 0 .. P-1, in order, of part[p * stride + i], i < n: SP_U
+// loads in flight ahead of their additions (one after the other, 64 slices
+// took 17 us whatever n; now 6)
+constexpr int SP_U = 16;
 __global__ void k_sum_partials(const float *__restrict__ part, int P, long long stride, long long n, float *__restrict__ out)
 {
     const long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x;
     if (i >= n) return;
     float s = 0.f;
-    for (int p = 0; p < P; p++) s += part[p * stride + i];
+    int p = 0;
+    for (; p + SP_U <= P; p += SP_U) {
+        float v[SP_U];
+#pragma unroll
+        for (int u = 0; u < SP_U; u++) v[u] = part[(p + u) * stride + i];
+#pragma unroll
+        for (int u = 0; u < SP_U; u++) s += v[u];
+    }
+    for (; p < P; p++) s += part[p * stride + i];
     out[i] = s;
 }
 
@@ -811,13 +861,28 @@ static int conv_bwd_data(hipStream_t st, const Dims &d, const Conv &c, const bf1
     return VFS_OK;
 }
 
-constexpr int WG_SLICES = 64;  // partial weight-gradient slices (fixed: the summation order is too)
+// partial weight-gradient slices (fixed by the layer's and the grid's sizes: the
+// summation order is too): 64, and up to 256 for a layer whose channels give
+// fewer than four wavefronts per SIMD while a slice keeps four rows or more (the
+// five such layers of a 64x48x64 network: 91 -> 57 us each)
+constexpr int WG_SLICES = 64, WG_SLICES_MAX = 256;
+static int wg_slices(const Conv &c, long long nrows)
+{
+    const int tiles = 9 * (c.cin / 16) * (c.cout / 16);
+    int n = WG_SLICES;
+    while (n < WG_SLICES_MAX && (long long)n * tiles < 4096 && 8LL * n <= nrows) n *= 2;
+    return n;
+}
 
 static int conv_bwd_weight(hipStream_t st, const Dims &d, const Conv &c, const bf16 *X, const bf16 *G, float *wpart)
 {
-    dim3 grid(WG_SLICES, (unsigned)(27 * (c.cin / 16) * (c.cout / 16)));
-    hipLaunchKernelGGL(k_conv3_wgrad, grid, dim3(64), 0, st, d, c.cin, c.cout, X, G, wpart);
-    hipLaunchKernelGGL(k_sum_partials, dim3(blocks_for(c.nw, 256)), dim3(256), 0, st, wpart, WG_SLICES, c.nw, c.nw, c.gw);
+    // two output tiles a wavefront where that leaves four wavefronts per SIMD
+    const int tiles = 9 * (c.cin / 16) * (c.cout / 16);
+    const bool two = (c.cout / 16) % 2 == 0 && WG_SLICES * tiles / 2 >= 4096;
+    const int slices = wg_slices(c, (long long)((d.ni + 63) / 64) * d.nj * d.nk);
+    hipLaunchKernelGGL(two ? k_conv3_wgrad<2> : k_conv3_wgrad<1>, dim3(slices, (unsigned)(two ? tiles / 2 : tiles)), dim3(64), 0,
+                       st, d, c.cin, c.cout, X, G, wpart);
+    hipLaunchKernelGGL(k_sum_partials, dim3(blocks_for(c.nw, 256)), dim3(256), 0, st, wpart, slices, c.nw, c.nw, c.gw);
     hipLaunchKernelGGL(k_bias_grad, dim3(BG_BLOCKS, c.cout), dim3(256), 0, st, d.np(), c.cout, G, wpart);
     hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(256), 0, st, wpart, BG_BLOCKS, (long long)c.cout, (long long)c.cout, c.gb);
     VFS_LAUNCH_CHECK("unet conv weight gradient");
@@ -1060,7 +1125,7 @@ int vfs_unet_create(vfs_ctx *c, int base, int levels, unsigned long long seed, v
     rc = rc ? rc : ualloc(u, (void **)&u->part, (RED_BLOCKS + 8) * sizeof(double));
     long long wmax = (long long)OB_BLOCKS * (base + 1);
     for (auto *v : {&u->enc, &u->dec})
-        for (auto &cv : *v) wmax = std::max({wmax, (long long)WG_SLICES * cv.nw, (long long)BG_BLOCKS * cv.cout});
+        for (auto &cv : *v) wmax = std::max({wmax, wg_slices(cv, 1LL << 40) * cv.nw, (long long)BG_BLOCKS * cv.cout});
     rc = rc ? rc : ualloc(u, (void **)&u->wpart, wmax * sizeof(float));
     if (!rc) rc = repack(u);
     if (rc) { vfs_unet_destroy(u); return rc; }
