@@ -18,9 +18,10 @@
 // default smoother is hybrid Gauss-Seidel, sequential Gauss-Seidel inside
 // one rank; here each level's rows are greedily coloured at setup so rows of
 // one colour share no matrix entry, and one colour is relaxed per launch
-// (forward colour order before the coarse correction, backward after).  CSR
-// products run one row per thread; the coarsest level is a dense inverse of
-// A_c + s 1 1^T (A's null space is the constant vector).
+// (forward colour order before the coarse correction, backward after), from a
+// copy of the rows laid out by colour.  CSR products take a group of lanes per
+// row; the coarsest level is a dense inverse of A_c + s 1 1^T (A's null space
+// is the constant vector).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

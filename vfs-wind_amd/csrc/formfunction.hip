@@ -11,8 +11,9 @@
 //     Rhs or, inside RungeKutta, writes Ucont = a*(Rhs - dP) + pUcont
 //     directly (rhs.c:1647-1658), so Rhs never round-trips through HBM.
 // The arithmetic follows the reference's operation order, with FP
-// contraction disabled for this file, so results match the FP64 CPU path to
-// a few ulps.
+// contraction disabled for this file, except inside the viscous face flux
+// (visc_face: the same products in fewer, fused operations), so results match
+// the FP64 CPU path to a few ulps and all paths here match each other to the bit.
 #include <hip/hip_runtime.h>
 
 #include <cstdlib>
