@@ -10,6 +10,10 @@ pytestmark = pytest.mark.gpu
 # whole hierarchies in one block (coarsenable, single odd level, one line
 # segment), the coarse levels only, and no level small enough but the last
 CELLS = [(16, 12, 16), (17, 11, 13), (4, 4, 6), (24, 16, 20), (40, 24, 36), (64, 48, 64), (36, 70, 44)]
+# odd periodic counts with one segment per line: lines of one colour, held by
+# different wavefronts, read each other's values from before the half-sweep (the
+# last grid on its coarsest level, 17x8x17, which has too many rows for a dense solve)
+CELLS += [(17, 7, 19), (16, 8, 17), (17, 8, 17), (19, 6, 16), (68, 32, 68)]
 
 
 @pytest.mark.parametrize("form", ["compact", "full", "fp64", "deep"])

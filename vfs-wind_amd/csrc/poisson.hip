@@ -1364,6 +1364,10 @@ __device__ __forceinline__ void tail_c4_half(const TailLevel<float> &L, const Ta
             r[v] = v < np ? rv : 0.f;
         }
     }
+    // Lines of one colour meet across the wrap of an odd periodic count and read
+    // each other's values from before this half-sweep.  With more than one segment
+    // tail_solve's barriers stand between these reads and its stores.
+    if (t.nseg == 1 && !zebra_fused_ok(g)) __syncthreads();
     tail_solve<float>(t, M, r, s.l, s.m, s.u, act, x + at + i, g.mx);
 }
 
