@@ -6,6 +6,7 @@ pseudo-periodic inlet and with -inlet 100.  Tolerance 1e-12 normwise
 relative (the inlet area and flux sums reduce in another order)."""
 import numpy as np
 import pytest
+import torch
 
 from helpers import cases, relerr, vfs
 import pyoracle as po
@@ -112,3 +113,33 @@ def test_unsupported_profiles_are_refused():
             vfs.Context(vfs.make_params(mx, my, mz, per=(0, 0, 0), bctype=c.bctype, les=0, inletprofile=prof))
     with pytest.raises(vfs.VFSError, match="-pseudo"):
         vfs.Context(vfs.make_params(mx, my, mz, per=(1, 0, 1), bctype=(100, 100, 1, 1, 100, 100), pseudo=1))
+
+
+class _Device:
+    """A field's device memory as torch reads it."""
+
+    def __init__(self, ctx, name):
+        self.__cuda_array_interface__ = {"shape": tuple(ctx.field_shape(name)), "typestr": "<f8", "version": 2,
+                                         "data": (ctx.device_ptr(name), False)}
+
+
+@pytest.mark.parametrize("profile,flux", [(1, -1.0), (14, 0.6)], ids=["uniform", "held"])
+def test_inlet_written_on_return(profile, flux):
+    """What the call writes is there when it returns, for a reader on a stream
+    that nothing orders with the library's."""
+    o, ctx = centred_pair(130, 100, 4, inletprofile=profile, inlet_flux=flux)
+    with ctx:
+        views = {f: torch.as_tensor(_Device(ctx, f), device="cuda") for f in ("UCONT", "UCAT")}
+        start = {f: ctx.download(f) for f in views}
+        side = torch.cuda.Stream()
+        for v in start.values():
+            v[0] = -7.0  # what the inlet plane holds before the call
+        for _ in range(3):
+            for f, v in start.items():
+                ctx.upload(f, v)
+            ctx.inflow_flux()
+            with torch.cuda.stream(side):
+                got = {f: v[0].cpu() for f, v in views.items()}
+            for f in views:
+                assert np.array_equal(got[f].numpy(), ctx.download(f)[0]), f
+            assert not (got["UCONT"][1:-1, 1:-1, 2] == -7.0).any()

@@ -505,7 +505,12 @@ int vfs_pseudo_periodic_plane(vfs_ctx *c)
 int vfs_inflow_flux(vfs_ctx *c, double *flux_in)
 {
     if (!c) return vfs::set_error(VFS_EINVAL, "null context");
-    return vfs::inflow_flux(c, flux_in);
+    int rc = vfs::inflow_flux(c, flux_in);
+    if (rc) return rc;
+    // the flux arrives while the kernel that also writes the inlet's Ucont and
+    // Ucat still runs: a caller may read those on a stream of its own
+    VFS_HIP(hipStreamSynchronize(c->stream));
+    return VFS_OK;
 }
 
 int vfs_min_dt(vfs_ctx *c, double *dt_cfl1)
