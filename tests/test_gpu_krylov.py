@@ -1,6 +1,11 @@
 """The Gram-Schmidt sweeps with their sums finished by the last block: every
 basis-size instance (4, 8, 16, 32 vectors) on grids from a handful of blocks to
 more than the partials hold, checked with the oracle's operator."""
+import os
+import subprocess
+import sys
+from pathlib import Path
+
 import numpy as np
 import pytest
 
@@ -27,3 +32,29 @@ def test_restart_lengths(cells, restart):
         assert r < 0.9 and (st.relres <= 1e-6 or st.iterations == 40)
         st2 = ctx.poisson_solve(opts, check=False)  # the counters are back at zero: the same bits again
         assert (st2.iterations, st2.relres) == (st.iterations, st.relres)
+
+
+SCALARS = """
+from helpers import channel_pair, vfs
+c, o, ctx = channel_pair(17, 11, 13, les=0)
+ctx.poisson_rhs()
+st = ctx.poisson_solve(vfs.default_solve_opts(tol=1e-8, use_guess=0))
+out = [ctx.min_dt(), ctx.calc_k_flux(), ctx.divergence(), st.iterations, st.relres]
+ctx.close()
+"""
+
+
+def test_host_results_without_coherent_default():
+    """The scalars the host polls for arrive where the runtime's default host
+    memory is not coherent (a process of its own: the setting is read at its
+    start), with the bits they have otherwise."""
+    here = {}
+    exec(SCALARS, here)
+    tests = Path(__file__).resolve().parent
+    env = dict(os.environ, HIP_HOST_COHERENT="0",
+               PYTHONPATH=os.pathsep.join(str(p) for p in (tests, tests.parent, tests.parent / "oracle")))
+    r = subprocess.run([sys.executable, "-c", SCALARS + "print('SCALARS', *map(float.hex, map(float, out)))"], env=env,
+                       cwd=tests.parent, capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, r.stderr[-2000:]
+    got = r.stdout.split("SCALARS")[1].split()
+    assert got == [float(v).hex() for v in here["out"]]

@@ -138,6 +138,7 @@ int red_wait(vfs_ctx *c)
 {
     volatile unsigned long long *flag = red_flag(c);
     for (unsigned spin = 1; *flag != c->red_seq; spin++) {
+        __builtin_ia32_pause();
         if (spin % 4096) continue;
         const hipError_t e = hipStreamQuery(c->stream);
         if (e == hipErrorNotReady) continue;
@@ -215,7 +216,9 @@ int vfs_ctx_create(const vfs_params *params, vfs_ctx **out)
     if (!rc) rc = alloc(&c->red, 1 << 16);
     if (!rc) rc = alloc(&c->inflow_plane, 3 * (size_t)c->g.plane);
     if (!rc) {
-        hipError_t ee = hipHostMalloc((void **)&c->red_host, 4096 * sizeof(double), hipHostMallocDefault);
+        // coherent by name: the host polls what running kernels store there, and
+        // the default's coherence is the environment's to choose
+        hipError_t ee = hipHostMalloc((void **)&c->red_host, 4096 * sizeof(double), hipHostMallocMapped | hipHostMallocCoherent);
         if (ee != hipSuccess) rc = vfs::check_hip(ee, "hipHostMalloc");
         else *vfs::red_flag(c) = 0;
     }
