@@ -937,8 +937,9 @@ __global__ void __launch_bounds__(FT_I * FT_J) k_cell_rhs(CellArgs a, int kc, co
             // Rhs = 0 + F; Rhs += -1*dP; Ucont = alpha*Rhs + pUcont  (rhs.c:1647-1658).
             // Every input is loaded before the three stores, which then leave
             // together (a store between loads wrote partial lines to HBM).
+            // (pucont and ucont_out are one array in the last stage.)
             const double *__restrict__ dp = a.dp + 3 * q;
-            const double *__restrict__ pu = a.pucont + 3 * q;
+            const double *pu = a.pucont + 3 * q;
             double d[3], u[3], o[3];
 #pragma unroll
             for (int c = 0; c < 3; c++) { d[c] = dp[c]; u[c] = pu[c]; }
@@ -948,7 +949,7 @@ __global__ void __launch_bounds__(FT_I * FT_J) k_cell_rhs(CellArgs a, int kc, co
                 rv += -1 * d[c];
                 o[c] = a.alpha * rv + u[c];
             }
-            double *__restrict__ out = a.ucont_out + 3 * q;
+            double *out = a.ucont_out + 3 * q;
 #pragma unroll
             for (int c = 0; c < 3; c++) out[c] = o[c];
         } else if (a.cn_r) {
@@ -1045,8 +1046,9 @@ __global__ void __launch_bounds__(CR_T) k_cell_rhs_pr(CellArgs a, int kc, const 
             // Rhs = 0 + F; Rhs += -1*dP; Ucont = alpha*Rhs + pUcont  (rhs.c:1647-1658).
             // Every input is loaded before the three stores, which then leave
             // together (a store between loads wrote partial lines to HBM).
+            // (pucont and ucont_out are one array in the last stage.)
             const double *__restrict__ dp = a.dp + 3 * q;
-            const double *__restrict__ pu = a.pucont + 3 * q;
+            const double *pu = a.pucont + 3 * q;
             double d[3], u[3], o[3];
 #pragma unroll
             for (int c = 0; c < 3; c++) { d[c] = dp[c]; u[c] = pu[c]; }
@@ -1056,7 +1058,7 @@ __global__ void __launch_bounds__(CR_T) k_cell_rhs_pr(CellArgs a, int kc, const 
                 rv += -1 * d[c];
                 o[c] = a.alpha * rv + u[c];
             }
-            double *__restrict__ out = a.ucont_out + 3 * q;
+            double *out = a.ucont_out + 3 * q;
 #pragma unroll
             for (int c = 0; c < 3; c++) out[c] = o[c];
         } else if (a.cn_r) {

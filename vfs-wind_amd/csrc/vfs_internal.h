@@ -224,7 +224,7 @@ struct vfs_ctx {
     double *f[VFS_NFIELDS];
     // scratch for Formfunction_2 and the RK driver
     double *face;     // 18 doubles per point: div1..3, visc1..3 (Cmpnts each)
-    double *pucont;   // RK base state
+    double *pucont;   // the RK stages' second Ucont (runge_kutta)
     double *snap;     // 3 doubles per point: snapshot for BC passes
     double *fpc;      // 3 planes of n doubles: Fp of every cell (Formfunction_2)
     double *red;      // reduction scratch (device)
