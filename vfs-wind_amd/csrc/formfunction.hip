@@ -138,8 +138,9 @@ __device__ inline void load_metrics(const Metrics9 &m, long long q0, unsigned of
 // twice the mean area vectors and a quarter of the mean Jacobian
 // (rhs2.c:595-647).  The viscous flux is quadratic in the vectors and linear in
 // the Jacobian, so the powers of two cancel and a face's flux has the bits it
-// has with the stored means (face_mean) themselves; a[9] and b[9] are the
-// reciprocal Jacobians, which a cell's faces share.
+// has with the stored face metrics (0.5 X + 0.5 Y and 2 / (1/aj + 1/aj) of the
+// two cells); a[9] and b[9] are the reciprocal Jacobians, which a cell's faces
+// share.
 __device__ inline void face_sum(const double a[10], const double b[10], double f[10])
 {
 #pragma unroll
