@@ -34,6 +34,28 @@ def test_restart_lengths(cells, restart):
         assert (st2.iterations, st2.relres) == (st.iterations, st.relres)
 
 
+@pytest.mark.parametrize("tol", [1e-12, 1e-18])
+@pytest.mark.parametrize("cells", [(4, 4, 6), (8, 6, 8)], ids=str)
+def test_exhausted_basis(cells, tol):
+    """A preconditioner that is the inverse (an algebraic hierarchy of one
+    level) leaves nothing but rounding of the first new vector.  Its norm is then
+    the small difference the second pass computes it as, and may come out as
+    zero: the solve stops at the residual a double can reach, finite, also when
+    it is asked for less.  96 and 384 rows, condition numbers 45 and 85: rows x
+    2^-53 x condition number is 4e-12 at most."""
+    c, o, ctx = channel_pair(*cells, les=0)
+    with ctx:
+        o.poisson_rhs()
+        ctx.poisson_rhs()
+        ctx.upload("PHI", np.zeros(o.shape))
+        st = ctx.poisson_solve(vfs.default_solve_opts(tol=tol, use_guess=0, amg=1, maxit=12), check=False)
+        phi = ctx.download("PHI")
+        assert np.isfinite(phi).all()
+        r = np.linalg.norm(o["b"] - o.poisson_apply(phi)) / np.linalg.norm(o["b"])
+        assert r <= 1e-11
+        assert st.iterations <= (2 if tol == 1e-12 else 12)
+
+
 SCALARS = """
 from helpers import channel_pair, vfs
 c, o, ctx = channel_pair(17, 11, 13, les=0)
