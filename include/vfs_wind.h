@@ -121,8 +121,9 @@ int vfs_form_bcs(vfs_ctx *ctx, int outflow_scale);
  * (Poiseuille) and 100 or -pseudo 1 (the inflow plane, vfs_inflow_set_plane /
  * vfs_pseudo_periodic_plane), with the held bulk flux of -inlet 14, 100 and
  * -pseudo when -flux is given: inlet fluxes and ghost velocities; FluxInSum
- * returned and kept for FormBCS.  Profile 11 (time-seeded noise) and the
- * profiles that leave the inlet velocity unset (13, 16, 20, 101) are refused. */
+ * returned and kept for FormBCS; the fields are written when the call returns.
+ * Profile 11 (time-seeded noise) and the profiles that leave the inlet velocity
+ * unset (13, 16, 20, 101) are refused. */
 int vfs_inflow_flux(vfs_ctx *ctx, double *flux_in);
 /* Compute_Smagorinsky_Constant_1 (les.c:75-1141) from VFS_UCAT into lCs:
  * 0 while ti < 2 on a fresh start (tistart == 0 and no restart), params.cs2
@@ -227,7 +228,8 @@ typedef struct {
     int poisson_iterations;
     double poisson_relres;
     double maxdiv;
-    double ms_momentum, ms_poisson, ms_total;
+    double ms_momentum, ms_poisson;  /* time on the device, from events on the context's stream */
+    double ms_total;                 /* time of the call on the host */
     int newton_iterations, linear_iterations;  /* implicit step only */
 } vfs_step_stats;
 

@@ -469,16 +469,26 @@ __global__ void __launch_bounds__(FT_I * FT_J) k_face_fluxes(FaceArgs a, int kc)
 // FormMetrics leave them) the faces at index 0 computed here are bitwise
 // those copies, so that fix is not applied.
 // Eight rows of points a block: two blocks fit a CU's LDS and, at 208 registers
-// a lane, its register files, so one block's loads and barriers overlap with
-// the other's arithmetic.  What bounds it is the wait for those loads with two
-// wavefronts per SIMD (the VALU is busy for a third of the time).  With the
-// faces' FP64 work at 90 instead of 187 instructions each, no face behind a
-// test, constant LDS offsets and scalar base addresses (600 instructions a point
-// instead of 1000; before, one block of 16 rows per CU): 766 -> 638 us at
-// 256x192x256, 1184 -> 965 at 384x192x256, 39 -> 30 at 96x64x80, 24 -> 17 at
-// 64x48x64, 14 -> 9 at 16x12x16.  Sixteen rows: 640, 923, 34, 21, 11; three
-// blocks per CU (168 registers) spill and take twice as long, and so does any
-// load of the next plane into registers that spill for it.
+// a lane (225 with blanking tests), its register files, so one block's loads and
+// barriers overlap with the other's arithmetic.  What bounds it is the wait for
+// those loads with two wavefronts per SIMD (the VALU is busy for a third of the
+// time).  With the faces' FP64 work at 90 instead of 187 instructions each, no
+// face behind a test, constant LDS offsets and scalar base addresses (600
+// instructions a point instead of 1000; before, one block of 16 rows per CU), in
+// a loop of residuals, with its two events:
+//                   16x12x16  64x48x64  96x64x80  136x104x88  256x192x256  384x192x256
+//   before               101       108       110         125          797         1179 us
+//   8 rows                10        20        31          81          625          943
+//   16 rows               12        19        30          76          596          900
+//   blanked, before      181       198       200         215         1273         1909
+//   8 rows                13        24        39         102          725         1079
+//   16 rows               14        23        37          94          687         1021
+// (16 rows: one block per CU, and runs of planes chosen for that.)  By this
+// measurement eight rows are the better ones on the smallest grid only; within
+// whole steps, where the choice was made, 16 gained nothing at 256x192x256 (640
+// against 638 us) and 4 % at 384x192x256 (923 against 965).  Three blocks per CU
+// (168 registers) spill and take twice as long, and so does any load of the next
+// plane into registers that spill for it.
 constexpr int FP_J = 8;
 constexpr int FP_T = FT_I * FP_J;
 constexpr int FP_WAVES = 2;  // wavefronts per SIMD, which is also blocks per CU

@@ -71,7 +71,10 @@ __global__ void __launch_bounds__(RED_THREADS) k_multidot(long long n, int nv, c
 // h2[nv + 1] receives the square of the final norm.  After the second pass it
 // follows from the dot products (V is orthonormal, so the pass takes sum h2^2
 // off it; that sum is a rounding error's square except where w is nothing but
-// rounding error), so that w need not be read again for it.
+// rounding error), so that w need not be read again for it.  Where w is nothing
+// but rounding error the difference has no correct digit; a negative one counts
+// as zero, the new vector is then zero and the caller's estimate of the residual
+// too: the basis is exhausted, which a measured norm of that rounding says as well.
 template <int NVM, int U>
 __global__ void __launch_bounds__(RED_THREADS) k_multiaxpy(long long n, int nv, const double *__restrict__ h,
                                                            const double *__restrict__ V, long long ld, double *__restrict__ w,
