@@ -133,7 +133,9 @@ RedSync red_sync(vfs_ctx *c, int at) { return {c->red_ctr, c->red_host + at, red
 RedSync red_quiet(vfs_ctx *c) { return {c->red_ctr, nullptr, nullptr, 0}; }
 
 // Waits on the flag in pinned memory; now and then the stream is asked too, so
-// that a kernel that failed ends the wait.
+// that a kernel that failed ends the wait.  The pause leaves the flag's cache line
+// to the store that is awaited: a time step of 16x12x16 cells 624 -> 583 us, of
+// 64x48x64 no different.
 int red_wait(vfs_ctx *c)
 {
     volatile unsigned long long *flag = red_flag(c);
